@@ -17,10 +17,10 @@
 //                 like the plain sensor's.
 //   k_mlp_collect features and plain labels (kp > 1) of the nodes of a
 //                 sub-lattice, for training.
-//   k_mlp_fwd / k_mlp_param   training in FP32: per-sample forward and
-//                 backward vectors, then one thread per parameter sums the
-//                 batch in sample order (no atomics: the gradients and the
-//                 Adam update do not depend on scheduling).
+//   k_mlp_grad / k_mlp_update   training in FP32 (FP32 MFMA): forward,
+//                 backward and partial gradient sums per wave, then the sum
+//                 of the partials and the Adam update (no atomics: neither
+//                 depends on scheduling).
 //
 // Parameters (1889 floats): W1 [32][24], b1 [32], W2 [32][32], b2 [32],
 // W3 [32], b3.
@@ -34,16 +34,6 @@ namespace {
 
 using namespace mlp;
 static_assert(OB3 + 1 == MLP_NPARAM, "parameter layout");
-constexpr int PER_SAMPLE = 4 * NH + 2;  // dz1, a1, dz2, a2, dz3, loss term
-
-__device__ __forceinline__ float gelu(float x) {
-    const float t = tanhf(0.7978845608028654f * (x + 0.044715f * x * x * x));
-    return 0.5f * x * (1.0f + t);
-}
-__device__ __forceinline__ float gelu_grad(float x) {
-    const float t = tanhf(0.7978845608028654f * (x + 0.044715f * x * x * x));
-    return 0.5f * (1.0f + t) + 0.5f * x * (1.0f - t * t) * 0.7978845608028654f * (1.0f + 3.0f * 0.044715f * x * x);
-}
 
 // ---------------------------------------------------------------------------
 // Inference
@@ -115,102 +105,182 @@ __global__ void __launch_bounds__(256) k_mlp_collect(FeatIn<S> F, int stride, in
     y[t] = jameson_kp(F, gidx(F.g, i, j, k), i1, i2) > 1 ? 1.f : 0.f;
 }
 
-// Per sample of the batch: forward, weighted BCE term and the backward
-// vectors dz1, a1, dz2, a2, dz3 (the batch mean is taken in k_mlp_param).
-__global__ void __launch_bounds__(256) k_mlp_fwd(const float* __restrict__ P, const float* __restrict__ X,
-                                                 const float* __restrict__ y, const int* __restrict__ idx, int nb,
-                                                 float wpos, float* __restrict__ out) {
-    const int s = blockIdx.x * 256 + threadIdx.x;
-    if (s >= nb) return;
-    const long long row = idx ? idx[s] : s;
-    float x[NF];
-#pragma unroll
-    for (int e = 0; e < NF; e++) x[e] = X[row * NF + e];
-    float z1[NH], a1[NH], z2[NH], a2[NH];
-    for (int o = 0; o < NH; o++) {
-        float acc = P[OB1 + o];
-#pragma unroll
-        for (int e = 0; e < NF; e++) acc += P[OW1 + o * NF + e] * x[e];
-        z1[o] = acc;
-        a1[o] = gelu(acc);
-    }
-    for (int o = 0; o < NH; o++) {
-        float acc = P[OB2 + o];
-#pragma unroll
-        for (int h = 0; h < NH; h++) acc += P[OW2 + o * NH + h] * a1[h];
-        z2[o] = acc;
-        a2[o] = gelu(acc);
-    }
-    float z3 = P[OB3];
-#pragma unroll
-    for (int h = 0; h < NH; h++) z3 += P[OW3 + h] * a2[h];
-    const float prob = 1.f / (1.f + expf(-z3));
-    const float yy = y[row];
-    const float w = yy > 0.5f ? wpos : 1.f;
-    const float eps = 1e-7f;
-    const float lt = -w * (yy * logf(prob + eps) + (1.f - yy) * logf(1.f - prob + eps));
-    const float dz3 = w * (prob - yy);
-    float* o_ = out + (long long)s * PER_SAMPLE;
-    float dz2[NH];
-    for (int o = 0; o < NH; o++) dz2[o] = dz3 * P[OW3 + o] * gelu_grad(z2[o]);
-    for (int h = 0; h < NH; h++) {
-        float da = 0.f;
-        for (int o = 0; o < NH; o++) da += P[OW2 + o * NH + h] * dz2[o];
-        o_[h] = da * gelu_grad(z1[h]);  // dz1
-    }
-    for (int h = 0; h < NH; h++) {
-        o_[NH + h] = a1[h];
-        o_[2 * NH + h] = dz2[h];
-        o_[3 * NH + h] = a2[h];
-    }
-    o_[4 * NH] = dz3;
-    o_[4 * NH + 1] = lt;
+// ---------------------------------------------------------------------------
+// Training: a wave takes tiles of 32 samples.  All five contractions of a
+// tile run on the FP32 matrix instruction v_mfma_f32_32x32x2_f32 (FP32
+// products and sums): Z1 = W1 X^T, Z2 = W2 A1, dA1 = W2^T dZ2, dW1 += dZ1 X,
+// dW2 += dZ2 A1^T.  A lane l of the instruction holds A[l%32][l/32],
+// B[l/32][l%32] and D[unit(r, l/32)][l%32], r = 0..15, unit(r, h) = 8 (r/4) +
+// 4 h + r%4.  With samples as columns, register r of one layer's output is
+// step r's B operand of the next when the weights are fed in the same unit
+// order, so the forward and the backward pass stay in registers; the two
+// weight gradients contract over samples and read their operands back from
+// LDS tiles (pitch 33: no bank conflicts).  A wave keeps its gradient sums in
+// registers over its tiles and writes one partial vector; k_mlp_update adds
+// the partials in wave order and applies Adam.  No atomics: a seed fixes the
+// result.
+//
+// Bound by latency, not by work (a batch of 4096 is 0.05 GFLOP): 128 waves of
+// one tile instead of one thread per sample and per parameter.  An epoch of
+// 65536 samples in batches of 4096, the shuffle on the host included: 33.8 ->
+// 0.47 ms (the sum over the samples was one thread per parameter).
+// ---------------------------------------------------------------------------
+typedef float v16f __attribute__((ext_vector_type(16)));
+constexpr int TS = 32;              // samples per tile
+constexpr int TP = 33;              // LDS pitch of a 32 x 32 tile
+constexpr int PART = MLP_NPARAM + 1;  // a wave's partial: the parameters' gradient sums, then the loss sum
+constexpr int MAX_PART = 1024;      // waves (partials) of one batch at most
+constexpr int UPD_SLICES = 16;      // partial sums taken beside each other in k_mlp_update
+
+int mlp_waves(int nb) {
+    const int t = (nb + TS - 1) / TS;
+    return t < MAX_PART ? t : MAX_PART;
 }
 
-// One thread per parameter: the batch-mean gradient summed in sample order,
-// then (adam_t > 0) the Adam update of the parameter.  Thread MLP_NPARAM sums
-// the loss.
-__global__ void __launch_bounds__(256) k_mlp_param(float* __restrict__ P, const float* __restrict__ X,
-                                                   const int* __restrict__ idx, const float* __restrict__ per, int nb,
-                                                   float* __restrict__ grad, float* __restrict__ m1,
-                                                   float* __restrict__ m2, int adam_t, float lr, float* loss) {
-    const int p = blockIdx.x * 256 + threadIdx.x;
-    if (p > MLP_NPARAM) return;
-    const float inv = 1.f / (float)nb;
-    float gsum = 0.f;
+// GELU and its derivative from one tanh.
+__device__ __forceinline__ void gelu_both(float x, float& g, float& dg) {
+    const float t = tanhf(0.7978845608028654f * (x + 0.044715f * x * x * x));
+    g = 0.5f * x * (1.0f + t);
+    dg = 0.5f * (1.0f + t) + 0.5f * x * (1.0f - t * t) * 0.7978845608028654f * (1.0f + 3.0f * 0.044715f * x * x);
+}
+
+// GRAD: partial gradient sums of the samples (idx[0..nb), or rows 0..nb) into
+// part[gridDim.x][PART]; else only the probabilities into prob.
+template <bool GRAD>
+__global__ void __launch_bounds__(64) k_mlp_grad(const float* __restrict__ P, const float* __restrict__ X,
+                                                 const float* __restrict__ y, const int* __restrict__ idx, int nb,
+                                                 float wpos, float* __restrict__ part, float* __restrict__ prob) {
+    __shared__ float sX[GRAD ? TS * TP : 1], sD1[GRAD ? TS * TP : 1], sA1[GRAD ? TS * TP : 1],
+        sD2[GRAD ? TS * TP : 1], sG3[GRAD ? TS * TP : 1];
+    const int lane = threadIdx.x, col = lane & 31, half = lane >> 5;
+    auto unit = [&](int r) { return 8 * (r >> 2) + 4 * half + (r & 3); };
+    float w1[12], w2[16], w2t[16], w3[16];
+    v16f b1, b2;
+#pragma unroll
+    for (int k = 0; k < 12; k++) w1[k] = P[OW1 + col * NF + 2 * k + half];
+#pragma unroll
+    for (int r = 0; r < 16; r++) {
+        w2[r] = P[OW2 + col * NH + unit(r)];
+        if (GRAD) w2t[r] = P[OW2 + unit(r) * NH + col];
+        w3[r] = P[OW3 + unit(r)];
+        b1[r] = P[OB1 + unit(r)];
+        b2[r] = P[OB2 + unit(r)];
+    }
+    const float b3 = P[OB3];
+    v16f gW1 = {}, gW2 = {};
+    float gb1 = 0.f, gb2 = 0.f, gw3 = 0.f, gb3 = 0.f, gl = 0.f;
+    for (int s0 = blockIdx.x * TS; s0 < nb; s0 += gridDim.x * TS) {
+        const int s = s0 + col;
+        const bool in = s < nb;
+        const long long row = in ? (idx ? idx[s] : s) : 0;
+        float x[12];
+#pragma unroll
+        for (int k = 0; k < 12; k++) x[k] = in ? X[row * NF + 2 * k + half] : 0.f;
+        v16f z1 = b1, z2 = b2;
+#pragma unroll
+        for (int k = 0; k < 12; k++) z1 = __builtin_amdgcn_mfma_f32_32x32x2f32(w1[k], x[k], z1, 0, 0, 0);
+        float a1[16], d1[16], a2[16], d2[16];
+#pragma unroll
+        for (int r = 0; r < 16; r++) gelu_both(z1[r], a1[r], d1[r]);
+#pragma unroll
+        for (int r = 0; r < 16; r++) z2 = __builtin_amdgcn_mfma_f32_32x32x2f32(w2[r], a1[r], z2, 0, 0, 0);
+        float z3 = 0.f;
+#pragma unroll
+        for (int r = 0; r < 16; r++) {
+            gelu_both(z2[r], a2[r], d2[r]);
+            z3 += w3[r] * a2[r];
+        }
+        z3 += __shfl_xor(z3, 32);
+        z3 += b3;
+        const float pr = 1.f / (1.f + expf(-z3));
+        if (!GRAD) {
+            if (in && half == 0) prob[s] = pr;
+            continue;
+        }
+        const float yy = in ? y[row] : 0.f;
+        const float w = !in ? 0.f : yy > 0.5f ? wpos : 1.f;
+        const float eps = 1e-7f;
+        const float dz3 = in ? w * (pr - yy) : 0.f;
+        if (half == 0) {
+            gb3 += dz3;
+            if (in) gl += -w * (yy * logf(pr + eps) + (1.f - yy) * logf(1.f - pr + eps));
+        }
+        v16f da = {};
+#pragma unroll
+        for (int r = 0; r < 16; r++) {
+            d2[r] *= dz3 * w3[r];  // dz2
+            da = __builtin_amdgcn_mfma_f32_32x32x2f32(w2t[r], d2[r], da, 0, 0, 0);
+        }
+        __syncthreads();  // the previous tile's reads are done
+#pragma unroll
+        for (int k = 0; k < 12; k++) sX[col * TP + 2 * k + half] = x[k];
+#pragma unroll
+        for (int r = 0; r < 16; r++) {
+            const int o = col * TP + unit(r);
+            sD1[o] = in ? da[r] * d1[r] : 0.f;  // dz1
+            sA1[o] = a1[r];
+            sD2[o] = d2[r];
+            sG3[o] = dz3 * a2[r];
+        }
+        __syncthreads();
+#pragma unroll
+        for (int k = 0; k < 16; k++) {
+            const int o = (2 * k + half) * TP + col;
+            const float v1 = sD1[o], v2 = sD2[o];
+            gW1 = __builtin_amdgcn_mfma_f32_32x32x2f32(v1, col < NF ? sX[o] : 0.f, gW1, 0, 0, 0);
+            gW2 = __builtin_amdgcn_mfma_f32_32x32x2f32(v2, sA1[o], gW2, 0, 0, 0);
+            gb1 += v1;
+            gb2 += v2;
+            gw3 += sG3[o];
+        }
+    }
+    if (!GRAD) return;
+    gb1 += __shfl_xor(gb1, 32);
+    gb2 += __shfl_xor(gb2, 32);
+    gw3 += __shfl_xor(gw3, 32);
+#pragma unroll
+    for (int m = 1; m < 32; m <<= 1) {  // held by the lanes of half 0
+        gb3 += __shfl_xor(gb3, m);
+        gl += __shfl_xor(gl, m);
+    }
+    float* o = part + (long long)blockIdx.x * PART;
+#pragma unroll
+    for (int r = 0; r < 16; r++) {
+        if (col < NF) o[OW1 + unit(r) * NF + col] = gW1[r];
+        o[OW2 + unit(r) * NH + col] = gW2[r];
+    }
+    if (half == 0) {
+        o[OB1 + col] = gb1;
+        o[OB2 + col] = gb2;
+        o[OW3 + col] = gw3;
+    }
+    if (lane == 0) {
+        o[OB3] = gb3;
+        o[MLP_NPARAM] = gl;
+    }
+}
+
+// Batch-mean gradient (and loss) from nw partial vectors: a block owns 64
+// parameters, slice t sums partials t, t + 16, ... in order, the slices are
+// added in order; then (adam_t > 0) the Adam update of the parameter.
+__global__ void __launch_bounds__(64 * UPD_SLICES) k_mlp_update(float* __restrict__ P, const float* __restrict__ part,
+                                                                int nw, int nb, float* __restrict__ grad,
+                                                                float* __restrict__ m1, float* __restrict__ m2,
+                                                                int adam_t, float lr, float* loss) {
+    __shared__ float sum[UPD_SLICES][64];
+    const int c = threadIdx.x, t = threadIdx.y, p = blockIdx.x * 64 + c;
+    float g = 0.f;
+    if (p < PART)
+        for (int w = t; w < nw; w += UPD_SLICES) g += part[(long long)w * PART + p];
+    sum[t][c] = g;
+    __syncthreads();
+    if (t != 0 || p >= PART) return;
+    for (int q = 1; q < UPD_SLICES; q++) g += sum[q][c];
+    const float gr = g * (1.f / (float)nb);
     if (p == MLP_NPARAM) {
-        for (int s = 0; s < nb; s++) gsum += per[(long long)s * PER_SAMPLE + 4 * NH + 1];
-        *loss = gsum * inv;
+        *loss = gr;
         return;
     }
-    if (p < OB1) {  // W1[o][e] = sum dz1[o] x[e]
-        const int o = p / NF, e = p % NF;
-        for (int s = 0; s < nb; s++) {
-            const long long row = idx ? idx[s] : s;
-            gsum += per[(long long)s * PER_SAMPLE + o] * X[row * NF + e];
-        }
-    } else if (p < OW2) {
-        const int o = p - OB1;
-        for (int s = 0; s < nb; s++) gsum += per[(long long)s * PER_SAMPLE + o];
-    } else if (p < OB2) {  // W2[o][h] = sum dz2[o] a1[h]
-        const int o = (p - OW2) / NH, h = (p - OW2) % NH;
-        for (int s = 0; s < nb; s++) {
-            const float* r = per + (long long)s * PER_SAMPLE;
-            gsum += r[2 * NH + o] * r[NH + h];
-        }
-    } else if (p < OW3) {
-        const int o = p - OB2;
-        for (int s = 0; s < nb; s++) gsum += per[(long long)s * PER_SAMPLE + 2 * NH + o];
-    } else if (p < OB3) {  // W3[h] = sum dz3 a2[h]
-        const int h = p - OW3;
-        for (int s = 0; s < nb; s++) {
-            const float* r = per + (long long)s * PER_SAMPLE;
-            gsum += r[4 * NH] * r[3 * NH + h];
-        }
-    } else {
-        for (int s = 0; s < nb; s++) gsum += per[(long long)s * PER_SAMPLE + 4 * NH];
-    }
-    const float gr = gsum * inv;
     if (grad) grad[p] = gr;
     if (adam_t > 0) {
         const float b1 = 0.9f, b2 = 0.999f, eps = 1e-8f;
@@ -265,14 +335,20 @@ long long mlp_collect_count(const Geo& g, int stride) {
     return (long long)((g.nx + stride - 1) / stride) * ((g.ny + stride - 1) / stride) * ((g.nz + stride - 1) / stride);
 }
 
-void launch_mlp_step(float* params, const float* X, const float* y, const int* idx, int nb, float wpos, float* per,
+void launch_mlp_step(float* params, const float* X, const float* y, const int* idx, int nb, float wpos, float* part,
                      float* grad, float* m1, float* m2, int adam_t, float lr, float* loss, hipStream_t st) {
-    hipLaunchKernelGGL(k_mlp_fwd, dim3((nb + 255) / 256), dim3(256), 0, st, params, X, y, idx, nb, wpos, per);
-    hipLaunchKernelGGL(k_mlp_param, dim3((MLP_NPARAM + 1 + 255) / 256), dim3(256), 0, st, params, X, idx, per, nb,
-                       grad, m1, m2, adam_t, lr, loss);
+    const int nw = mlp_waves(nb);
+    hipLaunchKernelGGL(k_mlp_grad<true>, dim3(nw), dim3(64), 0, st, params, X, y, idx, nb, wpos, part, nullptr);
+    hipLaunchKernelGGL(k_mlp_update, dim3((PART + 63) / 64), dim3(64, UPD_SLICES), 0, st, params, part, nw, nb, grad,
+                       m1, m2, adam_t, lr, loss);
 }
 
-size_t mlp_per_sample_floats() { return PER_SAMPLE; }
+void launch_mlp_predict(const float* params, const float* X, int nb, float* prob, hipStream_t st) {
+    hipLaunchKernelGGL(k_mlp_grad<false>, dim3(mlp_waves(nb)), dim3(64), 0, st, params, X, nullptr, nullptr, nb, 1.f,
+                       nullptr, prob);
+}
+
+size_t mlp_part_floats(int nb) { return (size_t)mlp_waves(nb) * PART; }
 
 template void launch_mlp_sensor<double>(const MlpSensorArgsT<double>&, int, hipStream_t);
 template void launch_mlp_sensor<float>(const MlpSensorArgsT<float>&, int, hipStream_t);

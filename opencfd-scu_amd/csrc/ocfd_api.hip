@@ -1843,8 +1843,10 @@ struct ocfd_mlp {
     long long cap = 0, n = 0;
     float *X = nullptr, *y = nullptr;   // [cap][24], [cap]
     float *P = nullptr, *m1 = nullptr, *m2 = nullptr, *grad = nullptr;
-    float *per = nullptr;               // per-sample vectors of one batch
-    int per_cap = 0;
+    float *part = nullptr;              // partial gradient sums of one batch
+    size_t part_cap = 0;                // floats
+    float *prob = nullptr;              // probabilities of one ocfd_mlp_predict call
+    int prob_cap = 0;
     int* idx = nullptr;                 // sample order of one epoch
     float* loss = nullptr;              // one value per batch of an epoch
     long long loss_cap = 0;
@@ -1854,14 +1856,17 @@ struct ocfd_mlp {
 
 namespace {
 int mlp_alloc(ocfd_mlp* m, void** p, size_t bytes) {
-    if (hipMalloc(p, bytes) != hipSuccess) return fail(OCFD_ERR_HIP, "hipMalloc failed (" + std::to_string(bytes) + " bytes)");
-    m->allocs.push_back(*p);
+    void* q = nullptr;  // *p keeps what it had if this fails
+    if (hipMalloc(&q, bytes) != hipSuccess) return fail(OCFD_ERR_HIP, "hipMalloc failed (" + std::to_string(bytes) + " bytes)");
+    m->allocs.push_back(q);
+    *p = q;
     return 0;
 }
 int mlp_ensure_batch(ocfd_mlp* m, int nb) {
-    if (nb <= m->per_cap) return 0;
-    TRY(mlp_alloc(m, (void**)&m->per, sizeof(float) * mlp_per_sample_floats() * (size_t)nb));
-    m->per_cap = nb;
+    const size_t n = mlp_part_floats(nb);
+    if (n <= m->part_cap) return 0;
+    TRY(mlp_alloc(m, (void**)&m->part, sizeof(float) * n));
+    m->part_cap = n;
     return 0;
 }
 // splitmix64: the seeded sample order of the training epochs
@@ -1986,7 +1991,7 @@ int ocfd_mlp_collect(ocfd_mlp* m, ocfd_ctx* x, int stride) {
 int ocfd_mlp_grad(ocfd_mlp* m, long long first, int n, float wpos, float* grads, float* loss) {
     if (!m || n <= 0 || first < 0 || first + n > m->n) return fail(OCFD_ERR_ARG, "bad range");
     TRY(mlp_ensure_batch(m, n));
-    launch_mlp_step(m->P, m->X + 24 * first, m->y + first, nullptr, n, wpos, m->per, m->grad, m->m1, m->m2, 0, 0.f,
+    launch_mlp_step(m->P, m->X + 24 * first, m->y + first, nullptr, n, wpos, m->part, m->grad, m->m1, m->m2, 0, 0.f,
                     m->grad + MLP_NPARAM, m->st);
     HIPCK(hipGetLastError());
     HIPCK(hipStreamSynchronize(m->st));
@@ -2014,7 +2019,7 @@ int ocfd_mlp_train(ocfd_mlp* m, int epochs, int batch, float lr, float wpos, uns
         HIPCK(hipMemcpyAsync(m->idx, order.data(), sizeof(int) * (size_t)m->n, hipMemcpyHostToDevice, m->st));
         for (long long b = 0; b < nbat; b++) {
             m->adam_t++;
-            launch_mlp_step(m->P, m->X, m->y, m->idx + b * batch, batch, wpos, m->per, nullptr, m->m1, m->m2,
+            launch_mlp_step(m->P, m->X, m->y, m->idx + b * batch, batch, wpos, m->part, nullptr, m->m1, m->m2,
                             m->adam_t, lr, m->loss + b, m->st);
         }
         HIPCK(hipGetLastError());
@@ -2032,17 +2037,14 @@ int ocfd_mlp_train(ocfd_mlp* m, int epochs, int batch, float lr, float wpos, uns
 int ocfd_mlp_predict(ocfd_mlp* m, long long first, int n, float* prob) {
     // FP32 forward on stored samples (the training arithmetic), for checks
     if (!m || !prob || n <= 0 || first < 0 || first + n > m->n) return fail(OCFD_ERR_ARG, "bad range");
-    TRY(mlp_ensure_batch(m, n));
-    launch_mlp_step(m->P, m->X + 24 * first, m->y + first, nullptr, n, 1.f, m->per, nullptr, m->m1, m->m2, 0, 0.f,
-                    m->grad + MLP_NPARAM, m->st);
+    if (n > m->prob_cap) {
+        TRY(mlp_alloc(m, (void**)&m->prob, sizeof(float) * (size_t)n));
+        m->prob_cap = n;
+    }
+    launch_mlp_predict(m->P, m->X + 24 * first, n, m->prob, m->st);
     HIPCK(hipGetLastError());
     HIPCK(hipStreamSynchronize(m->st));
-    // dz3 = (prob - y) with weight 1: recover prob from the per-sample vectors
-    const size_t ps = mlp_per_sample_floats();
-    std::vector<float> per(ps * (size_t)n), y((size_t)n);
-    HIPCK(hipMemcpy(per.data(), m->per, sizeof(float) * ps * (size_t)n, hipMemcpyDeviceToHost));
-    HIPCK(hipMemcpy(y.data(), m->y + first, sizeof(float) * (size_t)n, hipMemcpyDeviceToHost));
-    for (int i = 0; i < n; i++) prob[i] = per[(size_t)i * ps + ps - 2] + y[(size_t)i];
+    HIPCK(hipMemcpy(prob, m->prob, sizeof(float) * (size_t)n, hipMemcpyDeviceToHost));
     return 0;
 }
 

@@ -241,12 +241,14 @@ template <typename S> void launch_mlp_sensor(const MlpSensorArgsT<S>& a, int pla
 template <typename S> void launch_mlp_collect(const MlpSensorArgsT<S>& a, int stride, float* X, float* y, hipStream_t st);
 long long mlp_collect_count(const Geo& g, int stride);
 // One training step on the nb samples idx[0..nb) of (X, y) (idx null: rows
-// 0..nb): per-sample vectors into per (nb * mlp_per_sample_floats()), the
+// 0..nb): partial gradient sums into part (mlp_part_floats(nb) floats), the
 // batch-mean gradient into grad (may be null), the mean loss into *loss, and
 // with adam_t > 0 the Adam update of params (moments m1, m2).
-void launch_mlp_step(float* params, const float* X, const float* y, const int* idx, int nb, float wpos, float* per,
+void launch_mlp_step(float* params, const float* X, const float* y, const int* idx, int nb, float wpos, float* part,
                      float* grad, float* m1, float* m2, int adam_t, float lr, float* loss, hipStream_t st);
-size_t mlp_per_sample_floats();
+size_t mlp_part_floats(int nb);
+// FP32 forward probabilities of rows 0..nb of X.
+void launch_mlp_predict(const float* params, const float* X, int nb, float* prob, hipStream_t st);
 
 // dst[i] = (To)src[i] for n elements (precision conversion of whole fields).
 template <typename To, typename From>
