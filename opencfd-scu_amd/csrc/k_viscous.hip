@@ -23,8 +23,7 @@
 // double.
 //
 // Both use 2.5-D blocking: a block owns a TX x TY tile of (x,y) columns and
-// marches through a chunk of z planes (32 on the FP64 path; 16 on the FP32
-// path).  x and y neighbours come from the
+// marches through a chunk of z planes (chunk_planes).  x and y neighbours come from the
 // current plane staged in LDS with its 4-point halo; z neighbours come from a
 // 9-plane queue each thread keeps in registers for its own column.
 #include <type_traits>
@@ -121,17 +120,16 @@ struct Tile25 {
     int i0, j0, i, j, kbeg, kend;
     bool own;
 };
-template <typename S, bool DIV, int TYB = TY_<S>::v>
-__device__ __forceinline__ Tile25 tile_of(const Geo& g) {
-    constexpr int KZ = KZ_<S, DIV>::v;
+template <int TYB>
+__device__ __forceinline__ Tile25 tile_of(const Geo& g, int kz) {
     Tile25 t;
     const Blk B = xcd_block();
     t.i0 = B.x * TX;
     t.j0 = B.y * TYB;
     t.i = t.i0 + threadIdx.x;
     t.j = t.j0 + threadIdx.y;
-    t.kbeg = B.z * KZ;
-    t.kend = min(t.kbeg + KZ, g.nz);
+    t.kbeg = B.z * kz;
+    t.kend = min(t.kbeg + kz, g.nz);
     t.own = t.i < g.nx && t.j < g.ny;
     return t;
 }
@@ -234,11 +232,11 @@ __device__ __forceinline__ bool near_closure(const ViscArgsT<S>& A, const Tile25
 // layers, stored as 0).  Loads for plane k+1 are issued before plane k is
 // computed.
 template <int SV, typename S>
-__global__ void __launch_bounds__(TX * TY_<S>::v) k_visc_gf(ViscArgsT<S> A) {
+__global__ void __launch_bounds__(TX * TY_<S>::v) k_visc_gf(ViscArgsT<S> A, int kz) {
     constexpr int TY = TY_<S>::v, NT = TX * TY;
     constexpr int PW = TX + 8, PN = PW * (TY + 8), NSL = (PN + NT - 1) / NT;
     const Geo& g = A.g;
-    const Tile25 t = tile_of<S, false>(g);
+    const Tile25 t = tile_of<TY>(g, kz);
     const int tx = threadIdx.x, ty = threadIdx.y, tid = ty * TX + tx;
     const int i0 = t.i0, j0 = t.j0;
     const S rhx = S(1.0 / g.hx), rhy = S(1.0 / g.hy), rhz = S(1.0 / g.hz);
@@ -408,11 +406,11 @@ __global__ void __launch_bounds__(TX * TY_<S>::v) k_visc_gf(ViscArgsT<S> A) {
 // registers).
 constexpr int NTD = TX * TYD;
 template <int SV, typename S, int NC, bool SEP>
-__global__ void __launch_bounds__(NTD) k_visc_div(ViscArgsT<S> A, int c0) {
+__global__ void __launch_bounds__(NTD) k_visc_div(ViscArgsT<S> A, int c0, int kz) {
     constexpr int XW = TX + 8, XN = TYD * XW, YN = (TYD + 8) * TX;
     constexpr int NSX = (XN + NTD - 1) / NTD, NSY = (YN + NTD - 1) / NTD;
     const Geo& g = A.g;
-    const Tile25 t = tile_of<S, true, TYD>(g);
+    const Tile25 t = tile_of<TYD>(g, kz);
     const int tx = threadIdx.x, ty = threadIdx.y, tid = ty * TX + tx;
     const int i0 = t.i0, j0 = t.j0;
     const S rhx = S(1.0 / g.hx), rhy = S(1.0 / g.hy), rhz = S(1.0 / g.hz);
@@ -572,18 +570,42 @@ __global__ void __launch_bounds__(256) k_qcrit(ViscArgsT<S> A, double* __restric
     qout[qi] = (ux * vy + ux * wz + vy * wz - uy * vx - uz * wx - vz * wy) * aj * aj;
 }
 
+// z planes per block.  A launch that does not fill the chip is bound by the
+// longest march: its planes are spread over as many blocks as the GPU holds
+// at once (2 per CU of the FP64 gradient kernel, 3 of the FP32 one, 4 of the
+// divergence), each block paying the 8 planes of its z queue again from
+// L2.  Measured, one gradient and one divergence launch, against the fixed
+// chunks: 64^3 82 -> 17.5 us and 38 -> 9.0, 61x47x39 84 -> 13.2 and 38.5 ->
+// 7.8, 203x93x45 142 -> 53.5 and 55 -> 21.2; 512x128x64, which 32 planes
+// fill exactly, keeps them (16: 196 -> 204 us).  Larger launches take the
+// fixed chunk, where the extra z reads are what counts.
 template <typename S, bool DIV>
-dim3 grid25(const Geo& g) {
-    constexpr int KZ = KZ_<S, DIV>::v, TYB = DIV ? TYD : TY_<S>::v;
-    return dim3((g.nx + TX - 1) / TX, (g.ny + TYB - 1) / TYB, (g.nz + KZ - 1) / KZ);
+int chunk_planes(const Geo& g, int cols) {
+    constexpr int RES = 256 * (DIV ? 4 : std::is_same<S, double>::value ? 2 : 3);
+    constexpr int MOST = 32;
+    if (cols <= RES) {
+        const int nch = RES / cols, kz = (g.nz + nch - 1) / nch;
+        if (kz <= MOST) return kz;
+    }
+    return KZ_<S, DIV>::v;
+}
+
+template <typename S, bool DIV>
+dim3 grid25(const Geo& g, int& kz) {
+    constexpr int TYB = DIV ? TYD : TY_<S>::v;
+    const int gx = (g.nx + TX - 1) / TX, gy = (g.ny + TYB - 1) / TYB;
+    kz = chunk_planes<S, DIV>(g, gx * gy);
+    return dim3(gx, gy, (g.nz + kz - 1) / kz);
 }
 
 }  // namespace
 
 template <typename S>
 void launch_visc_gf(const ViscArgsT<S>& a, hipStream_t st) {
-    if (a.svis == OCFD_CD6) hipLaunchKernelGGL((k_visc_gf<OCFD_CD6, S>), (grid25<S, false>(a.g)), dim3(TX, TY_<S>::v), 0, st, a);
-    else hipLaunchKernelGGL((k_visc_gf<OCFD_CD8, S>), (grid25<S, false>(a.g)), dim3(TX, TY_<S>::v), 0, st, a);
+    int kz;
+    const dim3 grid = grid25<S, false>(a.g, kz), blk(TX, TY_<S>::v);
+    if (a.svis == OCFD_CD6) hipLaunchKernelGGL((k_visc_gf<OCFD_CD6, S>), grid, blk, 0, st, a, kz);
+    else hipLaunchKernelGGL((k_visc_gf<OCFD_CD8, S>), grid, blk, 0, st, a, kz);
 }
 // Flux components per divergence launch: two (measured on the 1024x384x256
 // swept ramp: FP64 3.00-3.30 ms per stage for two launches of two against
@@ -604,13 +626,14 @@ template <typename S>
 void launch_visc_div(const ViscArgsT<S>& a, int c0, hipStream_t st) {
     constexpr int NC = NC_<S>::v;
     // SEP: the terms go to dv (set) or are added to du (null)
-    const dim3 grid = grid25<S, true>(a.g), blk(TX, TYD);
+    int kz;
+    const dim3 grid = grid25<S, true>(a.g, kz), blk(TX, TYD);
     if (a.svis == OCFD_CD6) {
-        if (a.dv) hipLaunchKernelGGL((k_visc_div<OCFD_CD6, S, NC, true>), grid, blk, 0, st, a, c0);
-        else hipLaunchKernelGGL((k_visc_div<OCFD_CD6, S, NC, false>), grid, blk, 0, st, a, c0);
+        if (a.dv) hipLaunchKernelGGL((k_visc_div<OCFD_CD6, S, NC, true>), grid, blk, 0, st, a, c0, kz);
+        else hipLaunchKernelGGL((k_visc_div<OCFD_CD6, S, NC, false>), grid, blk, 0, st, a, c0, kz);
     } else {
-        if (a.dv) hipLaunchKernelGGL((k_visc_div<OCFD_CD8, S, NC, true>), grid, blk, 0, st, a, c0);
-        else hipLaunchKernelGGL((k_visc_div<OCFD_CD8, S, NC, false>), grid, blk, 0, st, a, c0);
+        if (a.dv) hipLaunchKernelGGL((k_visc_div<OCFD_CD8, S, NC, true>), grid, blk, 0, st, a, c0, kz);
+        else hipLaunchKernelGGL((k_visc_div<OCFD_CD8, S, NC, false>), grid, blk, 0, st, a, c0, kz);
     }
 }
 template <typename S>
