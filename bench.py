@@ -38,8 +38,9 @@ ALGO_BYTES = {
     "sweep_y": (5 + 3 + 5 + 5) * 8,       # same + read-modify-write du(5)
     "sweep_z": (5 + 3 + 5 + 5) * 8,
     "visc_flux": (4 + 10 + 12) * 8,       # u,v,w,T, 9 cofactors + Ajac; write 12 Ev (mu formed from T)
-    "visc_div": (2 * 3 + 2) * 8,          # two flux components per launch: their 6 Ev; write 2 dv
-    "stage": (5 + 4 + 1 + 5 + 5 + 5 + 5) * 8,  # du, dv, Ajac, fn, f; write f, 5 primitives (stages 2-3; p in 3)
+    # divergence and RK stage: 12 Ev, du, Ajac, fn; write 5 primitives; the
+    # primitives in stages 2-3; f and p written in stage 3 (mean of the stages)
+    "visc_stage": (12 + 5 + 1 + 5 + 5) * 8 + (2 * 5 + 6) * 8 / 3,
     "sensor": 2 * 8 + 3,                  # rho, T; write 3 int8 flags
 }
 

@@ -10,12 +10,12 @@
 //                contravariant viscous fluxes Ev1..4 of all three directions
 //                (vis_flux_ker, src/OCFD_NS_Jacobian3d.cu:80-281).  The
 //                gradients never leave registers.
-//   k_visc_div : du[1..4] += Ajac*d(Ev)/dxi, then eta, then zeta (OCFD_d?0 of
-//                Ev + YF_Pe_XF, src/OCFD_NS_Jacobian3d.cu:304-440,
-//                src/commen_kernel.cu:158-169), no atomics; on the FP64 path
-//                the three terms go to their own buffer dv instead and the
-//                RK stage adds du + dv, so that the divergence need not wait
-//                for the inviscid sweeps.
+//   k_visc_div : d(Ev)/dxi + d(Ev)/deta + d(Ev)/dzeta (OCFD_d?0 of Ev +
+//                YF_Pe_XF, src/OCFD_NS_Jacobian3d.cu:304-440,
+//                src/commen_kernel.cu:158-169), no atomics, and with it the
+//                RK stage of the point; or, for callers that want the
+//                right-hand side in memory, the divergence alone (FP64: into
+//                its own buffer dv, so that it may run beside the sweeps).
 //   k_qcrit    : the Q criterion of the analysis events (same derivatives).
 //
 // S (double or float) is the type of u,v,w,T, mu, the derivatives, the
@@ -400,92 +400,135 @@ __global__ void __launch_bounds__(TX * TY_<S>::v) k_visc_gf(ViscArgsT<S> A, int 
     }
 }
 
-// Ev_x (4 fields) needs x neighbours, Ev_y y neighbours, Ev_z z neighbours.
-// One launch handles NC of the four flux components, starting at c0 (each
-// component is independent; fewer components per launch need fewer
-// registers).
+// prim->cons of one point (pri_to_cons_kernel, src/commen_kernel.cu:32-64).
+__device__ __forceinline__ void p2c5(double d, double u, double v, double w, double T, double cv, double* f) {
+    f[0] = d;
+    f[1] = u * d;
+    f[2] = v * d;
+    f[3] = w * d;
+    f[4] = d * ((u * u + v * v + w * w) * 0.5 + cv * T);
+}
+
+// The divergence of Ev (Ev_x needs x neighbours, Ev_y y neighbours, Ev_z z
+// neighbours; periodic neighbours are read where they are, so the Ev ghost
+// layers are never filled and stay 0) and, with KRK = 1..3, the RK stage of
+// the point that it completes: the viscous terms never go to memory.  KRK = 0
+// leaves the right-hand side in memory (dv, or added to du) for the callers
+// that want it there.
+//
+// The stage as OCFD_time_advance_ker1/2/3 (src/OCFD_time.cu:44-94) with
+// cons->prim + p (cons_to_pri_kernel, src/commen_kernel.cu:77-109).  FP64: the
+// conserved state of stages 1 and 2 is not written; the next stage forms it
+// from the primitives, which hold the same state in the same precision (an
+// ulp).  The mixed path, whose primitives are FP32, keeps f in every stage.
+// G.faces: f of the six faces from the primitives as OCFD_bc leaves it
+// (src/OCFD_boundary.cu:40-91), for runs whose boundary condition changes
+// nothing else; G.ghost[dir]: the point's copy in the periodic ghost layers.
+//
+// Bound by HBM.  The strips of the next plane are in flight while a plane is
+// computed.  All accesses are raw buffer accesses (Buf): with plain pointers
+// the 40 addresses of a point took the kernel to 255 VGPRs and spills, 2 waves
+// per SIMD; with them it needs 168 (3 waves), FP32 114 (4 waves).  Divergence
+// and stage as one launch against three (two of two flux components, then the
+// stage): 1024x256x128 2.42 -> 2.02 ms, 512x128x64 296 -> 224 us, mixed 215 ->
+// 170 us, 640x192x96 mixed 567 -> 467 us.
 constexpr int NTD = TX * TYD;
-template <int SV, typename S, int NC, bool SEP>
-__global__ void __launch_bounds__(NTD) k_visc_div(ViscArgsT<S> A, int c0, int kz) {
-    constexpr int XW = TX + 8, XN = TYD * XW, YN = (TYD + 8) * TX;
-    constexpr int NSX = (XN + NTD - 1) / NTD, NSY = (YN + NTD - 1) / NTD;
+template <int SV, typename S, int KRK>
+__global__ void __launch_bounds__(NTD, sizeof(S) == 8 ? 3 : 4) k_visc_div(ViscArgsT<S> A, StageArgsT<S> G, int kz) {
+    static_assert(TYD == 8, "one y-halo value per thread: 8 halo rows of TX columns");
+    constexpr bool FROM_PRIM = std::is_same<S, double>::value;  // f of stages 1 and 2 lives in the primitives
+    // FP64: the point's values after the derivatives, whose registers they
+    // take over (3 waves per SIMD); FP32 has room for them before
+    constexpr bool LATE = sizeof(S) == 8;
+    constexpr int XW = TX + 8, NC = 4;
     const Geo& g = A.g;
     const Tile25 t = tile_of<TYD>(g, kz);
     const int tx = threadIdx.x, ty = threadIdx.y, tid = ty * TX + tx;
-    const int i0 = t.i0, j0 = t.j0;
     const S rhx = S(1.0 / g.hx), rhy = S(1.0 / g.hy), rhz = S(1.0 / g.hz);
-    __shared__ S ex[NC][XN];
-    __shared__ S ey[NC][YN];
+    __shared__ S ex[NC][TYD * XW];
+    __shared__ S ey[NC][(TYD + 8) * TX];
     const long long fs = A.fs;
-    const S* EX = A.ev + c0 * fs;
-    const S* EY = A.ev + (4 + c0) * fs;
-    const S* EZ = A.ev + (8 + c0) * fs;
-    const int ic = min(t.i, g.nx - 1), jc = min(t.j, g.ny - 1);
-    const long long col = gidx(g, ic, jc, 0);
-    int slx[NSX], sly[NSY];
-    long long sox[NSX], soy[NSY];
+    // byte offset of (i, j) in a plane; i and j up to the ghost layers,
+    // wrapped where the direction is periodic
+    auto off = [&](int i, int j) { return (unsigned)((i + 4) + g.ldx * (j + 4)) * (unsigned)sizeof(S); };
+    auto wrap = [](int i, int n, int per) { return per ? (i < 0 ? i + n : i >= n ? i - n : i) : i; };
+    auto off_x = [&](int i, int j) { return i < g.nx + 4 && j < g.ny ? off(wrap(i, g.nx, A.per[0]), j) : BUF_NONE; };
+    auto off_y = [&](int i, int j) { return i < g.nx && j < g.ny + 4 ? off(i, wrap(j, g.ny, A.per[1])) : BUF_NONE; };
+    // halo: x strips of 4 + 4 columns (the first 8 * TYD threads), y strips of
+    // 4 + 4 rows (one value per thread)
+    const int hc = tid & 7, hr = (tid >> 3) & (TYD - 1);
+    const bool xh = tid < 8 * TYD;
+    const unsigned oo = t.own ? off(t.i, t.j) : BUF_NONE;
+    const unsigned od = t.own ? oo / (unsigned)sizeof(S) * 8u : BUF_NONE;  // in the FP64 fields
+    const unsigned ox = off_x(t.i, t.j), oy = off_y(t.i, t.j);
+    const unsigned oxh = xh ? off_x(hc < 4 ? t.i0 - 4 + hc : t.i0 + TX + hc - 4, t.j0 + hr) : BUF_NONE;
+    const unsigned oyh = off_y(t.i, ty < 4 ? t.j0 - 4 + ty : t.j0 + TYD + ty - 4);
+    const int lx = ty * XW + tx + 4, lxh = hr * XW + (hc < 4 ? hc : TX + hc);
+    const int ly = (ty + 4) * TX + tx, lyh = (ty < 4 ? ty : TYD + ty) * TX + tx;
+    auto zwrap = [&](int k) { return A.per[2] ? (k < 0 ? k + g.nz : k >= g.nz ? k - g.nz : k) : k; };
+    // plane k of field m of a group
+    auto bs = [&](const S* base, int m, int k) { return Buf<S>(base + m * fs + (long long)(k + 4) * g.sz, g.sz); };
+    auto bd = [&](const double* base, int m, int k) { return Buf<double>(base + m * fs + (long long)(k + 4) * g.sz, g.sz); };
+
+    S xv[NC], yv[NC], xhv[NC] = {}, yhv[NC], q[NC][9], nq[NC];
+    auto load_strips = [&](int k) {
 #pragma unroll
-    for (int r = 0; r < NSX; r++) {
-        const int p = tid + NTD * r;
-        const int hx = p % XW, hy = p / XW;
-        const int gi = i0 - 4 + hx, gj = j0 + hy;
-        slx[r] = p < XN ? p : -1;
-        sox[r] = (gi <= g.nx + 3 && gj < g.ny) ? gidx(g, gi, gj, 0) : -1;
-    }
+        for (int f = 0; f < NC; f++) xv[f] = bs(A.ev, f, k).ld(ox);
 #pragma unroll
-    for (int r = 0; r < NSY; r++) {
-        const int p = tid + NTD * r;
-        const int hx = p % TX, hy = p / TX;
-        const int gi = i0 + hx, gj = j0 - 4 + hy;
-        sly[r] = p < YN ? p : -1;
-        soy[r] = (gi < g.nx && gj <= g.ny + 3) ? gidx(g, gi, gj, 0) : -1;
-    }
-    S xv[NSX][NC], yv[NSY][NC];
-    auto load_plane = [&](int k) {
-        const long long pk = (long long)k * g.sz;
+        for (int f = 0; f < NC; f++) yv[f] = bs(A.ev, 4 + f, k).ld(oy);
 #pragma unroll
-        for (int r = 0; r < NSX; r++)
+        for (int f = 0; f < NC; f++) yhv[f] = bs(A.ev, 4 + f, k).ld(oyh);
+        if (xh)
 #pragma unroll
-            for (int f = 0; f < NC; f++) xv[r][f] = (slx[r] >= 0 && sox[r] >= 0) ? EX[f * fs + sox[r] + pk] : S(0);
-#pragma unroll
-        for (int r = 0; r < NSY; r++)
-#pragma unroll
-            for (int f = 0; f < NC; f++) yv[r][f] = (sly[r] >= 0 && soy[r] >= 0) ? EY[f * fs + soy[r] + pk] : S(0);
+            for (int f = 0; f < NC; f++) xhv[f] = bs(A.ev, f, k).ld(oxh);
     };
-    S q[NC][9], nq[NC];
+    // the stage's own values of the point: du, Ajac, the base state fn and
+    // the state before the stage (the primitives, or f on the mixed path)
+    double sr[5], sj = 0.0, sn[5], so[5];
+    auto load_point = [&](int k) {
+        if (KRK || !A.dv)
+#pragma unroll
+            for (int m = 0; m < 5; m++) sr[m] = double(bs(A.du, m, k).template ld<BUF_STREAM>(oo));
+        if (!KRK) return;
+        sj = bd(G.jac, 0, k).template ld<BUF_STREAM>(od);
+#pragma unroll
+        for (int m = 0; m < 5; m++) sn[m] = bd(G.fn, m, k).template ld<BUF_STREAM>(od);
+        if (KRK == 1) return;
+#pragma unroll
+        for (int m = 0; m < 5; m++)
+            so[m] = FROM_PRIM ? double(bs(G.d, m, k).ld(oo)) : bd(G.f, m, k).template ld<BUF_STREAM>(od);
+    };
 #pragma unroll
     for (int m = 0; m < 8; m++)
 #pragma unroll
-        for (int f = 0; f < NC; f++) q[f][m] = EZ[f * fs + col + (long long)(t.kbeg - 4 + m) * g.sz];
+        for (int f = 0; f < NC; f++) q[f][m] = bs(A.ev, 8 + f, zwrap(t.kbeg - 4 + m)).ld(oo);
+    auto load_next = [&](int k) {
 #pragma unroll
-    for (int f = 0; f < NC; f++) nq[f] = EZ[f * fs + col + (long long)(t.kbeg + 4) * g.sz];
-    load_plane(t.kbeg);
+        for (int f = 0; f < NC; f++) nq[f] = bs(A.ev, 8 + f, zwrap(k)).ld(oo);
+    };
+    load_next(t.kbeg + 4);
+    load_strips(t.kbeg);
     for (int k = t.kbeg; k < t.kend; k++) {
-        if (!VISC_PREFETCH && k > t.kbeg) {
-#pragma unroll
-            for (int f = 0; f < NC; f++) nq[f] = EZ[f * fs + col + (long long)(k + 4) * g.sz];
-            load_plane(k);
-        }
 #pragma unroll
         for (int f = 0; f < NC; f++) {
             q[f][8] = nq[f];
-#pragma unroll
-            for (int r = 0; r < NSX; r++)
-                if (slx[r] >= 0) ex[f][slx[r]] = xv[r][f];
-#pragma unroll
-            for (int r = 0; r < NSY; r++)
-                if (sly[r] >= 0) ey[f][sly[r]] = yv[r][f];
+            ex[f][lx] = xv[f];
+            ey[f][ly] = yv[f];
+            ey[f][lyh] = yhv[f];
+            if (xh) ex[f][lxh] = xhv[f];
         }
         __syncthreads();
-        if (VISC_PREFETCH && k + 1 < t.kend) {
-#pragma unroll
-            for (int f = 0; f < NC; f++) nq[f] = EZ[f * fs + col + (long long)(k + 5) * g.sz];
-            load_plane(k + 1);
+        if (k + 1 < t.kend) {
+            load_next(k + 5);
+            load_strips(k + 1);
         }
-        // CL = false: no closure in reach of the block's plane (straight-line code)
-        auto point = [&](auto cl) {
+        // CL = false: no closure in reach of the block's plane (straight-line
+        // code).  The sums are double; the node's Ajac, by which the reference
+        // multiplies each of these terms, is applied to the whole right-hand
+        // side by the RK stage.
+        double dv[NC];
+        auto derivs = [&](auto cl) {
             constexpr bool CL = decltype(cl)::value;
-            const long long qi = gidx(g, t.i, t.j, k);
 #pragma unroll
             for (int m = 0; m < NC; m++) {
                 S s[9];
@@ -496,27 +539,57 @@ __global__ void __launch_bounds__(NTD) k_visc_div(ViscArgsT<S> A, int c0, int kz
                 for (int r = 0; r < 9; r++) s[r] = ey[m][(ty + r) * TX + tx];
                 const S vy = cd9<SV, S, CL>(s, t.j, g.ny, A.bnd[2], A.bnd[3], rhy);
                 const S vz = cd9<SV, S, CL>(q[m], k, g.nz, A.bnd[4], A.bnd[5], rhz);
-                // the sums are double; the node's Ajac, by which the
-                // reference multiplies each of these terms, is applied to the
-                // whole right-hand side by the RK stage
-                if (SEP) {
-                    double acc = double(vx);
-                    acc = acc + double(vy);
-                    acc = acc + double(vz);
-                    A.dv[(long long)(c0 + m) * fs + qi] = S(acc);
-                } else {
-                    S* du = A.du + (long long)(c0 + m + 1) * fs + qi;
-                    double acc = double(*du);
-                    acc = acc + double(vx);
-                    acc = acc + double(vy);
-                    acc = acc + double(vz);
-                    *du = S(acc);
-                }
+                dv[m] = (double(vx) + double(vy)) + double(vz);
             }
         };
-        if (t.own) {
-            if (near_closure<TYD>(A, t, k)) point(std::true_type{});
-            else point(std::false_type{});
+        if (!LATE) load_point(k);
+        if (near_closure<TYD>(A, t, k)) derivs(std::true_type{});
+        else derivs(std::false_type{});
+        if (LATE) load_point(k);
+        if (!KRK) {
+#pragma unroll
+            for (int m = 0; m < NC; m++) {
+                if (A.dv) bs(A.dv, m, k).st(oo, S(dv[m]));
+                else bs(A.du, m + 1, k).st(oo, S(sr[m + 1] + dv[m]));
+            }
+        } else {
+            const double dt = G.dt;
+            double fo[5], fv[5];
+            if (KRK > 1) {
+                if (FROM_PRIM) p2c5(so[0], so[1], so[2], so[3], so[4], G.c.cv, fo);
+                else
+#pragma unroll
+                    for (int m = 0; m < 5; m++) fo[m] = so[m];
+            }
+#pragma unroll
+            for (int m = 0; m < 5; m++) {
+                const double r = (m ? sr[m] + dv[m - 1] : sr[m]) * sj;
+                if (KRK == 1) fv[m] = sn[m] + dt * r;
+                else if (KRK == 2) fv[m] = 3.0 / 4.0 * sn[m] + 1.0 / 4.0 * (fo[m] + dt * r);
+                else fv[m] = 1.0 / 3.0 * sn[m] + 2.0 / 3.0 * (fo[m] + dt * r);
+            }
+            const double d1 = fv[0], u1 = fv[1] / d1, v1 = fv[2] / d1, w1 = fv[3] / d1;
+            const double T2 = (fv[4] - 0.5 * d1 * (u1 * u1 + v1 * v1 + w1 * w1)) / (d1 * G.c.cv);
+            const S pr[5] = {S(d1), S(u1), S(v1), S(w1), S(T2)};
+#pragma unroll
+            for (int m = 0; m < 5; m++) bs(G.d, m, k).st(oo, pr[m]);
+            if (KRK == 3) bs(G.P, 0, k).template st<BUF_STREAM>(oo, S(T2 * d1 / (G.c.gamma * G.c.ama * G.c.ama)));
+            if (KRK == 3 || !FROM_PRIM) {
+                if (KRK == 3 && G.flap)
+#pragma unroll
+                    for (int m = 0; m < 5; m++) bd(G.flap, m, k).template st<BUF_STREAM>(od, fv[m]);
+                if (G.faces && (t.i == 0 || t.i == g.nx - 1 || t.j == 0 || t.j == g.ny - 1 || k == 0 || k == g.nz - 1))
+                    p2c5(double(pr[0]), double(pr[1]), double(pr[2]), double(pr[3]), double(pr[4]), G.c.cv, fv);
+#pragma unroll
+                for (int m = 0; m < 5; m++) bd(G.f, m, k).template st<BUF_STREAM>(od, fv[m]);
+            }
+            auto copy_to = [&](int kk, unsigned o) {
+#pragma unroll
+                for (int m = 0; m < 5; m++) bs(G.d, m, kk).st(o, pr[m]);
+            };
+            if (G.ghost[0] && t.own && (t.i < 4 || t.i >= g.nx - 4)) copy_to(k, off(t.i < 4 ? t.i + g.nx : t.i - g.nx, t.j));
+            if (G.ghost[1] && t.own && (t.j < 4 || t.j >= g.ny - 4)) copy_to(k, off(t.i, t.j < 4 ? t.j + g.ny : t.j - g.ny));
+            if (G.ghost[2] && (k < 4 || k >= g.nz - 4)) copy_to(k < 4 ? k + g.nz : k - g.nz, oo);
         }
 #pragma unroll
         for (int f = 0; f < NC; f++)
@@ -572,16 +645,16 @@ __global__ void __launch_bounds__(256) k_qcrit(ViscArgsT<S> A, double* __restric
 
 // z planes per block.  A launch that does not fill the chip is bound by the
 // longest march: its planes are spread over as many blocks as the GPU holds
-// at once (2 per CU of the FP64 gradient kernel, 3 of the FP32 one, 4 of the
-// divergence), each block paying the 8 planes of its z queue again from
-// L2.  Measured, one gradient and one divergence launch, against the fixed
-// chunks: 64^3 82 -> 17.5 us and 38 -> 9.0, 61x47x39 84 -> 13.2 and 38.5 ->
-// 7.8, 203x93x45 142 -> 53.5 and 55 -> 21.2; 512x128x64, which 32 planes
+// at once (2 per CU of the FP64 kernels, 3 of the FP32 gradient kernel, 4 of
+// the FP32 divergence), each block paying the 8 planes of its z queue again
+// from L2.  Measured, a gradient launch, against the fixed chunks: 64^3 82 ->
+// 17.5 us, 61x47x39 84 -> 13.2, 203x93x45 142 -> 53.5 (a divergence of two
+// components 38 -> 9.0, 38.5 -> 7.8, 55 -> 21.2); 512x128x64, which 32 planes
 // fill exactly, keeps them (16: 196 -> 204 us).  Larger launches take the
 // fixed chunk, where the extra z reads are what counts.
 template <typename S, bool DIV>
 int chunk_planes(const Geo& g, int cols) {
-    constexpr int RES = 256 * (DIV ? 4 : std::is_same<S, double>::value ? 2 : 3);
+    constexpr int RES = 256 * (std::is_same<S, double>::value ? 2 : DIV ? 4 : 3);
     constexpr int MOST = 32;
     if (cols <= RES) {
         const int nch = RES / cols, kz = (g.nz + nch - 1) / nch;
@@ -607,34 +680,27 @@ void launch_visc_gf(const ViscArgsT<S>& a, hipStream_t st) {
     if (a.svis == OCFD_CD6) hipLaunchKernelGGL((k_visc_gf<OCFD_CD6, S>), grid, blk, 0, st, a, kz);
     else hipLaunchKernelGGL((k_visc_gf<OCFD_CD8, S>), grid, blk, 0, st, a, kz);
 }
-// Flux components per divergence launch: two (measured on the 1024x384x256
-// swept ramp: FP64 3.00-3.30 ms per stage for two launches of two against
-// 3.34-3.59 ms for four of one and 3.27-3.44 ms for one of four; the mixed
-// step 43.5 -> 43.0 ms with two launches of two instead of one of four; on
-// the 512x128x64 ramp four of one had been the fastest).
-#ifndef OCFD_VDIV_NC_D
-#define OCFD_VDIV_NC_D 2  // flux components per divergence launch, FP64 path
-#endif
-template <typename S> struct NC_ { static constexpr int v = OCFD_VDIV_NC_D; };
-#ifndef OCFD_VDIV_NC_F
-#define OCFD_VDIV_NC_F 2  // flux components per divergence launch, FP32 path
-#endif
-template <> struct NC_<float> { static constexpr int v = OCFD_VDIV_NC_F; };
-template <typename S>
-int visc_div_components() { return NC_<S>::v; }
-template <typename S>
-void launch_visc_div(const ViscArgsT<S>& a, int c0, hipStream_t st) {
-    constexpr int NC = NC_<S>::v;
-    // SEP: the terms go to dv (set) or are added to du (null)
+namespace {
+template <int SV, typename S>
+void launch_div(const ViscArgsT<S>& a, const StageArgsT<S>& st_, int krk, hipStream_t st) {
     int kz;
     const dim3 grid = grid25<S, true>(a.g, kz), blk(TX, TYD);
-    if (a.svis == OCFD_CD6) {
-        if (a.dv) hipLaunchKernelGGL((k_visc_div<OCFD_CD6, S, NC, true>), grid, blk, 0, st, a, c0, kz);
-        else hipLaunchKernelGGL((k_visc_div<OCFD_CD6, S, NC, false>), grid, blk, 0, st, a, c0, kz);
-    } else {
-        if (a.dv) hipLaunchKernelGGL((k_visc_div<OCFD_CD8, S, NC, true>), grid, blk, 0, st, a, c0, kz);
-        else hipLaunchKernelGGL((k_visc_div<OCFD_CD8, S, NC, false>), grid, blk, 0, st, a, c0, kz);
-    }
+    if (krk == 0) hipLaunchKernelGGL((k_visc_div<SV, S, 0>), grid, blk, 0, st, a, st_, kz);
+    else if (krk == 1) hipLaunchKernelGGL((k_visc_div<SV, S, 1>), grid, blk, 0, st, a, st_, kz);
+    else if (krk == 2) hipLaunchKernelGGL((k_visc_div<SV, S, 2>), grid, blk, 0, st, a, st_, kz);
+    else hipLaunchKernelGGL((k_visc_div<SV, S, 3>), grid, blk, 0, st, a, st_, kz);
+}
+}  // namespace
+template <typename S>
+void launch_visc_div(const ViscArgsT<S>& a, hipStream_t st) {
+    const StageArgsT<S> none{};
+    if (a.svis == OCFD_CD6) launch_div<OCFD_CD6>(a, none, 0, st);
+    else launch_div<OCFD_CD8>(a, none, 0, st);
+}
+template <typename S>
+void launch_visc_stage(const ViscArgsT<S>& a, const StageArgsT<S>& s, hipStream_t st) {
+    if (a.svis == OCFD_CD6) launch_div<OCFD_CD6>(a, s, s.krk, st);
+    else launch_div<OCFD_CD8>(a, s, s.krk, st);
 }
 template <typename S>
 void launch_qcrit(const ViscArgsT<S>& a, double* q, hipStream_t st) {
@@ -646,7 +712,7 @@ template void launch_qcrit<double>(const ViscArgsT<double>&, double*, hipStream_
 template void launch_qcrit<float>(const ViscArgsT<float>&, double*, hipStream_t);
 template void launch_visc_gf<double>(const ViscArgsT<double>&, hipStream_t);
 template void launch_visc_gf<float>(const ViscArgsT<float>&, hipStream_t);
-template void launch_visc_div<double>(const ViscArgsT<double>&, int, hipStream_t);
-template void launch_visc_div<float>(const ViscArgsT<float>&, int, hipStream_t);
-template int visc_div_components<double>();
-template int visc_div_components<float>();
+template void launch_visc_div<double>(const ViscArgsT<double>&, hipStream_t);
+template void launch_visc_div<float>(const ViscArgsT<float>&, hipStream_t);
+template void launch_visc_stage<double>(const ViscArgsT<double>&, const StageArgsT<double>&, hipStream_t);
+template void launch_visc_stage<float>(const ViscArgsT<float>&, const StageArgsT<float>&, hipStream_t);

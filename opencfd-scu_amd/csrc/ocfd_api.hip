@@ -109,6 +109,8 @@ struct ocfd_ctx {
     int fpara[OCFD_MAX_FILTERS][11];
     bool filter_dir[3] = {false, false, false};
     // profiling
+    // the last right-hand side's viscous part is still only in Ev (finish_rhs)
+    bool div_pending = false;
     bool prof = false;
     std::vector<ProfRec> recs;
     std::vector<hipEvent_t> pool;
@@ -302,11 +304,17 @@ int download_interior(ocfd_ctx* x, const double* src, double* dst) {
     return 0;
 }
 
+// IPERIODIC as a mask (bit 0: x, 1: y, 2: z).
+int periodic_dirs(const ocfd_ctx* x) {
+    int m = 0;
+    for (int dir = 0; dir < 3; dir++)
+        if (x->cfg.iperiodic[dir]) m |= 1 << dir;
+    return m;
+}
 template <typename T>
 int fill_periodic(ocfd_ctx* x, T* base, int nf, const char* name) {
-    for (int dir = 0; dir < 3; dir++)
-        if (x->cfg.iperiodic[dir])
-            TRY(timed(x, name, [&] { launch_fill(x->g, base, nf, x->fs, dir, x->st); }));
+    if (const int dirs = periodic_dirs(x))
+        TRY(timed(x, name, [&] { launch_fill(x->g, base, nf, x->fs, dirs, x->st); }));
     return 0;
 }
 
@@ -432,7 +440,26 @@ MlpSensorArgsT<S> mlp_args(ocfd_ctx* x) {
 }
 
 template <typename S>
-int rhs(ocfd_ctx* x, int krk) {
+ViscArgsT<S> visc_args(ocfd_ctx* x) {
+    const View<S> V = view<S>(x);
+    ViscArgsT<S> va;
+    va.g = x->g;
+    va.c = x->c;
+    va.svis = x->cfg.scheme_vis;
+    for (int q = 0; q < 6; q++) va.bnd[q] = x->cfg.dif_bound[q];
+    for (int q = 0; q < 3; q++) va.per[q] = x->cfg.iperiodic[q];
+    va.u = V.u; va.v = V.v; va.w = V.w; va.T = V.T; va.amu = V.amu;
+    for (int m = 0; m < M_COUNT; m++) va.M[m] = x->M[m];
+    va.ev = V.ev; va.du = V.du; va.dv = V.dv; va.fs = x->fs;
+    return va;
+}
+
+// The right-hand side of a stage: the inviscid part into du, the viscous
+// fluxes into Ev and, unless the caller's stage takes their divergence itself
+// (fused: launch_visc_stage), the viscous part into dv or du.  ghosts: the
+// periodic ghost layers of the primitives already hold the stage's state.
+template <typename S>
+int rhs(ocfd_ctx* x, int krk, bool fused = false, bool ghosts = false) {
     const ocfd_config& C = x->cfg;
     const View<S> V = view<S>(x);
     // hybrid_auto flags, once per step at the first stage: the plain sensor
@@ -449,7 +476,7 @@ int rhs(ocfd_ctx* x, int krk) {
     const bool fuse_learned = learned && x->mlp_fused && !C.charteric;
     if (C.scheme_invis == OCFD_HYBRIDAUTO && krk == 1 && !learned)
         TRY(timed(x, "sensor", [&] { launch_sensor(x->g, x->c, V.d, V.T, x->flag[0], x->flag[1], x->flag[2], x->st); }));
-    TRY(fill_prims<S>(x));
+    if (!ghosts) TRY(fill_prims<S>(x));
     const MlpSensorArgsT<S> ma = mlp_args<S>(x);
     if (learned) {
         if (!fuse_learned) {
@@ -459,27 +486,16 @@ int rhs(ocfd_ctx* x, int krk) {
             TRY(timed(x, "sensor_mlp_planes", [&] { launch_mlp_sensor(ma, 2, x->st); }));
         }
     }
-    ViscArgsT<S> va;
-    va.g = x->g;
-    va.c = x->c;
-    va.svis = C.scheme_vis;
-    for (int q = 0; q < 6; q++) va.bnd[q] = C.dif_bound[q];
-    va.u = V.u; va.v = V.v; va.w = V.w; va.T = V.T; va.amu = V.amu;
-    for (int m = 0; m < M_COUNT; m++) va.M[m] = x->M[m];
-    va.ev = V.ev; va.du = V.du; va.dv = V.dv; va.fs = x->fs;
+    const ViscArgsT<S> va = visc_args<S>(x);
     // the viscous terms read the primitives and metrics and write only Ev
     // and dv: on the second stream they overlap the sweeps (which write only
-    // du); the stage adds du + dv.  Kernel timing runs everything in order on
-    // one stream.
+    // du).  Kernel timing runs everything in order on one stream.
     const bool overlap = !x->prof && !x->serial;
     if (overlap) {
         HIPCK(hipEventRecord(x->ev_fork, x->st));
         HIPCK(hipStreamWaitEvent(x->st2, x->ev_fork, 0));
         launch_visc_gf(va, x->st2);
-        for (int dir = 0; dir < 3; dir++)
-            if (C.iperiodic[dir]) launch_fill(x->g, V.ev + 4LL * dir * x->fs, 4, x->fs, dir, x->st2);
-        if (va.dv)
-            for (int c0 = 0; c0 < 4; c0 += visc_div_components<S>()) launch_visc_div(va, c0, x->st2);
+        if (va.dv && !fused) launch_visc_div(va, x->st2);
         HIPCK(hipGetLastError());
         HIPCK(hipEventRecord(x->ev_join, x->st2));
     }
@@ -516,14 +532,24 @@ int rhs(ocfd_ctx* x, int krk) {
         HIPCK(hipStreamWaitEvent(x->st, x->ev_join, 0));
     } else {
         TRY(timed(x, "visc_flux", [&] { launch_visc_gf(va, x->st); }));
-        for (int dir = 0; dir < 3; dir++)
-            if (C.iperiodic[dir])
-                TRY(timed(x, "fill_ev", [&] { launch_fill(x->g, V.ev + 4LL * dir * x->fs, 4, x->fs, dir, x->st); }));
     }
-    if (!overlap || !va.dv)
-        for (int c0 = 0; c0 < 4; c0 += visc_div_components<S>())
-            TRY(timed(x, "visc_div", [&] { launch_visc_div(va, c0, x->st); }));
+    if (!fused && (!overlap || !va.dv)) TRY(timed(x, "visc_div", [&] { launch_visc_div(va, x->st); }));
+    x->div_pending = fused;
     return 0;
+}
+
+// The viscous part of the last right-hand side, where its stage took it from
+// Ev without leaving it in memory (Ev still holds that stage's fluxes).
+template <typename S>
+int finish_rhs_t(ocfd_ctx* x) {
+    const ViscArgsT<S> va = visc_args<S>(x);
+    TRY(timed(x, "visc_div", [&] { launch_visc_div(va, x->st); }));
+    x->div_pending = false;
+    return 0;
+}
+int finish_rhs(ocfd_ctx* x) {
+    if (!x->div_pending) return 0;
+    return x->mixed ? finish_rhs_t<float>(x) : finish_rhs_t<double>(x);
 }
 
 bool filter_due(ocfd_ctx* x, int istep) {
@@ -540,11 +566,14 @@ template <typename S>
 int do_filter(ocfd_ctx* x) {
     if (!filter_due(x, x->istep)) return 0;
     const View<S> V = view<S>(x);
+    int dirs = 0;
     for (int dir = 0; dir < 3; dir++)
-        if (x->filter_dir[dir] && x->cfg.iperiodic[dir]) {
-            TRY(timed(x, "fill_filter", [&] { launch_fill(x->g, V.P, 1, x->fs, dir, x->st); }));
-            TRY(timed(x, "fill_filter", [&] { launch_fill(x->g, x->flap, 5, x->fs, dir, x->st); }));
-        }
+        if (x->filter_dir[dir]) dirs |= 1 << dir;
+    dirs &= periodic_dirs(x);
+    if (dirs) {
+        TRY(timed(x, "fill_filter", [&] { launch_fill(x->g, V.P, 1, x->fs, dirs, x->st); }));
+        TRY(timed(x, "fill_filter", [&] { launch_fill(x->g, x->flap, 5, x->fs, dirs, x->st); }));
+    }
     for (int m = 0; m < x->cfg.nfilter; m++) {
         if (!(x->tt <= x->cfg.filter_rpara[m][2])) continue;
         const int* p = x->fpara[m];
@@ -588,6 +617,8 @@ StageArgsT<S> stage_args(ocfd_ctx* x, int krk, bool write_flap) {
     // the first two stages skip it
     sa.P = krk == 3 ? V.P : nullptr;
     sa.fs = x->fs;
+    sa.faces = 0;
+    for (int q = 0; q < 3; q++) sa.ghost[q] = 0;
     return sa;
 }
 
@@ -595,13 +626,18 @@ template <typename S>
 int one_step_t(ocfd_ctx* x) {
     std::swap(x->f, x->fn);
     const bool fdue = x->flap && filter_due(x, x->istep + 1);
+    // without a boundary condition nothing changes the primitives between a
+    // stage and the next right-hand side: the stage refreshes f on the faces
+    // and, before stages 2 and 3, writes the periodic ghost layers itself (at
+    // stage 1 the plain sensor still reads the layers of the stage before)
+    const bool plain = x->cfg.ibc == 0;
     for (int krk = 1; krk <= 3; krk++) {
-        // no viscosity field: the gradient kernel forms mu from T at its points
         StageArgsT<S> sa = stage_args<S>(x, krk, krk == 3 && fdue);
-        sa.amu = nullptr;
-        TRY(rhs<S>(x, krk));
-        TRY(timed(x, "stage", [&] { launch_stage(sa, x->st); }));
-        TRY(apply_bc<S>(x));
+        sa.faces = plain;
+        for (int q = 0; q < 3; q++) sa.ghost[q] = plain && krk < 3 && x->cfg.iperiodic[q];
+        TRY(rhs<S>(x, krk, true, plain && krk > 1));
+        TRY(timed(x, "visc_stage", [&] { launch_visc_stage(visc_args<S>(x), sa, x->st); }));
+        if (!plain) TRY(apply_bc<S>(x));
     }
     x->istep++;
     x->tt += x->cfg.dt;
@@ -1306,6 +1342,7 @@ int ocfd_get_state(ocfd_ctx* x, double* f5) {
 
 int ocfd_get_du(ocfd_ctx* x, double* du5) {
     if (!x || !du5) return fail(OCFD_ERR_ARG, "null argument");
+    TRY(finish_rhs(x));
     const size_t n = (size_t)x->g.nx * x->g.ny * x->g.nz;
     for (int m = 0; m < 5; m++)
         TRY(x->mixed ? download_any(x, x->sdu + m * x->fs, du5 + m * n)
@@ -2273,6 +2310,7 @@ void du_comput(int KRK) { SHIM(rhs_any(g_ctx, KRK)); }
 
 void OCFD_time_advance(int KRK) {
     ocfd_ctx* x = g_ctx;
+    SHIM(finish_rhs(x));
     const bool flap = KRK == 3 && x->flap && filter_due(x, x->istep + 1);
     if (x->mixed) {
         const StageArgsT<float> sa = stage_args<float>(x, KRK, flap);

@@ -52,6 +52,31 @@ __device__ __forceinline__ Blk xcd_block() {
     return o;
 }
 
+// Raw buffer access to a range of one array (a z plane of a field): the base
+// is a scalar resource and the lane's address one 32-bit byte offset, where a
+// plain pointer costs two registers and a 64-bit add per access.  Loads past
+// the range return 0 and stores past it are dropped, so lanes without a point
+// take the offset BUF_NONE instead of a branch.
+constexpr unsigned BUF_NONE = 0x80000000u;  // past every range: a plane holds at most 2^31 / 16 elements
+enum { BUF_PLAIN = 0, BUF_STREAM = 2 };     // cache policy: BUF_STREAM = non-temporal
+template <typename T> struct Buf {
+    __amdgpu_buffer_rsrc_t r;
+    __device__ __forceinline__ Buf(const T* base, long long elems)
+        : r(__builtin_amdgcn_make_buffer_rsrc(const_cast<T*>(base), 0, (int)(elems * (long long)sizeof(T)), 0x00020000)) {}
+    template <int AUX = BUF_PLAIN> __device__ __forceinline__ T ld(unsigned off) const {
+        if constexpr (sizeof(T) == 8) return __builtin_bit_cast(T, __builtin_amdgcn_raw_buffer_load_b64(r, (int)off, 0, AUX));
+        else return __builtin_bit_cast(T, __builtin_amdgcn_raw_buffer_load_b32(r, (int)off, 0, AUX));
+    }
+    template <int AUX = BUF_PLAIN> __device__ __forceinline__ void st(unsigned off, T v) const {
+        if constexpr (sizeof(T) == 8) {
+            typedef unsigned u2 __attribute__((ext_vector_type(2)));
+            __builtin_amdgcn_raw_buffer_store_b64(__builtin_bit_cast(u2, v), r, (int)off, 0, AUX);
+        } else {
+            __builtin_amdgcn_raw_buffer_store_b32(__builtin_bit_cast(unsigned, v), r, (int)off, 0, AUX);
+        }
+    }
+};
+
 // The 10 metric fields kept on the device (cofactors and Ajac,
 // src/OCFD_Comput_Jacobian3d.cu:285-295).
 enum { M_KX = 0, M_KY, M_KZ, M_IX, M_IY, M_IZ, M_SX, M_SY, M_SZ, M_JAC, M_COUNT };

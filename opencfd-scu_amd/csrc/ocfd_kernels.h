@@ -50,6 +50,7 @@ struct ViscArgsT {
     Consts c;
     int svis;                                // 203 / 204
     int bnd[6];                              // DIF_BOUND
+    int per[3];                              // IPERIODIC: Ev neighbours across the face are read wrapped
     const S *u, *v, *w, *T, *amu;
     const double *M[M_COUNT];
     S *ev;                                   // 12 fields: Ev1..4 for x, y, z
@@ -59,19 +60,18 @@ struct ViscArgsT {
 };
 // Gradients of u,v,w,T (kept in registers) and the 12 viscous fluxes.
 template <typename S> void launch_visc_gf(const ViscArgsT<S>& a, hipStream_t st);
-// The divergence in launches of visc_div_components<S>() flux components
-// each, starting at component c0 (0..3): written to dv when it is set (the
-// stage adds du + dv, so the divergence may run beside the inviscid sweeps),
-// else added to du after the sweeps.
-template <typename S> int visc_div_components();
-template <typename S> void launch_visc_div(const ViscArgsT<S>& a, int c0, hipStream_t st);
+// The divergence of the fluxes: written to dv when it is set (so that it may
+// run beside the inviscid sweeps), else added to du after the sweeps.
+template <typename S> void launch_visc_div(const ViscArgsT<S>& a, hipStream_t st);
 // Q criterion of u, v, w at every interior point into q (LAP layout, FP64).
 template <typename S> void launch_qcrit(const ViscArgsT<S>& a, double* q, hipStream_t st);
 
 // Periodic face fill (exchange_boundary_?_packed_dev at one rank): copy the
-// 4-layer faces of `nf` fields (stride fs) in direction dir.
+// 4-layer faces of `nf` fields (stride fs) in the directions of the mask
+// `dirs` (bit 0: x, 1: y, 2: z), in one launch (a face's source is interior
+// and its target a face ghost layer, so the directions are independent).
 template <typename T>
-void launch_fill(const Geo& g, T* base, int nf, long long fs, int dir, hipStream_t st);
+void launch_fill(const Geo& g, T* base, int nf, long long fs, int dirs, hipStream_t st);
 
 // RK stage + cons->prim + viscosity.
 template <typename S>
@@ -90,8 +90,18 @@ struct StageArgsT {
     S *amu;                                  // viscosity, or null (the stage then skips it)
     S *P;                                    // pressure, or null (the stage then skips it)
     long long fs;
+    // launch_visc_stage: f of the six faces from the primitives; periodic
+    // directions whose primitive ghost layers the stage writes as well
+    int faces;
+    int ghost[3];
 };
 template <typename S> void launch_stage(const StageArgsT<S>& a, hipStream_t st);
+// The divergence of the viscous fluxes and the RK stage in one pass (a.du
+// holds the inviscid part; the viscous part never goes to memory).  On the
+// FP64 path f is written in stage 3 only: stages 2 and 3 form it from the
+// primitives.
+template <typename S>
+void launch_visc_stage(const ViscArgsT<S>& a, const StageArgsT<S>& s, hipStream_t st);
 
 // SSP-RK3 stage of one point (OCFD_time_advance_ker1/2/3, src/OCFD_time.cu:
 // 44-94) with cons->prim + p (cons_to_pri_kernel, src/commen_kernel.cu:
