@@ -832,8 +832,12 @@ __device__ __forceinline__ void mv5(const double* M, const double* x, double* y)
 template <int DIR> struct CharTile { static constexpr int NS = 24, NA = 8; };
 template <> struct CharTile<0> { static constexpr int NS = 56, NA = 4; };
 
+// hybrid_auto is held to 3 waves per SIMD (168 VGPRs, 8 spilled): at 2 the
+// kernel is latency-bound (203x93x45, one launch: x 139 -> 111 us; y and z,
+// which were at 3, 79 -> 77 and 62 -> 60; at 4 waves 124, 90, 69).  The SYMBO
+// forms need 256 and would spill half of them.
 template <int DIR, int SCH, bool FIRST, typename S>
-__global__ void __launch_bounds__(256) k_char(SweepArgsT<S> A) {
+__global__ void __launch_bounds__(256, SCH == OCFD_HYBRIDAUTO ? 3 : 2) k_char(SweepArgsT<S> A) {
     constexpr int NS = CharTile<DIR>::NS, NA = CharTile<DIR>::NA, NN = NS + 8, NF = NS + 1;
     static_assert(NN * NA == 256 && NF * NA <= 256 && (DIR != 0 || (NA == 4 && NF <= 64)),
                   "one node and at most one face per thread; x: one row per wave");

@@ -10,6 +10,7 @@
 
 #include <hip/hip_runtime.h>
 #include <stdint.h>
+#include <type_traits>
 
 #define OCFD_LAPD 4
 
@@ -105,40 +106,61 @@ template <typename R> __device__ __forceinline__ R d_minmod4(R a, R b, R c, R d)
     return m * fmin(fmin(a, b), fmin(c, d));
 }
 
+// num / den of weights and weighted values, den > 0 and far from the ends of
+// the range: reciprocal by two Newton steps from the hardware's estimate and
+// one product (6 instructions; the IEEE division with its scaling, 12).
+// The quotients here are corrections to a nodal value, so their last ulp is
+// far below the ulp of the result.
+__device__ __forceinline__ double weight_div(double num, double den) {
+    double y = __builtin_amdgcn_rcp(den);
+    y = fma(fma(-den, y, 1.0), y, y);
+    y = fma(fma(-den, y, 1.0), y, y);
+    return num * y;
+}
+
 // WENO7 upwind (P) half-node value from nodes s[0..6] (src/OCFD_Schemes.cu:616-663).
 // R: type of the stencil values and smoothness indicators; W: type of the
 // epsilon/weight arithmetic (the mixed-precision path keeps W = double).
+//
+// The reference's sums over the stencil values, regrouped over the
+// differences the four sub-stencils share: e_i = s_{i+1} - s_i, D_i = e_i -
+// e_{i-1}, T_k = D_{k+2} - D_{k+1}.  Its a (first derivative at node 3), b =
+// 6 beta and c = 6 T are
+//   a = 6 e2 + 3 D2 + 2 T0, 3 (e2 + e3) - T1, 3 (e2 + e3) - T2, 6 e3 - 3 D4 + 2 T3
+//   beta = D2 + T0, D3, D4, D4 - T3   (its stencil 2 takes the node i+1)
+// its indicator 960 a^2 + 1040 b^2 + 1043 c^2 + 80 a c is 480 (a (2 a + T) +
+// 78 beta^2 + 78.225 T^2), and its candidates q_k are 12 s3 + delta_k.  The
+// weights do not change when epsilon and the indicators are divided by 480.
+// 88 instructions per value against about 130; cancellation happens in the
+// differences, which are exact for neighbouring values, and the weighted part
+// is a correction to s3: the error against 64-bit (and on the FP32 path
+// against FP64) values is no larger.
 template <typename R, typename W = R> __device__ __forceinline__ R weno7_up(const R* s) {
-    R a, b, c, S0, S1, S2, S3;
-    a = R(-2) * s[0] + R(9) * s[1] - R(18) * s[2] + R(11) * s[3];
-    b = R(-6) * s[0] + R(24) * s[1] - R(30) * s[2] + R(12) * s[3];
-    c = R(-6) * s[0] + R(18) * (s[1] - s[2]) + R(6) * s[3];
-    S0 = R(960) * a * a; S0 += R(1040) * b * b; S0 += R(1043) * c * c; S0 += R(80) * (a * c);
-    a = s[1] - R(6) * s[2] + R(3) * s[3] + R(2) * s[4];
-    b = R(6) * s[2] - R(12) * s[3] + R(6) * s[4];
-    c = R(-6) * s[1] + R(18) * (s[2] - s[3]) + R(6) * s[4];
-    S1 = R(960) * a * a; S1 += R(1040) * b * b; S1 += R(1043) * c * c; S1 += R(80) * (a * c);
-    a = R(-2) * s[2] - R(3) * s[3] + R(6) * s[4] - s[5];
-    b = R(6) * s[3] - R(12) * s[4] + R(6) * s[5];
-    c = R(-6) * s[2] + R(18) * (s[3] - s[4]) + R(6) * s[5];
-    S2 = R(960) * a * a; S2 += R(1040) * b * b; S2 += R(1043) * c * c; S2 += R(80) * (a * c);
-    a = R(-11) * s[3] + R(18) * s[4] - R(9) * s[5] + R(2) * s[6];
-    b = R(12) * s[3] - R(30) * s[4] + R(24) * s[5] - R(6) * s[6];
-    c = R(-6) * s[3] + R(18) * (s[4] - s[5]) + R(6) * s[6];
-    S3 = R(960) * a * a; S3 += R(1040) * b * b; S3 += R(1043) * c * c; S3 += R(80) * (a * c);
-    const W e = W(3.456e-4);
-    W q0 = (e + W(S0)) * (e + W(S0)), q1 = (e + W(S1)) * (e + W(S1)), q2 = (e + W(S2)) * (e + W(S2)),
-      q3 = (e + W(S3)) * (e + W(S3));
-    W w0 = q1 * q2 * q3;
-    W w1 = W(12) * q0 * q2 * q3;
-    W w2 = W(18) * q0 * q1 * q3;
-    W w3 = W(4) * q0 * q1 * q2;
-    W am = w0 + w1 + w2 + w3;
-    W r = w0 * W(R(-3) * s[0] + R(13) * s[1] - R(23) * s[2] + R(25) * s[3]);
-    r += w1 * W(s[1] - R(5) * s[2] + R(13) * s[3] + R(3) * s[4]);
-    r += w2 * W(-s[2] + R(7) * s[3] + R(7) * s[4] - s[5]);
-    r += w3 * W(R(3) * s[3] + R(13) * s[4] - R(5) * s[5] + s[6]);
-    return R(r / (W(12) * am));
+    const R e0 = s[1] - s[0], e1 = s[2] - s[1], e2 = s[3] - s[2], e3 = s[4] - s[3], e4 = s[5] - s[4], e5 = s[6] - s[5];
+    const R D1 = e1 - e0, D2 = e2 - e1, D3 = e3 - e2, D4 = e4 - e3, D5 = e5 - e4;
+    const R T0 = D2 - D1, T1 = D3 - D2, T2 = D4 - D3, T3 = D5 - D4;
+    const R m3 = R(3) * (e2 + e3);
+    const W e = W(3.456e-4 / 480.0);
+    auto ind = [&](R a, R be, R T) {  // epsilon + indicator, squared
+        W q;
+        if constexpr (std::is_same<R, W>::value)
+            q = fma(a, fma(R(2), a, T), fma(R(78) * be, be, fma(R(78.225) * T, T, e)));
+        else
+            q = e + W(fma(a, fma(R(2), a, T), fma(R(78) * be, be, R(78.225) * T * T)));
+        return q * q;
+    };
+    const W q0 = ind(fma(R(2), T0, fma(R(3), D2, R(6) * e2)), D2 + T0, T0);
+    const W q1 = ind(m3 - T1, D3, T1);
+    const W q2 = ind(m3 - T2, D4, T2);
+    const W q3 = ind(fma(R(2), T3, fma(R(-3), D4, R(6) * e3)), D4 - T3, T3);
+    const W q01 = q0 * q1, q23 = q2 * q3;
+    const W w0 = q1 * q23, w1 = W(12) * q0 * q23, w2 = W(18) * q01 * q3, w3 = W(4) * q01 * q2;
+    const W d0 = W(fma(R(13), e2, fma(R(-10), e1, R(3) * e0)));
+    const W d1 = W(fma(R(3), e3, fma(R(4), e2, -e1)));
+    const W d2 = W(fma(R(6), e3, e2 - e4));
+    const W d3 = W(fma(R(9), e3, fma(R(-4), e4, e5)));
+    const W num = fma(w3, d3, fma(w2, d2, fma(w1, d1, w0 * d0)));
+    return R(W(s[3]) + weight_div(num, W(12) * ((w0 + w1) + (w2 + w3))));
 }
 // WENO7 M side: the same reconstruction on the mirrored stencil
 // (src/OCFD_Schemes.cu:692-741); s[0..6].
@@ -230,44 +252,46 @@ template <typename R, typename W = R> __device__ __forceinline__ R weno5_dn_righ
 
 // WENO7-SYMBO (src/OCFD_Schemes.cu:391-589); P side with optional TV
 // limiter; the M side never takes the linear branch (TVmin stays 0).
+// Regrouped over shared differences like weno7_up: its indicators 720 t^2 +
+// 780 b^2 + 781 c^2 are 720 (a^2 + 39 beta^2 + 39.05 T^2), with a, beta, T of
+// stencils 0..3 as there and, for stencil 4, a = 26 e4 - 31 e5 + 11 e6, beta =
+// D5 - 2 T4.
 template <typename R, typename W = R> __device__ __forceinline__ R symbo_core(const R* s, bool linear) {
-    W S0, S1, S2, S3, S4;
+    const R e0 = s[1] - s[0], e1 = s[2] - s[1], e2 = s[3] - s[2], e3 = s[4] - s[3], e4 = s[5] - s[4], e5 = s[6] - s[5],
+            e6 = s[7] - s[6];
+    W w0, w1, w2, w3, w4;
     if (linear) {
-        S0 = W(0.0401954833730); S1 = W(0.2493800006710); S2 = W(0.4802686256260);
-        S3 = W(0.2009775476730); S4 = W(0.0291783426580);
+        w0 = W(0.0401954833730); w1 = W(0.2493800006710); w2 = W(0.4802686256260);
+        w3 = W(0.2009775476730); w4 = W(0.0291783426580);
     } else {
-        R t, B0, B1, B2, B3, B4;
-        t = R(-2) * s[0] + R(9) * s[1] - R(18) * s[2] + R(11) * s[3]; B0 = R(720) * t * t;
-        t = s[1] - R(6) * s[2] + R(3) * s[3] + R(2) * s[4]; B1 = R(720) * t * t;
-        t = R(-2) * s[2] - R(3) * s[3] + R(6) * s[4] - s[5]; B2 = R(720) * t * t;
-        t = R(-11) * s[3] + R(18) * s[4] - R(9) * s[5] + R(2) * s[6]; B3 = R(720) * t * t;
-        t = R(-26) * s[4] + R(57) * s[5] - R(42) * s[6] + R(11) * s[7]; B4 = R(720) * t * t;
-        t = R(-6) * s[0] + R(24) * s[1] - R(30) * s[2] + R(12) * s[3]; B0 += R(780) * t * t;
-        t = R(6) * s[2] - R(12) * s[3] + R(6) * s[4]; B1 += R(780) * t * t;
-        t = R(6) * s[3] - R(12) * s[4] + R(6) * s[5]; B2 += R(780) * t * t;
-        t = R(12) * s[3] - R(30) * s[4] + R(24) * s[5] - R(6) * s[6]; B3 += R(780) * t * t;
-        t = R(18) * s[4] - R(48) * s[5] + R(42) * s[6] - R(12) * s[7]; B4 += R(780) * t * t;
-        t = R(-6) * s[0] + R(18) * (s[1] - s[2]) + R(6) * s[3]; B0 += R(781) * t * t;
-        t = R(-6) * s[1] + R(18) * (s[2] - s[3]) + R(6) * s[4]; B1 += R(781) * t * t;
-        t = R(-6) * s[2] + R(18) * (s[3] - s[4]) + R(6) * s[5]; B2 += R(781) * t * t;
-        t = R(-6) * s[3] + R(18) * (s[4] - s[5]) + R(6) * s[6]; B3 += R(781) * t * t;
-        t = R(-6) * s[4] + R(18) * (s[5] - s[6]) + R(6) * s[7]; B4 += R(781) * t * t;
-        B4 = fmax(fmax(fmax(B0, B1), fmax(B2, B3)), B4);
-        const W e = W(2.592e-6);
-        W e0 = e + W(B0), e1 = e + W(B1), e2 = e + W(B2), e3 = e + W(B3), e4 = e + W(B4);
-        S0 = W(0.0401954833730) * e1 * e2 * e3 * e4;
-        S1 = W(0.2493800006710) * e0 * e2 * e3 * e4;
-        S2 = W(0.4802686256260) * e0 * e1 * e3 * e4;
-        S3 = W(0.2009775476730) * e0 * e1 * e2 * e4;
-        S4 = W(0.0291783426580) * e0 * e1 * e2 * e3;
+        const R D1 = e1 - e0, D2 = e2 - e1, D3 = e3 - e2, D4 = e4 - e3, D5 = e5 - e4, D6 = e6 - e5;
+        const R T0 = D2 - D1, T1 = D3 - D2, T2 = D4 - D3, T3 = D5 - D4, T4 = D6 - D5;
+        const R m3 = R(3) * (e2 + e3);
+        const W e = W(2.592e-6 / 720.0);
+        auto ind = [&](R a, R be, R T) {  // epsilon + indicator
+            if constexpr (std::is_same<R, W>::value) return fma(a, a, fma(R(39) * be, be, fma(R(39.05) * T, T, e)));
+            else return e + W(fma(a, a, fma(R(39) * be, be, R(39.05) * T * T)));
+        };
+        const W q0 = ind(fma(R(2), T0, fma(R(3), D2, R(6) * e2)), D2 + T0, T0);
+        const W q1 = ind(m3 - T1, D3, T1);
+        const W q2 = ind(m3 - T2, D4, T2);
+        const W q3 = ind(fma(R(2), T3, fma(R(-3), D4, R(6) * e3)), D4 - T3, T3);
+        W q4 = ind(fma(R(11), e6, fma(R(-31), e5, R(26) * e4)), fma(R(-2), T4, D5), T4);
+        q4 = fmax(fmax(fmax(q0, q1), fmax(q2, q3)), q4);
+        const W q01 = q0 * q1, q34 = q3 * q4, q234 = q2 * q34, q012 = q01 * q2;
+        w0 = W(0.0401954833730) * q1 * q234;
+        w1 = W(0.2493800006710) * q0 * q234;
+        w2 = W(0.4802686256260) * q01 * q34;
+        w3 = W(0.2009775476730) * q012 * q4;
+        w4 = W(0.0291783426580) * q012 * q3;
     }
-    W am = S0 + S1 + S2 + S3 + S4;
-    W r = S0 * W(R(-3) * s[0] + R(13) * s[1] - R(23) * s[2] + R(25) * s[3]);
-    r += S1 * W(s[1] - R(5) * s[2] + R(13) * s[3] + R(3) * s[4]);
-    r += S2 * W(-s[2] + R(7) * s[3] + R(7) * s[4] - s[5]);
-    r += S3 * W(R(3) * s[3] + R(13) * s[4] - R(5) * s[5] + s[6]);
-    r += S4 * W(R(25) * s[4] - R(23) * s[5] + R(13) * s[6] - R(3) * s[7]);
-    return R(r / (W(12) * am));
+    const W d0 = W(fma(R(13), e2, fma(R(-10), e1, R(3) * e0)));
+    const W d1 = W(fma(R(3), e3, fma(R(4), e2, -e1)));
+    const W d2 = W(fma(R(6), e3, e2 - e4));
+    const W d3 = W(fma(R(9), e3, fma(R(-4), e4, e5)));
+    const W d4 = W(fma(R(12), e3, fma(R(-13), e4, fma(R(10), e5, R(-3) * e6))));
+    const W num = fma(w4, d4, fma(w3, d3, fma(w2, d2, fma(w1, d1, w0 * d0))));
+    return R(W(s[3]) + weight_div(num, W(12) * (((w0 + w1) + (w2 + w3)) + w4)));
 }
 template <typename R, typename W = R> __device__ __forceinline__ R symbo_up(const R* s, int lmt, R tvlim, R tvmax) {
     bool lin = false;
