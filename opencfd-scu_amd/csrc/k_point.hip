@@ -732,6 +732,16 @@ __global__ void __launch_bounds__(256) k_diag_final(const double* __restrict__ p
     }
 }
 
+template <typename S>
+__global__ void __launch_bounds__(256) k_pack(PackArgsT<S> A) {
+    const Geo& g = A.g;
+    const int i = blockIdx.x * 64 + threadIdx.x, j = blockIdx.y * 4 + threadIdx.y, k = blockIdx.z;
+    if (i >= g.nx || j >= g.ny) return;
+    const long long q = gidx(g, i, j, k), n = (long long)g.nx * g.ny * g.nz;
+    S* d = A.dst + i + (long long)g.nx * (j + (long long)g.ny * k);
+    for (int f = 0; f < A.nf; f++) __builtin_nontemporal_store(A.src[f][q], &d[f * n]);
+}
+
 template <typename To, typename From>
 __global__ void k_convert(To* dst, const From* src, long long n) {
     const long long t = (long long)blockIdx.x * blockDim.x + threadIdx.x;
@@ -840,6 +850,11 @@ void launch_set(const Geo& g, double* base, long long n, double value, hipStream
     hipLaunchKernelGGL(k_set, dim3((unsigned)((n + 255) / 256)), dim3(256), 0, st, base, n, value);
 }
 
+template <typename S>
+void launch_pack(const PackArgsT<S>& a, hipStream_t st) {
+    hipLaunchKernelGGL(k_pack<S>, pgrid(a.g), dim3(64, 4), 0, st, a);
+}
+
 template <typename To, typename From>
 void launch_convert(To* dst, const From* src, long long n, hipStream_t st) {
     hipLaunchKernelGGL((k_convert<To, From>), dim3((unsigned)((n + 255) / 256)), dim3(256), 0, st, dst, src, n);
@@ -878,6 +893,7 @@ void launch_diag_final(const double* partE, const double* partT, long long nb, c
                                    hipStream_t);                                                              \
     template void launch_filter<S>(const FilterArgsT<S>&, hipStream_t);                                      \
     template void launch_p2c_all<S>(const BCArgsT<S>&, hipStream_t);                                         \
+    template void launch_pack<S>(const PackArgsT<S>&, hipStream_t);                                          \
     template void launch_c2p_all<S>(const StageArgsT<S>&, hipStream_t);                                      \
     template void launch_amu_all<S>(const BCArgsT<S>&, hipStream_t);                                        \
     template void launch_diag<S>(const Geo&, const double*, const S*, double*, double*, int*, hipStream_t);  \
@@ -887,4 +903,3 @@ OCFD_INSTANTIATE(double)
 OCFD_INSTANTIATE(float)
 #undef OCFD_INSTANTIATE
 template void launch_convert<float, double>(float*, const double*, long long, hipStream_t);
-template void launch_convert<double, float>(double*, const float*, long long, hipStream_t);

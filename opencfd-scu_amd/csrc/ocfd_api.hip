@@ -60,6 +60,7 @@ struct ocfd_ctx {
     // pinned staging buffer of the device-to-host downloads (grown on demand)
     void* pin = nullptr;
     size_t pin_bytes = 0;
+    hipEvent_t pin_ev[3] = {};  // one per slot of a download in pieces
     Geo g;
     Consts c;
     long long fs = 0;  // elements per field
@@ -256,7 +257,21 @@ int upload_interior(ocfd_ctx* x, double* dst, const double* src, double ghost_va
     return 0;
 }
 
-// Interior of a padded field (base pointer = allocation + 12 elements).
+// The pinned staging buffer, grown to at least `bytes`.
+int ensure_pin(ocfd_ctx* x, size_t bytes) {
+    if (bytes <= x->pin_bytes) return 0;
+    HIPCK(hipStreamSynchronize(x->st));
+    if (x->pin) (void)hipHostFree(x->pin);
+    x->pin = nullptr;
+    x->pin_bytes = 0;
+    if (hipHostMalloc(&x->pin, bytes, hipHostMallocDefault) != hipSuccess) {
+        x->pin = nullptr;
+        return fail(OCFD_ERR_HIP, "hipHostMalloc failed (" + std::to_string(bytes) + " bytes)");
+    }
+    x->pin_bytes = bytes;
+    return 0;
+}
+
 // Device-to-host copy of `bytes` at src, ordered after the work on the
 // context's stream, through a pinned staging buffer; returns the staged
 // host copy (valid until the next call).  A plain hipMemcpy into pageable
@@ -265,19 +280,7 @@ int upload_interior(ocfd_ctx* x, double* dst, const double* src, double ghost_va
 // overlap of its two streams (mixed path on the 512x128x64 ramp: 2.13 ->
 // 2.37 ms/step).
 const void* d2h(ocfd_ctx* x, const void* src, size_t bytes, int& rc) {
-    rc = 0;
-    if (bytes > x->pin_bytes) {
-        if (hipStreamSynchronize(x->st) != hipSuccess) { rc = fail(OCFD_ERR_HIP, "hipStreamSynchronize failed"); return nullptr; }
-        if (x->pin) (void)hipHostFree(x->pin);
-        x->pin = nullptr;
-        x->pin_bytes = 0;
-        if (hipHostMalloc(&x->pin, bytes, hipHostMallocDefault) != hipSuccess) {
-            x->pin = nullptr;
-            rc = fail(OCFD_ERR_HIP, "hipHostMalloc failed (" + std::to_string(bytes) + " bytes)");
-            return nullptr;
-        }
-        x->pin_bytes = bytes;
-    }
+    if ((rc = ensure_pin(x, bytes))) return nullptr;
     if (hipMemcpyAsync(x->pin, src, bytes, hipMemcpyDeviceToHost, x->st) != hipSuccess ||
         hipStreamSynchronize(x->st) != hipSuccess) {
         rc = fail(OCFD_ERR_HIP, "device-to-host copy failed");
@@ -292,16 +295,73 @@ const void* d2h(ocfd_ctx* x, const void* src, size_t bytes, int& rc) {
         if (rc_) return rc_;                          \
     } while (0)
 
-int download_interior(ocfd_ctx* x, const double* src, double* dst) {
-    const Geo& g = x->g;
-    const void* hv;
-    D2H(hv, x, src - 12, sizeof(double) * x->fs);
-    const double* h = (const double*)hv;
-    for (int k = 0; k < g.nz; k++)
-        for (int j = 0; j < g.ny; j++)
-            std::memcpy(dst + ((size_t)k * g.ny + j) * g.nx, &h[(size_t)gidx(g, 0, j, k) + 12],
-                        sizeof(double) * g.nx);
+// The interiors of nf fields (null destinations are left out) to host arrays,
+// widened from S.  The GPU packs them without their ghost layers, so that the
+// host copies long runs instead of rows; up to DIRECT bytes it packs straight
+// into the pinned buffer (no copy of its own: a 20x16x12 state 5 copies and
+// waits -> 1), above that the packed values come over in pieces of PIECE bytes,
+// three in flight, while the host copies the one before.
+template <typename S>
+int download_fields(ocfd_ctx* x, const S* const* src, double* const* dst, int nf) {
+    constexpr size_t DIRECT = 1u << 20, PIECE = 16u << 20;
+    constexpr int SLOTS = 3;
+    const size_t n = (size_t)x->g.nx * x->g.ny * x->g.nz;
+    PackArgsT<S> a;
+    double* out[PACK_FIELDS];
+    a.g = x->g;
+    a.nf = 0;
+    for (int q = 0; q < nf; q++)
+        if (dst[q]) {
+            out[a.nf] = dst[q];
+            a.src[a.nf++] = src[q];
+        }
+    if (!a.nf) return 0;
+    const size_t total = n * a.nf, bytes = total * sizeof(S);
+    auto unpack = [&](const S* p, size_t first, size_t count) {
+        while (count) {
+            const size_t o = first % n, m = std::min(count, n - o);
+            double* d = out[first / n] + o;
+            if constexpr (std::is_same<S, double>::value) std::memcpy(d, p, m * sizeof(double));
+            else
+                for (size_t q = 0; q < m; q++) d[q] = double(p[q]);
+            p += m;
+            first += m;
+            count -= m;
+        }
+    };
+    if (bytes <= DIRECT) {
+        TRY(ensure_pin(x, bytes));
+        a.dst = (S*)x->pin;
+        TRY(timed(x, "pack", [&] { launch_pack(a, x->st); }));
+        HIPCK(hipStreamSynchronize(x->st));
+        unpack((const S*)x->pin, 0, total);
+        return 0;
+    }
+    // packed into the scratch fields after the first (which ocfd_get_q fills)
+    a.dst = (S*)(x->grad + x->fs);
+    const size_t piece = PIECE / sizeof(S), np = (total + piece - 1) / piece;
+    TRY(ensure_pin(x, std::min(bytes, SLOTS * PIECE)));
+    for (auto& e : x->pin_ev)
+        if (!e) HIPCK(hipEventCreateWithFlags(&e, hipEventDisableTiming));
+    TRY(timed(x, "pack", [&] { launch_pack(a, x->st); }));
+    auto slot = [&](size_t c) { return (S*)x->pin + (c % SLOTS) * piece; };
+    auto count = [&](size_t c) { return std::min(piece, total - c * piece); };
+    auto fetch = [&](size_t c) -> int {
+        HIPCK(hipMemcpyAsync(slot(c), a.dst + c * piece, count(c) * sizeof(S), hipMemcpyDeviceToHost, x->st));
+        HIPCK(hipEventRecord(x->pin_ev[c % SLOTS], x->st));
+        return 0;
+    };
+    for (size_t c = 0; c < np && c < SLOTS; c++) TRY(fetch(c));
+    for (size_t c = 0; c < np; c++) {
+        HIPCK(hipEventSynchronize(x->pin_ev[c % SLOTS]));
+        unpack(slot(c), c * piece, count(c));
+        if (c + SLOTS < np) TRY(fetch(c + SLOTS));
+    }
     return 0;
+}
+template <typename S>
+int download_any(ocfd_ctx* x, const S* src, double* dst) {
+    return download_fields(x, &src, &dst, 1);
 }
 
 // IPERIODIC as a mask (bit 0: x, 1: y, 2: z).
@@ -337,16 +397,6 @@ int upload_any(ocfd_ctx* x, S* dst, const double* src, double ghost_value) {
         return 0;
     }
 }
-template <typename S>
-int download_any(ocfd_ctx* x, const S* src, double* dst) {
-    if constexpr (std::is_same<S, double>::value) {
-        return download_interior(x, src, dst);
-    } else {
-        TRY(timed(x, "convert", [&] { launch_convert(x->grad, src, x->fs, x->st); }));
-        return download_interior(x, x->grad, dst);
-    }
-}
-
 template <typename S>
 BCArgsT<S> bc_args(ocfd_ctx* x) {
     BCArgsT<S> a;
@@ -1099,6 +1149,8 @@ int ocfd_destroy(ocfd_ctx* x) {
     if (x->st2) (void)hipStreamSynchronize(x->st2);
     for (void* p : x->allocs) (void)hipFree(p);
     if (x->pin) (void)hipHostFree(x->pin);
+    for (auto e : x->pin_ev)
+        if (e) (void)hipEventDestroy(e);
     if (x->ev_fork) (void)hipEventDestroy(x->ev_fork);
     if (x->ev_join) (void)hipEventDestroy(x->ev_join);
     if (x->st2) (void)hipStreamDestroy(x->st2);
@@ -1321,12 +1373,10 @@ int ocfd_get_flow(ocfd_ctx* x, double* d, double* u, double* v, double* w, doubl
         // the stored FP32 primitives: like the reference's they lag the
         // filter, which changes only f at the end of a step
         const float* src[5] = {x->sd, x->su, x->sv, x->sw, x->sT};
-        for (int q = 0; q < 5; q++)
-            if (dst[q]) TRY(download_any(x, src[q], dst[q]));
+        TRY(download_fields(x, src, dst, 5));
     } else {
         const double* src[5] = {x->d, x->u, x->v, x->w, x->T};
-        for (int q = 0; q < 5; q++)
-            if (dst[q]) TRY(download_interior(x, src[q], dst[q]));
+        TRY(download_fields(x, src, dst, 5));
     }
     if (istep) *istep = x->istep;
     if (tt) *tt = x->tt;
@@ -1336,8 +1386,13 @@ int ocfd_get_flow(ocfd_ctx* x, double* d, double* u, double* v, double* w, doubl
 int ocfd_get_state(ocfd_ctx* x, double* f5) {
     if (!x || !f5) return fail(OCFD_ERR_ARG, "null argument");
     const size_t n = (size_t)x->g.nx * x->g.ny * x->g.nz;
-    for (int m = 0; m < 5; m++) TRY(download_interior(x, x->f + m * x->fs, f5 + m * n));
-    return 0;
+    const double* src[5];
+    double* dst[5];
+    for (int m = 0; m < 5; m++) {
+        src[m] = x->f + m * x->fs;
+        dst[m] = f5 + m * n;
+    }
+    return download_fields(x, src, dst, 5);
 }
 
 int ocfd_get_du(ocfd_ctx* x, double* du5) {
@@ -1345,14 +1400,14 @@ int ocfd_get_du(ocfd_ctx* x, double* du5) {
     TRY(finish_rhs(x));
     const size_t n = (size_t)x->g.nx * x->g.ny * x->g.nz;
     for (int m = 0; m < 5; m++)
-        TRY(x->mixed ? download_any(x, x->sdu + m * x->fs, du5 + m * n)
-                     : download_any(x, x->du + m * x->fs, du5 + m * n));
+        TRY(x->mixed ? download_any(x, (const float*)x->sdu + m * x->fs, du5 + m * n)
+                     : download_any(x, (const double*)x->du + m * x->fs, du5 + m * n));
     // the viscous part of components 1..4 when it is kept apart, added as
     // the RK stage adds it, then the Jacobian factor the stage applies
     std::vector<double> tmp(n);
     if (!x->mixed) {
         for (int m = 1; m < 5; m++) {
-            TRY(download_any(x, x->dv + (m - 1) * x->fs, tmp.data()));
+            TRY(download_any(x, (const double*)x->dv + (m - 1) * x->fs, tmp.data()));
             for (size_t p = 0; p < n; p++) du5[m * n + p] += tmp[p];
         }
     }
@@ -1364,7 +1419,7 @@ int ocfd_get_du(ocfd_ctx* x, double* du5) {
 
 int ocfd_get_pressure(ocfd_ctx* x, double* p) {
     if (!x || !p) return fail(OCFD_ERR_ARG, "null argument");
-    return x->mixed ? download_any(x, x->sP, p) : download_any(x, x->P, p);
+    return x->mixed ? download_any(x, (const float*)x->sP, p) : download_any(x, (const double*)x->P, p);
 }
 
 int ocfd_get_amu(ocfd_ctx* x, double* a) {
@@ -1374,11 +1429,11 @@ int ocfd_get_amu(ocfd_ctx* x, double* a) {
     if (x->mixed) {
         const BCArgsT<float> b = bc_args<float>(x);
         TRY(timed(x, "amu", [&] { launch_amu_all(b, x->st); }));
-        return download_any(x, x->samu, a);
+        return download_any(x, (const float*)x->samu, a);
     }
     const BCArgsT<double> b = bc_args<double>(x);
     TRY(timed(x, "amu", [&] { launch_amu_all(b, x->st); }));
-    return download_any(x, x->amu, a);
+    return download_any(x, (const double*)x->amu, a);
 }
 
 int ocfd_get_metrics(ocfd_ctx* x, double* a13) {
@@ -1386,8 +1441,13 @@ int ocfd_get_metrics(ocfd_ctx* x, double* a13) {
     const size_t n = (size_t)x->g.nx * x->g.ny * x->g.nz;
     if (x->mesh.size() == 3 * n) std::memcpy(a13, x->mesh.data(), sizeof(double) * 3 * n);
     else std::memset(a13, 0, sizeof(double) * 3 * n);
-    for (int m = 0; m < M_COUNT; m++) TRY(download_interior(x, x->M[m], a13 + (3 + m) * n));
-    return 0;
+    const double* src[M_COUNT];
+    double* dst[M_COUNT];
+    for (int m = 0; m < M_COUNT; m++) {
+        src[m] = x->M[m];
+        dst[m] = a13 + (3 + m) * n;
+    }
+    return download_fields(x, src, dst, M_COUNT);
 }
 
 int ocfd_diagnostics(ocfd_ctx* x, double* mean_energy, double* mean_T, long long* n_nan_T, long long* n_neg_T) {
@@ -1645,7 +1705,7 @@ int ana_time_average(ocfd_ctx* x) {
     x->avg_tt += x->cfg.dt;
     if (x->cfg.kstep_save > 0 && x->istep % x->cfg.kstep_save == 0) {
         std::vector<double> h(5 * n);
-        for (int m = 0; m < 5; m++) TRY(download_interior(x, x->avg + m * x->fs, h.data() + m * n));
+        for (int m = 0; m < 5; m++) TRY(download_any(x, (const double*)(x->avg + m * x->fs), h.data() + m * n));
         char name[64];
         std::snprintf(name, sizeof name, "OCFD%08d.average", x->avg_n);
         std::printf("write data file: %s\n", name);
@@ -1802,7 +1862,7 @@ int ocfd_get_q(ocfd_ctx* x, double* q) {
         va.ev = x->ev; va.du = x->du; va.dv = x->dv; va.fs = x->fs;
         TRY(timed(x, "qcrit", [&] { launch_qcrit(va, out, x->st); }));
     }
-    return download_interior(x, out, q);
+    return download_any(x, (const double*)out, q);
 }
 
 int ocfd_get_time_average(ocfd_ctx* x, double* d, double* u, double* v, double* w, double* T, int* nsamples,
@@ -1811,7 +1871,7 @@ int ocfd_get_time_average(ocfd_ctx* x, double* d, double* u, double* v, double* 
     if (!x->avg) return fail(OCFD_ERR_STATE, "no time average yet (analysis style 101)");
     double* outs[5] = {d, u, v, w, T};
     for (int m = 0; m < 5; m++)
-        if (outs[m]) TRY(download_interior(x, x->avg + m * x->fs, outs[m]));
+        if (outs[m]) TRY(download_any(x, (const double*)(x->avg + m * x->fs), outs[m]));
     if (nsamples) *nsamples = x->avg_n;
     if (tt_avg) *tt_avg = x->avg_tt;
     return 0;

@@ -260,6 +260,18 @@ size_t mlp_part_floats(int nb);
 // FP32 forward probabilities of rows 0..nb of X.
 void launch_mlp_predict(const float* params, const float* X, int nb, float* prob, hipStream_t st);
 
+// The interiors of nf fields, packed without ghost layers one after another
+// (x fastest) into dst.
+constexpr int PACK_FIELDS = 10;
+template <typename S>
+struct PackArgsT {
+    Geo g;
+    const S* src[PACK_FIELDS];
+    int nf;
+    S* dst;
+};
+template <typename S> void launch_pack(const PackArgsT<S>& a, hipStream_t st);
+
 // dst[i] = (To)src[i] for n elements (precision conversion of whole fields).
 template <typename To, typename From>
 void launch_convert(To* dst, const From* src, long long n, hipStream_t st);

@@ -1,0 +1,39 @@
+"""Downloads in one piece and in several: the values a context returns equal
+the ones loaded into it, at sizes below and above the direct and the piecewise
+limits (1 MiB and 16 MiB of packed values) and with fields left out."""
+import ctypes as C
+
+import numpy as np
+import pytest
+
+from pyocfd import capi, cases
+
+pytestmark = pytest.mark.gpu
+
+
+# 5 FP64 fields: 0.02 MiB; just above 1 MiB; 16.0 MiB +- a row; 2 pieces and a
+# remainder; more pieces than slots
+@pytest.mark.parametrize("size", [(8, 9, 8), (35, 29, 27), (64, 64, 102), (64, 64, 103), (131, 99, 80), (160, 130, 110)])
+@pytest.mark.parametrize("prec", [capi.PREC_FP64, capi.PREC_MIXED])
+def test_flow_comes_back_as_loaded(size, prec):
+    nx, ny, nz = size
+    rng = np.random.default_rng(1)
+    # exactly representable in FP32, so the mixed path returns them unchanged
+    prims = [1.0 + rng.integers(0, 1 << 16, (nz, ny, nx)) / float(1 << 20) for _ in range(5)]
+    cfg = cases.wavy_box(8, 8, 8).cfg
+    cfg.nx, cfg.ny, cfg.nz, cfg.precision = nx, ny, nz, prec
+    s = capi.Solver(cfg)
+    s.load_flow(*prims, istep=3, tt=0.5)
+    got, istep, tt = s.get_flow()
+    assert (istep, tt) == (3, 0.5)
+    for a, b in zip(got, prims):
+        assert np.array_equal(a, b)
+    # only u and T
+    dp = C.POINTER(C.c_double)
+    fn = C.cast(s.lib.ocfd_get_flow, C.c_void_p).value
+    get = C.CFUNCTYPE(C.c_int, C.c_void_p, dp, dp, dp, dp, dp, C.POINTER(C.c_int), dp)(fn)
+    u, T = np.zeros((nz, ny, nx)), np.zeros((nz, ny, nx))
+    as_p = lambda a: a.ctypes.data_as(dp)  # noqa: E731
+    assert get(s.h, None, as_p(u), None, None, as_p(T), None, None) == 0
+    assert np.array_equal(u, prims[1]) and np.array_equal(T, prims[4])
+    s.close()
