@@ -33,57 +33,13 @@
 
 namespace {
 
-#ifndef OCFD_VISC_KZ_D
-#define OCFD_VISC_KZ_D 32  // z planes per block, FP64 path (16 / 24 / 32 / 64: 4.57 / 4.55 / 4.46 /
-                           // 4.74 ms per launch on the 1024x384x256 swept ramp)
-#endif
-#ifndef OCFD_VISC_KZ_F
-#define OCFD_VISC_KZ_F 16  // z planes per block, FP32 path: 8 is the fastest alone, 16 the faster
-                           // step beside the sweeps (2.016 -> 2.008 ms on the 512x128x64 ramp)
-#endif
-#ifndef OCFD_VISC_TX
-#define OCFD_VISC_TX 32  // x columns per block
-#endif
-#ifndef OCFD_VISC_TY_D
-#define OCFD_VISC_TY_D 8  // y columns per block of the gradient kernel, FP64 path (16 measured 4.45 ->
-                          // 4.41 ms per launch on the 1024x384x256 swept ramp, the step 64.47 -> 64.18
-                          // ms, and passes the parity tests; 2 waves per SIMD either way)
-#endif
-#ifndef OCFD_VISC_TY_F
-#define OCFD_VISC_TY_F 8  // FP32 path: a 512-thread block would cost it its third wave per SIMD
-#endif
-#ifndef OCFD_VISC_PREFETCH
-#define OCFD_VISC_PREFETCH 1  // fetch plane k+1 while plane k is computed
-#endif
-constexpr int TX = OCFD_VISC_TX;
-// y columns per block of the gradient/flux kernel
-template <typename S> struct TY_ { static constexpr int v = OCFD_VISC_TY_D; };
-template <> struct TY_<float> { static constexpr int v = OCFD_VISC_TY_F; };
-#ifndef OCFD_VDIV_KZ_D
-#define OCFD_VDIV_KZ_D 32  // z planes per block of the divergence, FP64 path: 32 against 16 on the
-                           // 1024x384x256 swept ramp, the divergence's share of the step 13.65 ->
-                           // 13.44 % and the step 64.34 -> 64.17 ms (bench runs alternated); no
-                           // change on the 512x128x64 and 1024x256x128 ramps
-#endif
-#ifndef OCFD_VDIV_KZ_F
-#define OCFD_VDIV_KZ_F 16  // z planes per block of the divergence, FP32 path
-#endif
-#ifndef OCFD_VDIV_TY
-#define OCFD_VDIV_TY 8  // y columns per block of the divergence
-#endif
-constexpr int TYD = OCFD_VDIV_TY;
-// z planes per block: KZ_<S, false> for the gradient/flux kernel, KZ_<S,
-// true> for the divergence
-template <typename S, bool DIV = false> struct KZ_ { static constexpr int v = DIV ? OCFD_VDIV_KZ_D : OCFD_VISC_KZ_D; };
-template <bool DIV> struct KZ_<float, DIV> { static constexpr int v = DIV ? OCFD_VDIV_KZ_F : OCFD_VISC_KZ_F; };
-constexpr bool VISC_PREFETCH = OCFD_VISC_PREFETCH;
-#ifndef OCFD_VISC_RING
-#define OCFD_VISC_RING 1  // FP64 gradient kernel: halo strips fetched five planes ahead into an LDS ring
-                          // (the FP32 form would lose its third wave per SIMD to the registers)
-#endif
-#ifndef OCFD_VISC_SKIP_CORNERS
-#define OCFD_VISC_SKIP_CORNERS 1  // the gradient kernel does not load the tile's halo corners
-#endif
+constexpr int TX = 32, TY = 8;  // columns per block
+// z planes per block where a launch fills the chip anyway (chunk_planes).
+// FP64, 1024x384x256: the gradient kernel 16 / 24 / 32 / 64 planes 4.57 / 4.55 /
+// 4.46 / 4.74 ms; FP32: 8 is the fastest alone, 16 the faster step beside the
+// sweeps.
+template <typename S> struct KZ_ { static constexpr int v = 32; };
+template <> struct KZ_<float> { static constexpr int v = 16; };
 
 // Central derivative at interior index i (0..n-1) from s[0..8] = values at
 // i-4..i+4 (OCFD_CD6/CD8_kernel + D0 closures + put_d0_kernel).  rh = 1/h; the
@@ -120,12 +76,11 @@ struct Tile25 {
     int i0, j0, i, j, kbeg, kend;
     bool own;
 };
-template <int TYB>
 __device__ __forceinline__ Tile25 tile_of(const Geo& g, int kz) {
     Tile25 t;
     const Blk B = xcd_block();
     t.i0 = B.x * TX;
-    t.j0 = B.y * TYB;
+    t.j0 = B.y * TY;
     t.i = t.i0 + threadIdx.x;
     t.j = t.j0 + threadIdx.y;
     t.kbeg = B.z * kz;
@@ -137,32 +92,17 @@ __device__ __forceinline__ Tile25 tile_of(const Geo& g, int kz) {
 // Gradients of u, v, w, T at (t.i, t.j, k) from the plane tile pl (the
 // current plane with its x and y strips, row pitch PW) and the thread's z
 // queue q, and at the same point the viscous fluxes Ev1..4 of the three
-// directions (vis_flux_s_ker / vis_flux_e_ker / vis_flus_ev_ker).  CL =
-// false: no derivative of the block's plane reaches a closure (the caller
-// decides per block and plane), and the body is straight-line code.
+// directions (vis_flux_s_ker / vis_flux_e_ker / vis_flus_ev_ker) from the
+// point's metrics met.  oo: the point's byte offset in a plane (BUF_NONE: no
+// point, nothing is written).  CL = false: no derivative of the block's plane
+// reaches a closure (the caller decides per block and plane), and the body is
+// straight-line code.
 template <int SV, typename S, int PW, bool CL>
-__device__ __forceinline__ void gf_point(const ViscArgsT<S>& A, const Tile25& t, int k,
-                                         const S (*pl)[PW * (TY_<S>::v + 8)],
+__device__ __forceinline__ void gf_point(const ViscArgsT<S>& A, const Tile25& t, int k, long long fs, unsigned oo,
+                                         const S* met,
+                                         const S (*pl)[PW * (TY + 8)],
                                          const S (*q)[9], int tx, int ty, S rhx, S rhy, S rhz) {
     const Geo& g = A.g;
-    // The point's metrics are loaded first, so that the loads are in flight
-    // while the derivatives are formed.  They are read once here and the
-    // fluxes are written once: all go through the caches as streaming
-    // (non-temporal) accesses, which leaves L2 to the plane strips that
-    // neighbouring tiles share (measured 203 -> 196 us, and the divergence
-    // that reads Ev next 42 -> 40 us).
-    const long long qi = gidx(g, t.i, t.j, k), fs = A.fs;
-    auto ld = [&](int m) { return S(__builtin_nontemporal_load(&A.M[m][qi])); };
-    const S Akx = ld(M_KX), Aky = ld(M_KY), Akz = ld(M_KZ);
-    const S Aix = ld(M_IX), Aiy = ld(M_IY), Aiz = ld(M_IZ);
-    const S Asx = ld(M_SX), Asy = ld(M_SY), Asz = ld(M_SZ);
-    const S Aj1 = ld(M_JAC);
-    // Sutherland's law at the point (get_Amu_kernal, src/commen_kernel.cu:
-    // 122-131) from its T (the centre of the z queue), in FP64 as the RK stage
-    // and the boundary kernels form it: the same value as a viscosity field
-    // written after each stage, without its 8 B/pt store and reload
-    const double Tp = double(q[3][4]);
-    const S Amu = S(A.c.amu_c0 * sqrt(Tp * Tp * Tp) / (A.c.tsb + Tp));
     S gr[4][3];
 #pragma unroll
     for (int f = 0; f < 4; f++) {
@@ -175,6 +115,16 @@ __device__ __forceinline__ void gf_point(const ViscArgsT<S>& A, const Tile25& t,
         gr[f][1] = cd9<SV, S, CL>(s, t.j, g.ny, A.bnd[2], A.bnd[3], rhy);
         gr[f][2] = cd9<SV, S, CL>(q[f], k, g.nz, A.bnd[4], A.bnd[5], rhz);
     }
+    const S Akx = met[M_KX], Aky = met[M_KY], Akz = met[M_KZ];
+    const S Aix = met[M_IX], Aiy = met[M_IY], Aiz = met[M_IZ];
+    const S Asx = met[M_SX], Asy = met[M_SY], Asz = met[M_SZ];
+    const S Aj1 = met[M_JAC];
+    // Sutherland's law at the point (get_Amu_kernal, src/commen_kernel.cu:
+    // 122-131) from its T (the centre of the z queue), in FP64 as the RK stage
+    // and the boundary kernels form it: the same value as a viscosity field
+    // written after each stage, without its 8 B/pt store and reload
+    const double Tp = double(q[3][4]);
+    const S Amu = S(A.c.amu_c0 * sqrt(Tp * Tp * Tp) / (A.c.tsb + Tp));
     // vis_flux_s_ker / vis_flux_e_ker / vis_flus_ev_ker
     const S uk = gr[0][0], ui = gr[0][1], us = gr[0][2];
     const S vk = gr[1][0], vi = gr[1][1], vs = gr[1][2];
@@ -209,194 +159,120 @@ __device__ __forceinline__ void gf_point(const ViscArgsT<S>& A, const Tile25& t,
 #pragma unroll
     for (int d = 0; d < 3; d++) {
         const S akx = ax[d] * Aj1, aky = ay[d] * Aj1, akz = az[d] * Aj1;
-        S* E = A.ev + (long long)(4 * d) * fs + qi;
-        __builtin_nontemporal_store(S(akx * s11 + aky * s12 + akz * s13), &E[0]);
-        __builtin_nontemporal_store(S(akx * s12 + aky * s22 + akz * s23), &E[fs]);
-        __builtin_nontemporal_store(S(akx * s13 + aky * s23 + akz * s33), &E[2 * fs]);
-        __builtin_nontemporal_store(S(akx * E1 + aky * E2 + akz * E3), &E[3 * fs]);
+        // written once here and read by another kernel: streamed
+        auto put = [&](int m, S v) {
+            Buf<S>(A.ev + (long long)(k + 4) * g.sz + (4 * d + m) * fs, g.sz).template st<BUF_STREAM>(oo, v);
+        };
+        put(0, akx * s11 + aky * s12 + akz * s13);
+        put(1, akx * s12 + aky * s22 + akz * s23);
+        put(2, akx * s13 + aky * s23 + akz * s33);
+        put(3, akx * E1 + aky * E2 + akz * E3);
     }
-    
 }
 
 // Whether a central-derivative closure is in reach of the block's plane k:
 // the same for every thread of the block.
-template <int TYB, typename S>
+template <typename S>
 __device__ __forceinline__ bool near_closure(const ViscArgsT<S>& A, const Tile25& t, int k) {
     const Geo& g = A.g;
     return (A.bnd[0] && t.i0 <= 3) || (A.bnd[1] && t.i0 + TX > g.nx - 4) || (A.bnd[2] && t.j0 <= 3) ||
-           (A.bnd[3] && t.j0 + TYB > g.ny - 4) || (A.bnd[4] && k <= 3) || (A.bnd[5] && k >= g.nz - 4);
+           (A.bnd[3] && t.j0 + TY > g.ny - 4) || (A.bnd[4] && k <= 3) || (A.bnd[5] && k >= g.nz - 4);
 }
 
-// The plane loads of both kernels go through per-thread slots: the slot's
-// LDS position and its global offset in plane 0 (-1: outside the ghost
-// layers, stored as 0).  Loads for plane k+1 are issued before plane k is
-// computed.
+// Gradients and viscous fluxes of a plane, marching in z.  The next plane's
+// strips and queue values and the point's metrics are in flight while a plane
+// is computed.  Bound by HBM (512x128x64 5.7 TB/s of traffic) and by latency
+// behind it: what moved it is when loads are issued.  Raw buffer accesses took
+// the FP64 kernel from 233 VGPRs to 206 (still 2 waves per SIMD) and the FP32
+// kernel from 3 waves to 4, and made the ring of strips fetched five planes
+// ahead pointless: 1024x256x128 1.58 -> 1.54 ms, 512x128x64 193 -> 182 us, mixed
+// 120 -> 117 us.  Dropped: metrics loaded after the derivatives to fit 3 waves
+// (182 -> 241 us, mixed 117 -> 167), a plane ahead (194, 141), 32x16 tiles (210,
+// 126).
 template <int SV, typename S>
-__global__ void __launch_bounds__(TX * TY_<S>::v) k_visc_gf(ViscArgsT<S> A, int kz) {
-    constexpr int TY = TY_<S>::v, NT = TX * TY;
-    constexpr int PW = TX + 8, PN = PW * (TY + 8), NSL = (PN + NT - 1) / NT;
+__global__ void __launch_bounds__(TX * TY, sizeof(S) == 8 ? 2 : 4) k_visc_gf(ViscArgsT<S> A, int kz) {
+    constexpr int NT = TX * TY;
+    constexpr int PW = TX + 8, PN = PW * (TY + 8);
+    static_assert(NT >= 8 * TX, "y strips: one position per thread");
     const Geo& g = A.g;
-    const Tile25 t = tile_of<TY>(g, kz);
+    const Tile25 t = tile_of(g, kz);
     const int tx = threadIdx.x, ty = threadIdx.y, tid = ty * TX + tx;
-    const int i0 = t.i0, j0 = t.j0;
     const S rhx = S(1.0 / g.hx), rhy = S(1.0 / g.hy), rhz = S(1.0 / g.hz);
     __shared__ S pl[4][PN];
-    const S* src[4] = {A.u, A.v, A.w, A.T};
-    const int ic = min(t.i, g.nx - 1), jc = min(t.j, g.ny - 1);  // clamped column for queue loads
-    const long long col = gidx(g, ic, jc, 0);
-    // halo slots: positions outside the TX x TY interior of the tile that a
-    // derivative reads (the x strips beside the interior rows and the y
-    // strips beside the interior columns; the corners are never read)
-    int sl[NSL];
-    long long so[NSL];
-#pragma unroll
-    for (int r = 0; r < NSL; r++) {
-        const int p = tid + NT * r;
-        const int hx = p % PW, hy = p / PW;
-        const bool xin = hx >= 4 && hx < TX + 4, yin = hy >= 4 && hy < TY + 4;
-        sl[r] = (p < PN && (xin != yin || !OCFD_VISC_SKIP_CORNERS) && !(xin && yin)) ? p : -1;
-        const int gi = i0 - 4 + hx, gj = j0 - 4 + hy;
-        so[r] = (gi <= g.nx + 3 && gj <= g.ny + 3) ? gidx(g, gi, gj, 0) : -1;
-    }
+    // byte offset of (i, j) in a plane, up to the ghost layers
+    auto off = [&](int i, int j) {
+        return i < g.nx + 4 && j < g.ny + 4 ? (unsigned)((i + 4) + g.ldx * (j + 4)) * (unsigned)sizeof(S) : BUF_NONE;
+    };
+    const unsigned oo = t.own ? off(t.i, t.j) : BUF_NONE;
+    const unsigned od = t.own ? oo / (unsigned)sizeof(S) * 8u : BUF_NONE;  // in the FP64 metric fields
     // the thread's own tile position: from the queue when owned, else from
-    // memory (x/y ghosts inside the tile) or 0
-    const long long co = t.own ? -1 : (t.i <= g.nx + 3 && t.j <= g.ny + 3) ? gidx(g, t.i, t.j, 0) : -1;
-    S hv[NSL][4], cv[4];
-    auto load_plane = [&](int k) {
-        const long long pk = (long long)k * g.sz;
+    // memory (x/y ghosts inside the tile)
+    const unsigned oc = t.own ? BUF_NONE : off(t.i, t.j);
+    // halo strips a derivative reads: 4 + 4 columns beside the tile's rows
+    // (the first 8 * TY threads) and 4 + 4 rows beside its columns (the first
+    // 8 * TX threads); the corners are never read
+    const int xc = tid & 7, xr = tid >> 3;
+    const bool xs = tid < 8 * TY, ys = tid < 8 * TX;
+    const int yr = tid / TX;
+    const unsigned ox = xs ? off(xc < 4 ? t.i0 - 4 + xc : t.i0 + TX + xc - 4, t.j0 + xr) : BUF_NONE;
+    const unsigned oy = ys ? off(t.i0 + tx, yr < 4 ? t.j0 - 4 + yr : t.j0 + TY + yr - 4) : BUF_NONE;
+    const int px = (xr + 4) * PW + (xc < 4 ? xc : TX + xc), py = (yr < 4 ? yr : TY + yr) * PW + tx + 4;
+    const int pc = (ty + 4) * PW + tx + 4;
+    // plane k of u, v, w, T (consecutive fields)
+    long long fs = A.fs;
+    auto bs = [&](int f, int k) { return Buf<S>(A.u + (long long)(k + 4) * g.sz + f * fs, g.sz); };
+    S xv[4] = {}, yv[4] = {}, cv[4];
+    auto load_strips = [&](int k) {
+        if (ys)
 #pragma unroll
-        for (int r = 0; r < NSL; r++)
+            for (int f = 0; f < 4; f++) yv[f] = bs(f, k).ld(oy);
+        if (xs)
 #pragma unroll
-            for (int f = 0; f < 4; f++) hv[r][f] = (sl[r] >= 0 && so[r] >= 0) ? src[f][so[r] + pk] : S(0);
+            for (int f = 0; f < 4; f++) xv[f] = bs(f, k).ld(ox);
+    };
+    auto load_own = [&](int k) {
 #pragma unroll
-        for (int f = 0; f < 4; f++) cv[f] = co >= 0 ? src[f][co + pk] : S(0);
+        for (int f = 0; f < 4; f++) cv[f] = bs(f, k).ld(oc);
     };
     // z queue of the own column: q[f][m] = field f at plane k-4+m
     S q[4][9], nq[4];
 #pragma unroll
     for (int m = 0; m < 8; m++)
 #pragma unroll
-        for (int f = 0; f < 4; f++) q[f][m] = src[f][col + (long long)(t.kbeg - 4 + m) * g.sz];
+        for (int f = 0; f < 4; f++) q[f][m] = bs(f, t.kbeg - 4 + m).ld(oo);
 #pragma unroll
-    for (int f = 0; f < 4; f++) nq[f] = src[f][col + (long long)(t.kbeg + 4) * g.sz];
-    if constexpr (OCFD_VISC_RING && std::is_same<S, double>::value) {
-    // The halo strips of plane k+5 are fetched in step k, when the
-    // neighbouring tiles fetch the same rows as their own z-queue plane k+5
-    // (so one of the two reads hits L2), and wait in an LDS ring of RING
-    // planes until step k+5.  Each thread keeps its own halo positions (a
-    // dense numbering h of the strips: x strips first, then y strips), so
-    // the ring needs no barrier of its own.
-    constexpr int NHALO = 8 * TY + 8 * TX, HPT = (NHALO + NT - 1) / NT, RING = 5;
-    __shared__ S ring[RING][4][NHALO];
-    int hpos[HPT];
-    long long hoff[HPT];
-#pragma unroll
-    for (int r = 0; r < HPT; r++) {
-        const int h = tid + NT * r;
-        int hx = 0, hy = 0;
-        if (h < 8 * TY) {
-            const int c = h % 8;
-            hx = c < 4 ? c : TX + c;
-            hy = 4 + h / 8;
-        } else {
-            const int h2 = h - 8 * TY, rw = h2 / TX;
-            hx = 4 + h2 % TX;
-            hy = rw < 4 ? rw : TY + rw;
-        }
-        const int gi = i0 - 4 + hx, gj = j0 - 4 + hy;
-        hpos[r] = h < NHALO ? hy * PW + hx : -1;
-        hoff[r] = (h < NHALO && gi <= g.nx + 3 && gj <= g.ny + 3) ? gidx(g, gi, gj, 0) : -1;
-    }
-    S hn[HPT][4];
-    auto load_strips = [&](int k) {
-        const long long pk = (long long)k * g.sz;
-#pragma unroll
-        for (int r = 0; r < HPT; r++)
-#pragma unroll
-            for (int f = 0; f < 4; f++) hn[r][f] = (hoff[r] >= 0 && k < t.kend) ? src[f][hoff[r] + pk] : S(0);
-    };
-    auto store_strips = [&](int k) {
-        const int sl = (k - t.kbeg) % RING;
-#pragma unroll
-        for (int r = 0; r < HPT; r++)
-            if (hpos[r] >= 0)
-#pragma unroll
-                for (int f = 0; f < 4; f++) ring[sl][f][tid + NT * r] = hn[r][f];
-    };
-#pragma unroll
-    for (int p = 0; p < RING; p++) {
-        load_strips(t.kbeg + p);
-        store_strips(t.kbeg + p);
-    }
-#pragma unroll
-    for (int f = 0; f < 4; f++) cv[f] = co >= 0 ? src[f][co + (long long)t.kbeg * g.sz] : S(0);
+    for (int f = 0; f < 4; f++) nq[f] = bs(f, t.kbeg + 4).ld(oo);
+    load_strips(t.kbeg);
+    load_own(t.kbeg);
     for (int k = t.kbeg; k < t.kend; k++) {
-        const int sl = (k - t.kbeg) % RING;
+        fs = opaque(fs);
 #pragma unroll
         for (int f = 0; f < 4; f++) {
             q[f][8] = nq[f];
-            pl[f][(ty + 4) * PW + tx + 4] = t.own ? q[f][4] : cv[f];
-#pragma unroll
-            for (int r = 0; r < HPT; r++)
-                if (hpos[r] >= 0) pl[f][hpos[r]] = ring[sl][f][tid + NT * r];
+            pl[f][pc] = t.own ? q[f][4] : cv[f];
+            if (ys) pl[f][py] = yv[f];
+            if (xs) pl[f][px] = xv[f];
         }
+        // the point's metrics: read once, streamed; in flight across the
+        // barrier and the derivatives
+        S met[M_COUNT];
+#pragma unroll
+        for (int m = 0; m < M_COUNT; m++)
+            met[m] = S(Buf<double>(A.M[0] + (long long)(k + 4) * g.sz + m * fs, g.sz).template ld<BUF_STREAM>(od));
         __syncthreads();
         if (k + 1 < t.kend) {
 #pragma unroll
-            for (int f = 0; f < 4; f++) {
-                nq[f] = src[f][col + (long long)(k + 5) * g.sz];
-                cv[f] = co >= 0 ? src[f][co + (long long)(k + 1) * g.sz] : S(0);
-            }
-            load_strips(k + 5);
+            for (int f = 0; f < 4; f++) nq[f] = bs(f, k + 5).ld(oo);
+            load_own(k + 1);
+            load_strips(k + 1);
         }
-        if (t.own) {
-            if (near_closure<TY>(A, t, k)) gf_point<SV, S, PW, true>(A, t, k, pl, q, tx, ty, rhx, rhy, rhz);
-            else gf_point<SV, S, PW, false>(A, t, k, pl, q, tx, ty, rhx, rhy, rhz);
-        }
-        // plane k+5 into the slot plane k has just left
-        if (k + 1 < t.kend) store_strips(k + 5);
+        if (near_closure(A, t, k)) gf_point<SV, S, PW, true>(A, t, k, fs, oo, met, pl, q, tx, ty, rhx, rhy, rhz);
+        else gf_point<SV, S, PW, false>(A, t, k, fs, oo, met, pl, q, tx, ty, rhx, rhy, rhz);
 #pragma unroll
         for (int f = 0; f < 4; f++)
 #pragma unroll
             for (int m = 0; m < 8; m++) q[f][m] = q[f][m + 1];
         __syncthreads();
-    }
-    (void)sl;
-    (void)so;
-    (void)hv;
-    (void)load_plane;
-    } else {
-    load_plane(t.kbeg);
-    for (int k = t.kbeg; k < t.kend; k++) {
-        if (!VISC_PREFETCH && k > t.kbeg) {
-#pragma unroll
-            for (int f = 0; f < 4; f++) nq[f] = src[f][col + (long long)(k + 4) * g.sz];
-            load_plane(k);
-        }
-#pragma unroll
-        for (int f = 0; f < 4; f++) {
-            q[f][8] = nq[f];
-            pl[f][(ty + 4) * PW + tx + 4] = t.own ? q[f][4] : cv[f];
-#pragma unroll
-            for (int r = 0; r < NSL; r++)
-                if (sl[r] >= 0) pl[f][sl[r]] = hv[r][f];
-        }
-        __syncthreads();
-        if (VISC_PREFETCH && k + 1 < t.kend) {
-#pragma unroll
-            for (int f = 0; f < 4; f++) nq[f] = src[f][col + (long long)(k + 5) * g.sz];
-            load_plane(k + 1);
-        }
-        if (t.own) {
-            if (near_closure<TY>(A, t, k)) gf_point<SV, S, PW, true>(A, t, k, pl, q, tx, ty, rhx, rhy, rhz);
-            else gf_point<SV, S, PW, false>(A, t, k, pl, q, tx, ty, rhx, rhy, rhz);
-        }
-#pragma unroll
-        for (int f = 0; f < 4; f++)
-#pragma unroll
-            for (int m = 0; m < 8; m++) q[f][m] = q[f][m + 1];
-        __syncthreads();
-    }
     }
 }
 
@@ -427,48 +303,51 @@ __device__ __forceinline__ void p2c5(double d, double u, double v, double w, dou
 //
 // Bound by HBM.  The strips of the next plane are in flight while a plane is
 // computed.  All accesses are raw buffer accesses (Buf): with plain pointers
-// the 40 addresses of a point took the kernel to 255 VGPRs and spills, 2 waves
-// per SIMD; with them it needs 168 (3 waves), FP32 114 (4 waves).  Divergence
-// and stage as one launch against three (two of two flux components, then the
-// stage): 1024x256x128 2.42 -> 2.02 ms, 512x128x64 296 -> 224 us, mixed 215 ->
-// 170 us, 640x192x96 mixed 567 -> 467 us.
-constexpr int NTD = TX * TYD;
+// the 40 addresses of a point took the kernel to 255 VGPRs and spills (FP32:
+// slower than the separate kernels, 252 us against 215 on 512x128x64); with
+// them it needs 203, FP32 124.  Divergence and stage as one launch against
+// three (two of two flux components, then the stage): 1024x256x128 2.42 -> 2.02
+// ms, 512x128x64 296 -> 232 us, mixed 215 -> 172 us, 640x192x96 mixed 567 -> 510
+// us.
+constexpr int NTD = TX * TY;
 template <int SV, typename S, int KRK>
-__global__ void __launch_bounds__(NTD, sizeof(S) == 8 ? 3 : 4) k_visc_div(ViscArgsT<S> A, StageArgsT<S> G, int kz) {
-    static_assert(TYD == 8, "one y-halo value per thread: 8 halo rows of TX columns");
+__global__ void __launch_bounds__(NTD, sizeof(S) == 8 ? 2 : 4) k_visc_div(ViscArgsT<S> A, StageArgsT<S> G, int kz) {
+    static_assert(TY == 8, "one y-halo value per thread: 8 halo rows of TX columns");
     constexpr bool FROM_PRIM = std::is_same<S, double>::value;  // f of stages 1 and 2 lives in the primitives
-    // FP64: the point's values after the derivatives, whose registers they
-    // take over (3 waves per SIMD); FP32 has room for them before
-    constexpr bool LATE = sizeof(S) == 8;
+    // FP64, at 2 waves per SIMD, has registers to fetch the point's values a
+    // plane ahead (512x128x64: 252 -> 232 us against loads after the derivatives
+    // at 3 waves); FP32 fetches them before the derivatives and keeps 4 waves
+    // (172 us; a plane ahead 179 at 3 waves, 192 at 4)
+    constexpr bool AHEAD = sizeof(S) == 8;
     constexpr int XW = TX + 8, NC = 4;
     const Geo& g = A.g;
-    const Tile25 t = tile_of<TYD>(g, kz);
+    const Tile25 t = tile_of(g, kz);
     const int tx = threadIdx.x, ty = threadIdx.y, tid = ty * TX + tx;
     const S rhx = S(1.0 / g.hx), rhy = S(1.0 / g.hy), rhz = S(1.0 / g.hz);
-    __shared__ S ex[NC][TYD * XW];
-    __shared__ S ey[NC][(TYD + 8) * TX];
-    const long long fs = A.fs;
+    __shared__ S ex[NC][TY * XW];
+    __shared__ S ey[NC][(TY + 8) * TX];
+    long long fs = A.fs;
     // byte offset of (i, j) in a plane; i and j up to the ghost layers,
     // wrapped where the direction is periodic
     auto off = [&](int i, int j) { return (unsigned)((i + 4) + g.ldx * (j + 4)) * (unsigned)sizeof(S); };
     auto wrap = [](int i, int n, int per) { return per ? (i < 0 ? i + n : i >= n ? i - n : i) : i; };
     auto off_x = [&](int i, int j) { return i < g.nx + 4 && j < g.ny ? off(wrap(i, g.nx, A.per[0]), j) : BUF_NONE; };
     auto off_y = [&](int i, int j) { return i < g.nx && j < g.ny + 4 ? off(i, wrap(j, g.ny, A.per[1])) : BUF_NONE; };
-    // halo: x strips of 4 + 4 columns (the first 8 * TYD threads), y strips of
+    // halo: x strips of 4 + 4 columns (the first 8 * TY threads), y strips of
     // 4 + 4 rows (one value per thread)
-    const int hc = tid & 7, hr = (tid >> 3) & (TYD - 1);
-    const bool xh = tid < 8 * TYD;
+    const int hc = tid & 7, hr = (tid >> 3) & (TY - 1);
+    const bool xh = tid < 8 * TY;
     const unsigned oo = t.own ? off(t.i, t.j) : BUF_NONE;
     const unsigned od = t.own ? oo / (unsigned)sizeof(S) * 8u : BUF_NONE;  // in the FP64 fields
     const unsigned ox = off_x(t.i, t.j), oy = off_y(t.i, t.j);
     const unsigned oxh = xh ? off_x(hc < 4 ? t.i0 - 4 + hc : t.i0 + TX + hc - 4, t.j0 + hr) : BUF_NONE;
-    const unsigned oyh = off_y(t.i, ty < 4 ? t.j0 - 4 + ty : t.j0 + TYD + ty - 4);
+    const unsigned oyh = off_y(t.i, ty < 4 ? t.j0 - 4 + ty : t.j0 + TY + ty - 4);
     const int lx = ty * XW + tx + 4, lxh = hr * XW + (hc < 4 ? hc : TX + hc);
-    const int ly = (ty + 4) * TX + tx, lyh = (ty < 4 ? ty : TYD + ty) * TX + tx;
+    const int ly = (ty + 4) * TX + tx, lyh = (ty < 4 ? ty : TY + ty) * TX + tx;
     auto zwrap = [&](int k) { return A.per[2] ? (k < 0 ? k + g.nz : k >= g.nz ? k - g.nz : k) : k; };
     // plane k of field m of a group
-    auto bs = [&](const S* base, int m, int k) { return Buf<S>(base + m * fs + (long long)(k + 4) * g.sz, g.sz); };
-    auto bd = [&](const double* base, int m, int k) { return Buf<double>(base + m * fs + (long long)(k + 4) * g.sz, g.sz); };
+    auto bs = [&](const S* base, int m, int k) { return Buf<S>(base + (long long)(k + 4) * g.sz + m * fs, g.sz); };
+    auto bd = [&](const double* base, int m, int k) { return Buf<double>(base + (long long)(k + 4) * g.sz + m * fs, g.sz); };
 
     S xv[NC], yv[NC], xhv[NC] = {}, yhv[NC], q[NC][9], nq[NC];
     auto load_strips = [&](int k) {
@@ -508,7 +387,9 @@ __global__ void __launch_bounds__(NTD, sizeof(S) == 8 ? 3 : 4) k_visc_div(ViscAr
     };
     load_next(t.kbeg + 4);
     load_strips(t.kbeg);
+    if (AHEAD) load_point(t.kbeg);
     for (int k = t.kbeg; k < t.kend; k++) {
+        fs = opaque(fs);
 #pragma unroll
         for (int f = 0; f < NC; f++) {
             q[f][8] = nq[f];
@@ -542,10 +423,9 @@ __global__ void __launch_bounds__(NTD, sizeof(S) == 8 ? 3 : 4) k_visc_div(ViscAr
                 dv[m] = (double(vx) + double(vy)) + double(vz);
             }
         };
-        if (!LATE) load_point(k);
-        if (near_closure<TYD>(A, t, k)) derivs(std::true_type{});
+        if (!AHEAD) load_point(k);
+        if (near_closure(A, t, k)) derivs(std::true_type{});
         else derivs(std::false_type{});
-        if (LATE) load_point(k);
         if (!KRK) {
 #pragma unroll
             for (int m = 0; m < NC; m++) {
@@ -591,6 +471,7 @@ __global__ void __launch_bounds__(NTD, sizeof(S) == 8 ? 3 : 4) k_visc_div(ViscAr
             if (G.ghost[1] && t.own && (t.j < 4 || t.j >= g.ny - 4)) copy_to(k, off(t.i, t.j < 4 ? t.j + g.ny : t.j - g.ny));
             if (G.ghost[2] && (k < 4 || k >= g.nz - 4)) copy_to(k < 4 ? k + g.nz : k - g.nz, oo);
         }
+        if (AHEAD && k + 1 < t.kend) load_point(k + 1);
 #pragma unroll
         for (int f = 0; f < NC; f++)
 #pragma unroll
@@ -645,29 +526,26 @@ __global__ void __launch_bounds__(256) k_qcrit(ViscArgsT<S> A, double* __restric
 
 // z planes per block.  A launch that does not fill the chip is bound by the
 // longest march: its planes are spread over as many blocks as the GPU holds
-// at once (2 per CU of the FP64 kernels, 3 of the FP32 gradient kernel, 4 of
-// the FP32 divergence), each block paying the 8 planes of its z queue again
+// at once (2 per CU of the FP64 kernels, 4 of the FP32 ones), each block paying the 8 planes of its z queue again
 // from L2.  Measured, a gradient launch, against the fixed chunks: 64^3 82 ->
 // 17.5 us, 61x47x39 84 -> 13.2, 203x93x45 142 -> 53.5 (a divergence of two
 // components 38 -> 9.0, 38.5 -> 7.8, 55 -> 21.2); 512x128x64, which 32 planes
 // fill exactly, keeps them (16: 196 -> 204 us).  Larger launches take the
 // fixed chunk, where the extra z reads are what counts.
-template <typename S, bool DIV>
+template <typename S>
 int chunk_planes(const Geo& g, int cols) {
-    constexpr int RES = 256 * (std::is_same<S, double>::value ? 2 : DIV ? 4 : 3);
-    constexpr int MOST = 32;
+    constexpr int RES = 256 * (sizeof(S) == 8 ? 2 : 4), MOST = 32;
     if (cols <= RES) {
         const int nch = RES / cols, kz = (g.nz + nch - 1) / nch;
         if (kz <= MOST) return kz;
     }
-    return KZ_<S, DIV>::v;
+    return KZ_<S>::v;
 }
 
-template <typename S, bool DIV>
+template <typename S>
 dim3 grid25(const Geo& g, int& kz) {
-    constexpr int TYB = DIV ? TYD : TY_<S>::v;
-    const int gx = (g.nx + TX - 1) / TX, gy = (g.ny + TYB - 1) / TYB;
-    kz = chunk_planes<S, DIV>(g, gx * gy);
+    const int gx = (g.nx + TX - 1) / TX, gy = (g.ny + TY - 1) / TY;
+    kz = chunk_planes<S>(g, gx * gy);
     return dim3(gx, gy, (g.nz + kz - 1) / kz);
 }
 
@@ -676,7 +554,7 @@ dim3 grid25(const Geo& g, int& kz) {
 template <typename S>
 void launch_visc_gf(const ViscArgsT<S>& a, hipStream_t st) {
     int kz;
-    const dim3 grid = grid25<S, false>(a.g, kz), blk(TX, TY_<S>::v);
+    const dim3 grid = grid25<S>(a.g, kz), blk(TX, TY);
     if (a.svis == OCFD_CD6) hipLaunchKernelGGL((k_visc_gf<OCFD_CD6, S>), grid, blk, 0, st, a, kz);
     else hipLaunchKernelGGL((k_visc_gf<OCFD_CD8, S>), grid, blk, 0, st, a, kz);
 }
@@ -684,7 +562,7 @@ namespace {
 template <int SV, typename S>
 void launch_div(const ViscArgsT<S>& a, const StageArgsT<S>& st_, int krk, hipStream_t st) {
     int kz;
-    const dim3 grid = grid25<S, true>(a.g, kz), blk(TX, TYD);
+    const dim3 grid = grid25<S>(a.g, kz), blk(TX, TY);
     if (krk == 0) hipLaunchKernelGGL((k_visc_div<SV, S, 0>), grid, blk, 0, st, a, st_, kz);
     else if (krk == 1) hipLaunchKernelGGL((k_visc_div<SV, S, 1>), grid, blk, 0, st, a, st_, kz);
     else if (krk == 2) hipLaunchKernelGGL((k_visc_div<SV, S, 2>), grid, blk, 0, st, a, st_, kz);

@@ -78,6 +78,15 @@ template <typename T> struct Buf {
     }
 };
 
+// The same value, opaque to the optimiser.  Taken anew in each step of a march,
+// a field stride keeps the addresses of a step's planes (a group's base plus a
+// multiple of the stride, scalar adds) from being hoisted out of the loop,
+// where two dozen of them overflow the scalar registers.
+__device__ __forceinline__ long long opaque(long long v) {
+    asm volatile("" : "+s"(v));
+    return v;
+}
+
 // The 10 metric fields kept on the device (cofactors and Ajac,
 // src/OCFD_Comput_Jacobian3d.cu:285-295).
 enum { M_KX = 0, M_KY, M_KZ, M_IX, M_IY, M_IZ, M_SX, M_SY, M_SZ, M_JAC, M_COUNT };
