@@ -1,12 +1,11 @@
 // k_inviscid.hip - fused inviscid sweep per direction (gfx950).
 //
-// One kernel per direction replaces the reference's split kernel
+// One pass per direction replaces the reference's split kernel
 // (split_Jac3d_Stager_Warming_ker, src/OCFD_split.cu:145-198) and its ten
 // derivative launches (OCFD_d?1 / OCFD_d?2, src/OCFD_Schemes_Choose.cu:88-765,
 // each launching one P or M kernel per variable with an atomicAdd into du,
 // src/OCFD_Schemes.cu:293-381):
 //
-// x (k_sweep, LDS tile):
 //   phase 1  load rho,u,v,w,T and the direction's cofactors for a tile of
 //            nodes (+4 ghost nodes each side along the sweep), compute the
 //            sound speed and the Steger-Warming f+/f- of all 5 variables,
@@ -15,13 +14,9 @@
 //            variables with the reference's boundary closures;
 //   phase 3  one thread per node: du += -(hP(i+1/2)-hP(i-1/2))/h, then += the
 //            M term, in the reference's order (x P, x M, y P, ...), with no
-//            atomics.  The reference multiplies every term by the node's Ajac;
-//            here the RK stage multiplies their sum once (k_stage), so the
-//            sweeps do not read Ajac.
-//
-// y and z (k_tile): the same three phases on tiles of x-consecutive columns;
-// k_march (the same steps per node while marching along the sweep, with the
-// split fluxes in a register queue) is the alternative for the float path.
+//            atomics; on small grids each direction into its own five fields.
+//            The reference multiplies every term by the node's Ajac; here the
+//            RK stage multiplies their sum once, so the sweeps do not read it.
 //
 // S (double or float) is the type of the primitives, the split fluxes, the
 // reconstructions and du; the WENO weight arithmetic and the Jacobian factor
@@ -98,71 +93,44 @@ __device__ __forceinline__ void sw_split(R tmp0d, R u, R v, R w, R cc, R A1, R A
     fm[4] = tmp0d * (E1M * vv + E2M * vvc1 + E3M * vvc2 + W2 * (E2M + E3M));
 }
 
-// P and M half-node values at face j+1/2 from gp/gm = f+/f- at nodes j-3..j+4.
-// c = j+1, r = j-n (the reference's coords and coords+start-end).
-template <typename R, typename W, int SCH>
-__device__ __forceinline__ void face_pm(const R* gp, const R* gm, int c, int r, int bl, int br, int hy,
-                                        R tvlim, R tvmax, R& hp, R& hm) {
-    constexpr int kaP = Ext<SCH, 0>::ka, kbP = Ext<SCH, 0>::kb;
-    constexpr int kaM = Ext<SCH, 1>::ka, kbM = Ext<SCH, 1>::kb;
-    // ---- P (OCFD_bound_scheme_kernel_p, src/OCFD_bound_Scheme.cu:739-819)
-    if (bl && c <= -kaP) {
-        if (c == 0) hp = gp[4];
-        else if (c == 1) hp = weno5_up_left<R, W>(gp + 1);
-        else if (c == 2) hp = weno5_up_leftplus<R, W>(gp + 1);
-        else hp = weno5_up<R, W>(gp + 1);
-    } else if (br && r >= -kbP) {
-        if (r == -1) hp = gp[3] + R(0.5) * d_minmod2(gp[3] - gp[2], gp[3] - gp[2]);
-        else if (r == -2) hp = weno5_up_rightplus<R, W>(gp + 1);
-        else hp = weno5_up<R, W>(gp + 1);
-    } else {
-        if (SCH == OCFD_WENO7) hp = weno7_up<R, W>(gp);
-        else if (SCH == OCFD_UP7) hp = up7_up(gp);
-        else if (SCH == OCFD_WENO5) hp = weno5_up<R, W>(gp + 1);
-        else if (SCH == OCFD_NND2) hp = nnd2_up(gp + 2);
-        else if (SCH == OCFD_WENO7_SYMBO) hp = symbo_up<R, W>(gp, 0, tvlim, tvmax);
-        else if (SCH == OCFD_WENO7_SYMBO_LIM) hp = symbo_up<R, W>(gp, 1, tvlim, tvmax);
-        else if (SCH == OCFD_OMP6_HR) hp = omp6_up(0, gp);
-        else if (SCH == OCFD_OMP6_LD) hp = omp6_up(1, gp);
-        else if (SCH == OCFD_OMP6_CD8) hp = omp6_up(2, gp);
-        else {  // hybrid_auto, src/OCFD_Schemes_hybrid_auto.cu:911-919
-            if (hy == 1) hp = up7_up(gp);
-            else if (hy == 2) hp = weno7_up<R, W>(gp);
-            else hp = weno5_up<R, W>(gp + 1);
-        }
-    }
-    // ---- M (OCFD_bound_scheme_kernel_m, src/OCFD_bound_Scheme.cu:855-944)
-    if (bl && c < -kaM) {
-        if (c == 0) hm = weno5_dn_left<R, W>(gm + 2);
-        else if (c == 1) hm = weno5_dn_leftplus<R, W>(gm + 2);
-        else hm = weno5_dn<R, W>(gm + 2);
-    } else if (br && r >= -kbM - 1) {
-        if (r == -1) hm = gm[3];
-        else if (r == -2) hm = gm[4] - R(0.5) * d_minmod2(gm[4] - gm[3], gm[4] - gm[3]);
-        else if (r == -3) hm = weno5_dn_rightplus<R, W>(gm + 2);
-        else hm = weno5_dn<R, W>(gm + 2);
-    } else {
-        if (SCH == OCFD_WENO7) hm = weno7_dn<R, W>(gm + 1);
-        else if (SCH == OCFD_UP7) hm = up7_dn(gm);
-        else if (SCH == OCFD_WENO5) hm = weno5_dn<R, W>(gm + 2);
-        else if (SCH == OCFD_NND2) hm = nnd2_dn(gm + 3);
-        else if (SCH == OCFD_WENO7_SYMBO || SCH == OCFD_WENO7_SYMBO_LIM) hm = symbo_dn<R, W>(gm);
-        else if (SCH == OCFD_OMP6_HR) hm = omp6_dn(0, gm);
-        else if (SCH == OCFD_OMP6_LD) hm = omp6_dn(1, gm);
-        else if (SCH == OCFD_OMP6_CD8) hm = omp6_dn(2, gm);
-        else {  // src/OCFD_Schemes_hybrid_auto.cu:1008-1016
-            if (hy == 1) hm = up7_dn(gm);
-            else if (hy == 2) hm = weno7_dn<R, W>(gm + 1);
-            else hm = weno5_dn<R, W>(gm + 2);
-        }
-    }
+// f+ and f- of node (i, j, k) along direction DIR.
+template <int DIR, typename S>
+__device__ __forceinline__ void split_node(const SweepArgsT<S>& A, int i, int j, int k, S* fp, S* fm) {
+    const long long q = gidx(A.g, i, j, k);
+    const S d = A.d[q], u = A.u[q], v = A.v[q], w = A.w[q], T = A.T[q];
+    const S cc = sqrt_s(T) * S(A.c.rama);  // sound_speed_kernel, src/commen_kernel.cu:144-153
+    sw_split<S>(d * S(A.c.tmp0), u, v, w, cc, S(A.M[3 * DIR][q]), S(A.M[3 * DIR + 1][q]), S(A.M[3 * DIR + 2][q]), A.c,
+                fp, fm);
 }
 
-// The same selection for all five variables of a face: the closure/scheme
-// case of the P and the M side is decided once per face, then each case loops
-// over the variables (ld(v, k) = f+ of variable v (v < 5) or f- of variable
-// v-5 at stencil node k, k = 0..7 for nodes j-3..j+4).  Same arithmetic as
-// face_pm, with the per-variable branching hoisted.
+// The direction's part of du at node i along it (linear index q): P then M, in
+// the reference's order, the sum in double.  face(v, 0 / 1): value v (P of
+// variable v < 5, M of v - 5) at the node's left / right face.  PARTS: into the
+// direction's own group of du, else into the one du.  ACC: added to pre, what
+// du holds there; else written, streamed (nothing reads it before the next
+// sweep or the RK stage).
+template <int DIR, bool PARTS, bool ACC, typename S, typename F>
+__device__ __forceinline__ void put_du(const SweepArgsT<S>& A, int i, long long q, const double* pre, F&& face) {
+    const int n_dir = DIR == 0 ? A.g.nx : DIR == 1 ? A.g.ny : A.g.nz;
+    const bool zp = A.nrp[DIR] && i == 0, zm = A.nrm[DIR] && i == n_dir - 1;
+    const double rh = 1.0 / A.h[DIR];
+#pragma unroll
+    for (int m = 0; m < 5; m++) {
+        const double dP = zp ? 0.0 : double(face(m, 1) - face(m, 0));
+        const double dM = zm ? 0.0 : double(face(5 + m, 1) - face(5 + m, 0));
+        S* o = &A.du[((PARTS ? 5 * DIR : 0) + m) * A.fs + q];
+        if constexpr (ACC) *o = S(fma(-dM, rh, fma(-dP, rh, pre[m])));
+        else __builtin_nontemporal_store(S(fma(-dM, rh, -dP * rh)), o);
+    }
+}
+// P and M half-node values of all five variables at face j+1/2 (c = j+1, r =
+// j-n, the reference's coords and coords+start-end): the closure/scheme case
+// of the P side (OCFD_bound_scheme_kernel_p, src/OCFD_bound_Scheme.cu:739-819)
+// and of the M side (OCFD_bound_scheme_kernel_m, 855-944; hybrid_auto:
+// src/OCFD_Schemes_hybrid_auto.cu:911-919, 1008-1016) is decided once per
+// face, then each case loops over the variables (ld(v, k) = f+ of variable v
+// (v < 5) or f- of variable v-5 at stencil node k, k = 0..7 for nodes
+// j-3..j+4).
 template <typename R, typename W, int SCH, typename LD>
 __device__ __forceinline__ void face_all_p(LD&& ld, int c, int r, int bl, int br, int hy, R tvlim, R tvmax, R* hp) {
     constexpr int kaP = Ext<SCH, 0>::ka, kbP = Ext<SCH, 0>::kb;
@@ -341,9 +309,6 @@ __device__ __forceinline__ R recon_m_hybrid(int mc, const R* g) {
 // VALU-bound (91 % VALU busy on the 1024x384x256 swept ramp; 2.40 -> 2.23 ms
 // per launch); the y and z tiles, at 48-60 % VALU busy, measured the same or
 // 2 % slower with it and keep the per-face path.
-#ifndef OCFD_SWEEP_COMPACT
-#define OCFD_SWEEP_COMPACT 1
-#endif
 constexpr int COMPACT_MAX = 6;  // special faces per wave spread in one pass (10 values each)
 // The lane of the n-th special face of the wave (n-th set bit of mask).
 __device__ __forceinline__ int nth_lane(unsigned long long mask, int n) {
@@ -351,111 +316,104 @@ __device__ __forceinline__ int nth_lane(unsigned long long mask, int n) {
     return mask ? __builtin_ctzll(mask) : 0;
 }
 
-// x sweep: a block owns XA rows of 56 output nodes (one wave per row); the
-// f+/f- of the 64 nodes of a row (4 ghost nodes each side) are staged in LDS.
-#ifndef OCFD_XA
-// rows per x-sweep block (one wave each): measured 146 us with 1 row, 156 us
-// with 2 and 158 us with 4 (FP64, 512x128x64 ramp, kernel alone)
-#define OCFD_XA 1
-#endif
-constexpr int XS = 56, XA = OCFD_XA, XN = XS + 8, XF = XS + 1;
+// Orders the LDS accesses of one wave (its own LDS operations execute in
+// order; this keeps the compiler from moving them).
+__device__ __forceinline__ void wave_sync() {
+    __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+    __builtin_amdgcn_wave_barrier();
+}
+
+// x sweep.  A wave owns XR row segments of XS output nodes: its 64 lanes are the
+// XS + 8 nodes of each segment (4 ghost nodes each side), then its XS + 1 faces,
+// then its XS nodes.  One segment of 56 nodes, or two of 24 (two rows) where
+// that leaves fewer lanes idle: 64 nodes are 3 x 24 on half as many waves per
+// row (67 % of the lanes at work against 50 %), 61 nodes 64 % against 48 %.  The
+// waves of a block share nothing and wait only for themselves.
+template <int XR> struct XSeg { static constexpr int L = 64 / XR, XS = L - 8; };
 
 // LEARN (first RK stage with the learned sensor, hybrid_auto): before phase
 // 1 the wave of a row runs the learned sensor on its 64 nodes s0-4..s0+59
 // (features, two BF16-MFMA layers, the flag rule; mlp_dev.h), writes the
 // flags and probabilities of the nodes its faces use (s0-1..s0+55) and takes
 // each face's flag from the lane of its node instead of loading it.
-template <int SCH, bool FIRST, typename S, bool LEARN = false>
-__global__ void __launch_bounds__(64 * XA) k_sweep(SweepArgsT<S> A) {
-    static_assert(XF <= 64 && XN == 64, "one row per wave; one node and one face per thread");
-    __shared__ S sh[10 * XN * XA];
+//
+// bx, by, bz: segment, group of WAVES * XR rows, plane; sh: the block's LDS (640
+// values per wave).
+template <int SCH, int XR, int WAVES, bool PARTS, typename S, bool LEARN>
+__device__ __forceinline__ void sweep_x(const SweepArgsT<S>& A, int bx, int by, int bz, S* sh) {
+    constexpr int L = XSeg<XR>::L, XS = XSeg<XR>::XS;
     const Geo& g = A.g;
-    const int tid = threadIdx.x;
-    const Blk B = xcd_block();
-    const int s0 = B.x * XS, a0 = B.y * XA, k2 = B.z;
+    const int lane = threadIdx.x & 63, wv = threadIdx.x >> 6;
+    const int pos = lane % L, s0 = bx * XS, k2 = bz;
+    const int j = (by * WAVES + wv) * XR + lane / L;  // the lane's row
     const int n_dir = g.nx;
-    // LDS element (v, n, a): node-contiguous so consecutive lanes hold
-    // consecutive x
-    auto at = [](int v, int n, int a) { return (v * XA + a) * XN + n; };
+    const bool row = j < g.ny;
+    S* w = sh + wv * 640;  // value v of lane n at w[64 v + n]
 
-    // phases 2 and 3: wave a handles row a, lane = position along the row
-    // (57 faces, 56 nodes), so that the LDS accesses of a wave are
-    // consecutive doubles of one row (no bank conflicts).  The hybrid flag of
-    // this thread's face is fetched first, so that its latency hides behind
-    // phase 1
-    const int lane = tid & 63, wrow = tid >> 6;
-    const bool fthread = lane < XF;
-    const int f_loc = fthread ? lane : 0, a_loc = wrow;
-    const int jf = s0 - 1 + f_loc, acf = a0 + a_loc;
-    const bool fvalid = fthread && (jf <= n_dir - 1) && (acf < g.ny);
+    const int jf = s0 - 1 + pos;  // the lane's face jf+1/2
+    const bool fvalid = pos <= XS && jf <= n_dir - 1 && row;
     int hy = 0;
     if constexpr (LEARN) {
-        static_assert(SCH == OCFD_HYBRIDAUTO, "the learned sensor selects hybrid_auto's schemes");
-        __shared__ unsigned short sXm[XA][64 * mlp::LS];
+        static_assert(SCH == OCFD_HYBRIDAUTO && XR == 1, "the learned sensor selects hybrid_auto's schemes");
+        __shared__ unsigned short sXm[WAVES][64 * mlp::LS];
         mlp::FeatIn<S> F;
         F.g = g;
         F.d = A.d; F.u = A.u; F.v = A.v; F.w = A.w; F.T = A.T;
-        for (int m = 0; m < M_COUNT; m++) F.M[m] = A.mlp.M[m];
+        for (int m = 0; m < M_COUNT; m++) F.M[m] = A.M[m];
         F.p00 = A.c.p00;
         F.rama = A.c.rama;
-        mlp::Lane L;
-        mlp::lane_weights_packed(A.mlp.P, lane, L);
+        mlp::Lane W;
+        mlp::lane_weights_packed(A.mlp.P, lane, W);
         const int sn = s0 - 4 + lane;  // this lane's node
         const int ic = sn < -1 ? -1 : (sn > n_dir - 1 ? n_dir - 1 : sn);
-        const int jr = acf < g.ny ? acf : g.ny - 1;
+        const int jr = row ? j : g.ny - 1;
         float f[mlp::NF];
         mlp::features(F, ic, jr, k2, f);
-        const float prob = mlp::wave_prob(f, sXm[wrow], L, lane);
+        const float prob = mlp::wave_prob(f, sXm[wv], W, lane);
         const long long qn = gidx(g, ic, jr, k2);
         const int fl = mlp::flag_rule(prob, mlp::jameson_kp(F, qn, A.c.hy_i1, A.c.hy_i2), A.mlp.lo, A.mlp.hi);
-        if (lane >= 3 && lane <= 3 + XS && sn == ic && acf < g.ny) {
-            A.mlp.fx[qn] = (int8_t)fl;
+        if (lane >= 3 && lane <= 3 + XS && sn == ic && row) {
+            A.flag[0][qn] = (int8_t)fl;
             if (sn >= 0) {
-                A.mlp.fy[qn] = (int8_t)fl;
-                A.mlp.fz[qn] = (int8_t)fl;
+                A.flag[1][qn] = (int8_t)fl;
+                A.flag[2][qn] = (int8_t)fl;
             }
             if (A.mlp.prob) A.mlp.prob[qn] = prob;
         }
-        hy = __shfl(fl, f_loc + 3);  // face jf+1/2 has the flag of node jf = s0-4 + (f_loc+3)
+        hy = __shfl(fl, (lane + 3) & 63);  // face jf+1/2 has the flag of node jf = s0-4 + (lane+3)
     } else {
-        if (SCH == OCFD_HYBRIDAUTO && fvalid) hy = A.flag[gidx(g, jf, acf, k2)];
+        if (SCH == OCFD_HYBRIDAUTO && fvalid) hy = A.flag[0][gidx(g, jf, j, k2)];
     }
-    const bool nthread = lane < XS;
-    const int n3 = nthread ? lane : 0, a3 = wrow;
-    const int i3 = s0 + n3, ac3 = a0 + a3;
-    const bool nvalid = nthread && i3 < n_dir && ac3 < g.ny;
-    const long long q3 = nvalid ? gidx(g, i3, ac3, k2) : 0;
 
-    // ---- phase 1: split of XN x XA nodes into LDS
+    // ---- phase 1: split of the lane's node into LDS
     {
-        const int n = tid % XN, a = tid / XN;
-        const int s = s0 - 4 + n, ac = a0 + a;
+        const int sn = s0 - 4 + pos;
         S fp[5], fm[5];
-        if (s <= n_dir + 3 && ac < g.ny) {
-            const long long q = gidx(g, s, ac, k2);
-            const S d = A.d[q], u = A.u[q], v = A.v[q], w = A.w[q], T = A.T[q];
-            const S cc = sqrt_s(T) * S(A.c.rama);  // sound_speed_kernel, src/commen_kernel.cu:144-153
-            sw_split<S>(d * S(A.c.tmp0), u, v, w, cc, S(A.m1[q]), S(A.m2[q]), S(A.m3[q]), A.c, fp, fm);
+        if (sn <= n_dir + 3 && row) {
+            split_node<0>(A, sn, j, k2, fp, fm);
         } else {
 #pragma unroll
             for (int m = 0; m < 5; m++) { fp[m] = S(0); fm[m] = S(0); }
         }
 #pragma unroll
         for (int m = 0; m < 5; m++) {
-            sh[at(m, n, a)] = fp[m];
-            sh[at(5 + m, n, a)] = fm[m];
+            w[64 * m + lane] = fp[m];
+            w[64 * (5 + m) + lane] = fm[m];
         }
     }
-    __syncthreads();
+    wave_sync();
 
-    // ---- phase 2: one half node per thread (face jf+1/2)
+    // ---- phase 2: the lane's face (its stencil nodes are those of lanes
+    // lane..lane+7 of its segment)
     S hp[5], hm[5];
-    if (SCH == OCFD_HYBRIDAUTO && OCFD_SWEEP_COMPACT) {
+#pragma unroll
+    for (int m = 0; m < 5; m++) { hp[m] = S(0); hm[m] = S(0); }
+    const int c = jf + 1, r = jf - n_dir;
+    if constexpr (SCH == OCFD_HYBRIDAUTO) {
         int pc = 7, mc = 7;
         if (fvalid) {
-            const int c = jf + 1, r = jf - n_dir;
-            pc = case_p<SCH>(c, r, A.bl, A.br, hy);
-            mc = case_m<SCH>(c, r, A.bl, A.br, hy);
+            pc = case_p<SCH>(c, r, A.bl[0], A.br[0], hy);
+            mc = case_m<SCH>(c, r, A.bl[0], A.br[0], hy);
         }
         const bool special = fvalid && (pc != 7 || mc != 7);
         if (fvalid && !special) {
@@ -464,8 +422,8 @@ __global__ void __launch_bounds__(64 * XA) k_sweep(SweepArgsT<S> A) {
                 S gp[8], gm[8];
 #pragma unroll
                 for (int k = 0; k < 8; k++) {
-                    gp[k] = sh[at(m, f_loc + k, a_loc)];
-                    gm[k] = sh[at(5 + m, f_loc + k, a_loc)];
+                    gp[k] = w[64 * m + lane + k];
+                    gm[k] = w[64 * (5 + m) + lane + k];
                 }
                 hp[m] = up7_up(gp);
                 hm[m] = up7_dn(gm);
@@ -483,115 +441,80 @@ __global__ void __launch_bounds__(64 * XA) k_sweep(SweepArgsT<S> A) {
         if (job) {
             S gg[8];
 #pragma unroll
-            for (int k = 0; k < 8; k++) gg[k] = sh[at(v, fl + k, a_loc)];
+            for (int k = 0; k < 8; k++) gg[k] = w[64 * v + fl + k];
             res = v < 5 ? recon_p_hybrid<S, double>(pcj, gg) : recon_m_hybrid<S, double>(mcj, gg);
         }
-        if (special && !spread) {
-            const int c = jf + 1, r = jf - n_dir;
-            face_all<S, double, SCH>([&](int vv, int k) { return sh[at(vv, f_loc + k, a_loc)]; }, c, r, A.bl, A.br,
-                                     hy, S(A.c.tv_lim), S(A.c.tv_max), hp, hm);
-        }
-        __syncthreads();
-        if (fthread && !(special && spread)) {
+        if (special && !spread)
+            face_all<S, double, SCH>([&](int vv, int k) { return w[64 * vv + lane + k]; }, c, r, A.bl[0], A.br[0], hy,
+                                     S(A.c.tv_lim), S(A.c.tv_max), hp, hm);
+        wave_sync();
+        if (!(special && spread)) {
 #pragma unroll
             for (int m = 0; m < 5; m++) {
-                sh[(m * XA + a_loc) * XF + f_loc] = fvalid ? hp[m] : S(0);
-                sh[((5 + m) * XA + a_loc) * XF + f_loc] = fvalid ? hm[m] : S(0);
+                w[64 * m + lane] = hp[m];
+                w[64 * (5 + m) + lane] = hm[m];
             }
         }
-        if (job) sh[(v * XA + a_loc) * XF + fl] = res;
+        if (job) w[64 * v + fl] = res;
     } else {
-        if (fvalid) {
-            const int c = jf + 1, r = jf - n_dir;
-            face_all<S, double, SCH>([&](int v, int k) { return sh[at(v, f_loc + k, a_loc)]; }, c, r, A.bl, A.br,
-                                     hy, S(A.c.tv_lim), S(A.c.tv_max), hp, hm);
-        }
-        __syncthreads();
-        if (fthread) {
+        if (fvalid)
+            face_all<S, double, SCH>([&](int v, int k) { return w[64 * v + lane + k]; }, c, r, A.bl[0], A.br[0], hy,
+                                     S(A.c.tv_lim), S(A.c.tv_max), hp, hm);
+        wave_sync();
 #pragma unroll
-            for (int m = 0; m < 5; m++) {
-                sh[(m * XA + a_loc) * XF + f_loc] = fvalid ? hp[m] : S(0);
-                sh[((5 + m) * XA + a_loc) * XF + f_loc] = fvalid ? hm[m] : S(0);
-            }
+        for (int m = 0; m < 5; m++) {
+            w[64 * m + lane] = hp[m];
+            w[64 * (5 + m) + lane] = hm[m];
         }
     }
-    __syncthreads();
+    wave_sync();
 
-    // ---- phase 3: du at nodes, in the reference's order P then M; the
-    // accumulation is in double
-    if (nvalid) {
-        const int n = n3, a = a3, i = i3;
-        {
-            const long long q = q3;
-            const bool zp = A.nrp && i == 0;
-            const bool zm = A.nrm && i == n_dir - 1;
-            const double rh = 1.0 / A.h;
-#pragma unroll
-            for (int m = 0; m < 5; m++) {
-                const S pr = sh[(m * XA + a) * XF + n + 1], pl = sh[(m * XA + a) * XF + n];
-                const S mr = sh[((5 + m) * XA + a) * XF + n + 1], ml = sh[((5 + m) * XA + a) * XF + n];
-                const double tP = zp ? 0.0 : -double(pr - pl) * rh;
-                const double tM = zm ? 0.0 : -double(mr - ml) * rh;
-                S* dv = A.du + (long long)m * A.fs;
-                double acc = FIRST ? 0.0 : double(dv[q]);
-                acc = acc + tP;
-                acc = acc + tM;
-                // streamed: the next sweep reads it back, not this one
-                // (measured: the y sweep 182 -> 176 us)
-                __builtin_nontemporal_store(S(acc), &dv[q]);
-            }
-        }
-    }
+    // ---- phase 3: du at the lane's node i (faces i-1/2 and i+1/2 of lanes
+    // lane and lane+1)
+    const int i = s0 + pos;
+    if (pos < XS && i < n_dir && row)
+        put_du<0, PARTS, false>(A, i, gidx(g, i, j, k2), nullptr, [&](int v, int right) { return w[64 * v + lane + right]; });
 }
 
-// y and z sweeps with LDS tiles: a block owns NA x-consecutive columns (one
-// NA*8-byte row segment per node) and NS output nodes along the sweep, for one
-// value of the third index.  Same three phases as the x sweep; a thread may
-// handle up to two faces and two nodes.
-#ifdef OCFD_TILE_WPE
-#define TILE_ATTR __attribute__((amdgpu_waves_per_eu(OCFD_TILE_WPE, 8)))
-#else
-#define TILE_ATTR
-#endif
-template <int DIR, int SCH, int NS, int NA, typename S>
-__global__ void __launch_bounds__(256) TILE_ATTR k_tile(SweepArgsT<S> A) {
-    static_assert(DIR == 1 || DIR == 2, "x is swept by k_sweep");
+// y and z sweeps: a block owns NA x-consecutive columns (one NA*8-byte row
+// segment per node) and NS output nodes along the sweep, for one value of the
+// third index.  The same three phases; a thread may handle up to two faces and
+// two nodes.
+template <int DIR, int SCH, int NS, int NA, bool ACC, typename S>
+__device__ __forceinline__ void sweep_yz(const SweepArgsT<S>& A, int bx, int by, int bz, S* sh) {
+    static_assert(DIR == 1 || DIR == 2, "x is swept by sweep_x");
     constexpr int NN = NS + 8, NF = NS + 1;
-    constexpr int FPT = (NF * NA + 255) / 256;
+    constexpr int FPT = (NF * NA + 255) / 256, NPT = (NS * NA + 255) / 256;
     static_assert(FPT <= 2 && NN * NA >= NF * NA, "at most two faces per thread");
-    __shared__ S sh[10 * NN * NA];
     const Geo& g = A.g;
     const int tid = threadIdx.x;
-    const Blk B = xcd_block();
-    const int a0 = B.x * NA, s0 = B.y * NS, k2 = B.z;
+    const int a0 = bx * NA, s0 = by * NS, k2 = bz;
     const int n_dir = DIR == 1 ? g.ny : g.nz;
     auto lin = [&](int s, int a) -> long long { return DIR == 1 ? gidx(g, a, s, k2) : gidx(g, a, k2, s); };
     auto at = [](int v, int n, int a) { return (v * NN + n) * NA + a; };
 
-    // the du of this thread's output nodes is fetched first, so that its
-    // latency hides behind phases 1 and 2
-    constexpr int NPT = (NS * NA + 255) / 256;
+    // the du of this thread's output nodes and the hybrid flags of its faces are
+    // fetched first, so that their latency hides behind phases 1 and 2
     double pre_du[NPT][5];
+    if constexpr (ACC) {
 #pragma unroll
-    for (int t = 0; t < NPT; t++) {
-        const int idx = tid + 256 * t;
-        const int a = idx % NA, n = idx / NA;
-        const int i = s0 + n, ac = a0 + a;
-        if (idx < NS * NA && i < n_dir && ac < g.nx) {
-            const long long q = lin(i, ac);
+        for (int t = 0; t < NPT; t++) {
+            const int idx = tid + 256 * t;
+            const int i = s0 + idx / NA, ac = a0 + idx % NA;
+            if (idx < NS * NA && i < n_dir && ac < g.nx) {
+                const long long q = lin(i, ac);
 #pragma unroll
-            for (int m = 0; m < 5; m++) pre_du[t][m] = double(A.du[(long long)m * A.fs + q]);
+                for (int m = 0; m < 5; m++) pre_du[t][m] = double(A.du[m * A.fs + q]);
+            }
         }
     }
-
-    // hybrid flags of this thread's faces, fetched before phase 1 as well
     int pre_hy[FPT];
 #pragma unroll
     for (int t = 0; t < FPT; t++) {
         pre_hy[t] = 0;
         const int idx = tid + 256 * t;
         const int j = s0 - 1 + idx / NA, ac = a0 + idx % NA;
-        if (SCH == OCFD_HYBRIDAUTO && idx < NF * NA && j <= n_dir - 1 && ac < g.nx) pre_hy[t] = A.flag[lin(j, ac)];
+        if (SCH == OCFD_HYBRIDAUTO && idx < NF * NA && j <= n_dir - 1 && ac < g.nx) pre_hy[t] = A.flag[DIR][lin(j, ac)];
     }
 
     // ---- phase 1: split of NN x NA nodes into LDS
@@ -600,10 +523,7 @@ __global__ void __launch_bounds__(256) TILE_ATTR k_tile(SweepArgsT<S> A) {
         const int s = s0 - 4 + n, ac = a0 + a;
         S fp[5], fm[5];
         if (s <= n_dir + 3 && ac < g.nx) {
-            const long long q = lin(s, ac);
-            const S d = A.d[q], u = A.u[q], v = A.v[q], w = A.w[q], T = A.T[q];
-            const S cc = sqrt_s(T) * S(A.c.rama);  // sound_speed_kernel, src/commen_kernel.cu:144-153
-            sw_split<S>(d * S(A.c.tmp0), u, v, w, cc, S(A.m1[q]), S(A.m2[q]), S(A.m3[q]), A.c, fp, fm);
+            split_node<DIR>(A, ac, DIR == 1 ? s : k2, DIR == 1 ? k2 : s, fp, fm);
         } else {
 #pragma unroll
             for (int m = 0; m < 5; m++) { fp[m] = S(0); fm[m] = S(0); }
@@ -626,10 +546,8 @@ __global__ void __launch_bounds__(256) TILE_ATTR k_tile(SweepArgsT<S> A) {
         const int j = s0 - 1 + f_loc;  // face j+1/2
         const int ac = a0 + a_loc;
         if (j <= n_dir - 1 && ac < g.nx) {
-            const int hy = pre_hy[t];
-            const int c = j + 1, r = j - n_dir;
-            face_all<S, double, SCH>([&](int v, int k) { return sh[at(v, f_loc + k, a_loc)]; }, c, r, A.bl, A.br, hy,
-                                     S(A.c.tv_lim), S(A.c.tv_max), hp[t], hm[t]);
+            face_all<S, double, SCH>([&](int v, int k) { return sh[at(v, f_loc + k, a_loc)]; }, j + 1, j - n_dir,
+                                     A.bl[DIR], A.br[DIR], pre_hy[t], S(A.c.tv_lim), S(A.c.tv_max), hp[t], hm[t]);
         } else {
 #pragma unroll
             for (int m = 0; m < 5; m++) { hp[t][m] = S(0); hm[t][m] = S(0); }
@@ -640,124 +558,21 @@ __global__ void __launch_bounds__(256) TILE_ATTR k_tile(SweepArgsT<S> A) {
     for (int t = 0; t < FPT; t++) {
         const int idx = tid + 256 * t;
         if (idx >= NF * NA) break;
-        const int a_loc = idx % NA, f_loc = idx / NA;
 #pragma unroll
         for (int m = 0; m < 5; m++) {
-            sh[(m * NF + f_loc) * NA + a_loc] = hp[t][m];
-            sh[((5 + m) * NF + f_loc) * NA + a_loc] = hm[t][m];
+            sh[m * NF * NA + idx] = hp[t][m];
+            sh[(5 + m) * NF * NA + idx] = hm[t][m];
         }
     }
     __syncthreads();
 
-    // ---- phase 3: du at nodes (P then M; the sum in double)
-    const double rh = 1.0 / A.h;
+    // ---- phase 3: du at nodes
 #pragma unroll
     for (int t = 0; t < NPT; t++) {
         const int idx = tid + 256 * t;
-        const int a = idx % NA, n = idx / NA;
-        const int i = s0 + n, ac = a0 + a;
-        if (idx < NS * NA && i < n_dir && ac < g.nx) {
-            const long long q = lin(i, ac);
-            const bool zp = A.nrp && i == 0;
-            const bool zm = A.nrm && i == n_dir - 1;
-#pragma unroll
-            for (int m = 0; m < 5; m++) {
-                const S pr = sh[(m * NF + n + 1) * NA + a], pl = sh[(m * NF + n) * NA + a];
-                const S mr = sh[((5 + m) * NF + n + 1) * NA + a], ml = sh[((5 + m) * NF + n) * NA + a];
-                const double tP = zp ? 0.0 : -double(pr - pl) * rh;
-                const double tM = zm ? 0.0 : -double(mr - ml) * rh;
-                double acc = pre_du[t][m];
-                acc = acc + tP;
-                acc = acc + tM;
-                A.du[(long long)m * A.fs + q] = S(acc);
-            }
-        }
-    }
-}
-
-// y and z sweeps: one thread per (x, across) column marching along the sweep
-// direction over a chunk of L output nodes.  The f+/f- of the 8 nodes a face
-// needs (j-3..j+4) live in a register queue: each node is split once per chunk
-// (plus the 8 warm-up nodes), rows of 64 x-consecutive nodes are read by one
-// wave (512 contiguous bytes in FP64), and there is no LDS and no barrier.
-// The next node's inputs are fetched one iteration ahead.
-template <int DIR, int SCH, int L, typename S>
-__global__ void __launch_bounds__(256) k_march(SweepArgsT<S> A) {
-    static_assert(DIR == 1 || DIR == 2, "x is swept by k_sweep");
-    const Geo& g = A.g;
-    const int i = blockIdx.x * 64 + threadIdx.x;
-    const int a = blockIdx.y * 4 + threadIdx.y;  // z for the y sweep, y for the z sweep
-    const int n_dir = DIR == 1 ? g.ny : g.nz;
-    const int n_acr = DIR == 1 ? g.nz : g.ny;
-    const int s0 = blockIdx.z * L;
-    const int s1 = min(s0 + L, n_dir);
-    const bool own = i < g.nx && a < n_acr;
-    const int ic = min(i, g.nx - 1), acl = min(a, n_acr - 1);
-    const long long st = DIR == 1 ? (long long)g.ldx : g.sz;
-    const long long base = DIR == 1 ? gidx(g, ic, 0, acl) : gidx(g, ic, acl, 0);
-    const S* __restrict__ pd = A.d;
-    const S* __restrict__ pu = A.u;
-    const S* __restrict__ pv = A.v;
-    const S* __restrict__ pw = A.w;
-    const S* __restrict__ pT = A.T;
-    const double* __restrict__ p1 = A.m1;
-    const double* __restrict__ p2 = A.m2;
-    const double* __restrict__ p3 = A.m3;
-    const double rh = 1.0 / A.h;
-
-    S qp[5][8], qm[5][8];
-    S in[8];
-    auto fetch = [&](int s) {
-        const long long q = base + (long long)s * st;
-        in[0] = pd[q]; in[1] = pu[q]; in[2] = pv[q]; in[3] = pw[q]; in[4] = pT[q];
-        in[5] = S(p1[q]); in[6] = S(p2[q]); in[7] = S(p3[q]);
-    };
-    auto split_into = [&](int slot) {
-        const S cc = sqrt_s(in[4]) * S(A.c.rama);  // sound_speed_kernel, src/commen_kernel.cu:144-153
-        S fp[5], fm[5];
-        sw_split<S>(in[0] * S(A.c.tmp0), in[1], in[2], in[3], cc, in[5], in[6], in[7], A.c, fp, fm);
-#pragma unroll
-        for (int m = 0; m < 5; m++) { qp[m][slot] = fp[m]; qm[m][slot] = fm[m]; }
-    };
-#pragma unroll
-    for (int t = 0; t < 7; t++) {
-        fetch(s0 - 4 + t);
-        split_into(t);
-    }
-    fetch(s0 + 3);
-    S pp[5] = {0, 0, 0, 0, 0}, pm[5] = {0, 0, 0, 0, 0};
-    for (int j = s0 - 1; j < s1; j++) {
-        split_into(7);
-        if (j + 5 <= n_dir + 3) fetch(j + 5);
-        int hy = 0;
-        if (SCH == OCFD_HYBRIDAUTO) hy = A.flag[base + (long long)j * st];
-        S hp[5], hm[5];
-#pragma unroll
-        for (int m = 0; m < 5; m++)
-            face_pm<S, double, SCH>(qp[m], qm[m], j + 1, j - n_dir, A.bl, A.br, hy, S(A.c.tv_lim), S(A.c.tv_max),
-                                    hp[m], hm[m]);
-        if (j >= s0 && own) {
-            const long long q = base + (long long)j * st;
-            const bool zp = A.nrp && j == 0;
-            const bool zm = A.nrm && j == n_dir - 1;
-#pragma unroll
-            for (int m = 0; m < 5; m++) {
-                const double tP = zp ? 0.0 : -double(hp[m] - pp[m]) * rh;
-                const double tM = zm ? 0.0 : -double(hm[m] - pm[m]) * rh;
-                S* dv = A.du + (long long)m * A.fs;
-                double acc = double(dv[q]);
-                acc = acc + tP;
-                acc = acc + tM;
-                dv[q] = S(acc);
-            }
-        }
-#pragma unroll
-        for (int m = 0; m < 5; m++) {
-            pp[m] = hp[m];
-            pm[m] = hm[m];
-#pragma unroll
-            for (int t = 0; t < 7; t++) { qp[m][t] = qp[m][t + 1]; qm[m][t] = qm[m][t + 1]; }
-        }
+        const int i = s0 + idx / NA, ac = a0 + idx % NA;
+        if (idx < NS * NA && i < n_dir && ac < g.nx)
+            put_du<DIR, !ACC, ACC>(A, i, lin(i, ac), pre_du[t], [&](int v, int right) { return sh[v * NF * NA + idx + right * NA]; });
     }
 }
 
@@ -832,21 +647,19 @@ __device__ __forceinline__ void mv5(const double* M, const double* x, double* y)
 template <int DIR> struct CharTile { static constexpr int NS = 24, NA = 8; };
 template <> struct CharTile<0> { static constexpr int NS = 56, NA = 4; };
 
-// hybrid_auto is held to 3 waves per SIMD (168 VGPRs, 8 spilled): at 2 the
-// kernel is latency-bound (203x93x45, one launch: x 139 -> 111 us; y and z,
-// which were at 3, 79 -> 77 and 62 -> 60; at 4 waves 124, 90, 69).  The SYMBO
-// forms need 256 and would spill half of them.
-template <int DIR, int SCH, bool FIRST, typename S>
-__global__ void __launch_bounds__(256, SCH == OCFD_HYBRIDAUTO ? 3 : 2) k_char(SweepArgsT<S> A) {
+// bx, by, bz: tile along and across the sweep, third index; sh and shb: the
+// block's LDS.
+template <int DIR, int SCH, bool ACC, typename S>
+__device__ __forceinline__ void sweep_char(const SweepArgsT<S>& A, int bx, int by, int bz, S* sh,
+                                           S (*shb)[10][8]) {
     constexpr int NS = CharTile<DIR>::NS, NA = CharTile<DIR>::NA, NN = NS + 8, NF = NS + 1;
     static_assert(NN * NA == 256 && NF * NA <= 256 && (DIR != 0 || (NA == 4 && NF <= 64)),
                   "one node and at most one face per thread; x: one row per wave");
-    __shared__ S sh[10 * NN * NA];
-    __shared__ S shb[2][10][NA];  // boundary differences: [low/high][P 0..4, M 5..9][column]
+    // shb: boundary differences [low/high][P 0..4, M 5..9][column]
     const Geo& g = A.g;
     const int tid = threadIdx.x;
-    const Blk B = xcd_block();
-    const int s0 = (DIR == 0 ? B.x : B.y) * NS, a0 = (DIR == 0 ? B.y : B.x) * NA, k2 = B.z;
+    const int s0 = (DIR == 0 ? bx : by) * NS, a0 = (DIR == 0 ? by : bx) * NA, k2 = bz;
+    const int bl = A.bl[DIR], br = A.br[DIR];
     const int n_dir = DIR == 0 ? g.nx : DIR == 1 ? g.ny : g.nz;
     const int n_acr = DIR == 0 ? g.ny : g.nx;
     auto lin = [&](int s, int a) -> long long {
@@ -855,7 +668,7 @@ __global__ void __launch_bounds__(256, SCH == OCFD_HYBRIDAUTO ? 3 : 2) k_char(Sw
     // lanes run along x: along the sweep for x, across it for y and z
     auto at = [](int v, int n, int a) { return DIR == 0 ? (v * NA + a) * NN + n : (v * NN + n) * NA + a; };
     auto fat = [](int v, int f, int a) { return DIR == 0 ? (v * NA + a) * NF + f : (v * NF + f) * NA + a; };
-    const int fyc = A.bl && A.br ? 3 : A.bl ? 1 : A.br ? 2 : 0;  // closures: both, low, high, none
+    const int fyc = bl && br ? 3 : bl ? 1 : br ? 2 : 0;  // closures: both, low, high, none
 
     // ---- phase 1: split into LDS
     {
@@ -863,10 +676,7 @@ __global__ void __launch_bounds__(256, SCH == OCFD_HYBRIDAUTO ? 3 : 2) k_char(Sw
         const int s = s0 - 4 + n, ac = a0 + a;
         S fp[5], fm[5];
         if (s <= n_dir + 3 && ac < n_acr) {
-            const long long q = lin(s, ac);
-            const S d = A.d[q], u = A.u[q], v = A.v[q], w = A.w[q], T = A.T[q];
-            const S cc = sqrt_s(T) * S(A.c.rama);
-            sw_split<S>(d * S(A.c.tmp0), u, v, w, cc, S(A.m1[q]), S(A.m2[q]), S(A.m3[q]), A.c, fp, fm);
+            split_node<DIR>(A, DIR == 0 ? s : ac, DIR == 0 ? ac : DIR == 1 ? s : k2, DIR == 2 ? s : k2, fp, fm);
         } else {
 #pragma unroll
             for (int m = 0; m < 5; m++) { fp[m] = S(0); fm[m] = S(0); }
@@ -889,17 +699,18 @@ __global__ void __launch_bounds__(256, SCH == OCFD_HYBRIDAUTO ? 3 : 2) k_char(Sw
     if (fvalid) {
         auto ld = [&](int v, int k) { return sh[at(v, f_loc + k, a_loc)]; };
         int hy = 0;
-        if (SCH == OCFD_HYBRIDAUTO) hy = A.flag[lin(j, ac)];
+        if (SCH == OCFD_HYBRIDAUTO) hy = A.flag[DIR][lin(j, ac)];
         const int c = j + 1, r = j - n_dir;
         if (SCH == OCFD_HYBRIDAUTO && hy == 1) {
-            face_all<S, double, SCH>(ld, c, r, A.bl, A.br, hy, S(A.c.tv_lim), S(A.c.tv_max), hp, hm);
+            face_all<S, double, SCH>(ld, c, r, bl, br, hy, S(A.c.tv_lim), S(A.c.tv_max), hp, hm);
         } else {
             const long long q0 = lin(j, ac), q1 = lin(j + 1, ac);
             const double rama = A.c.rama;
+            const double *m1 = A.M[3 * DIR], *m2 = A.M[3 * DIR + 1], *m3 = A.M[3 * DIR + 2];
             CharFace F;
-            char_face(double(A.u[q0]), double(A.v[q0]), double(A.w[q0]), sqrt(double(A.T[q0])) * rama, A.m1[q0],
-                      A.m2[q0], A.m3[q0], double(A.u[q1]), double(A.v[q1]), double(A.w[q1]),
-                      sqrt(double(A.T[q1])) * rama, A.m1[q1], A.m2[q1], A.m3[q1], A.c.gamma, F);
+            char_face(double(A.u[q0]), double(A.v[q0]), double(A.w[q0]), sqrt(double(A.T[q0])) * rama, m1[q0],
+                      m2[q0], m3[q0], double(A.u[q1]), double(A.v[q1]), double(A.w[q1]),
+                      sqrt(double(A.T[q1])) * rama, m1[q1], m2[q1], m3[q1], A.c.gamma, F);
             S cs[5][8];
             double x[5], y[5], hc[5];
             S hcs[5];
@@ -911,7 +722,7 @@ __global__ void __launch_bounds__(256, SCH == OCFD_HYBRIDAUTO ? 3 : 2) k_char(Sw
 #pragma unroll
                 for (int m = 0; m < 5; m++) cs[m][k] = S(y[m]);
             }
-            face_all_p<S, double, SCH>([&](int v, int k) { return cs[v][k]; }, c, r, A.bl, A.br, hy,
+            face_all_p<S, double, SCH>([&](int v, int k) { return cs[v][k]; }, c, r, bl, br, hy,
                                        S(A.c.tv_lim), S(A.c.tv_max), hcs);
 #pragma unroll
             for (int m = 0; m < 5; m++) hc[m] = double(hcs[m]);
@@ -926,7 +737,7 @@ __global__ void __launch_bounds__(256, SCH == OCFD_HYBRIDAUTO ? 3 : 2) k_char(Sw
 #pragma unroll
                 for (int m = 0; m < 5; m++) cs[m][k] = S(y[m]);
             }
-            face_all_m<S, double, SCH>([&](int v, int k) { return cs[v - 5][k]; }, c, r, A.bl, A.br, hy, hcs);
+            face_all_m<S, double, SCH>([&](int v, int k) { return cs[v - 5][k]; }, c, r, bl, br, hy, hcs);
 #pragma unroll
             for (int m = 0; m < 5; m++) hc[m] = double(hcs[m]);
             mv5(F.R, hc, y);
@@ -968,144 +779,215 @@ __global__ void __launch_bounds__(256, SCH == OCFD_HYBRIDAUTO ? 3 : 2) k_char(Sw
         const int i = s0 + n, ai = a0 + a;
         if (i < n_dir && ai < n_acr) {
             const long long q = lin(i, ai);
-            const double rh = 1.0 / A.h;
+            const double rh = 1.0 / A.h[DIR];
             const bool lowP = fyc == 1 && i == 0, highP = fyc == 2 && i == n_dir - 1;
             const bool highM = fyc == 2 && i == n_dir - 1, lowM = fyc == 1 && i == 0 && DIR != 1;
 #pragma unroll
             for (int m = 0; m < 5; m++) {
                 double tP, tM;
-                if (lowP) tP = A.nrp ? 0.0 : -double(shb[0][m][a]) * rh;
+                if (lowP) tP = A.nrp[DIR] ? 0.0 : -double(shb[0][m][a]) * rh;
                 else if (highP) tP = -double(shb[1][m][a]) * rh;
                 else tP = -double(sh[fat(m, n + 1, a)] - sh[fat(m, n, a)]) * rh;
-                if (highM) tM = A.nrm ? 0.0 : -double(shb[1][5 + m][a]) * rh;
+                if (highM) tM = A.nrm[DIR] ? 0.0 : -double(shb[1][5 + m][a]) * rh;
                 else if (lowM) tM = -double(shb[0][5 + m][a]) * rh;
                 else tM = -double(sh[fat(5 + m, n + 1, a)] - sh[fat(5 + m, n, a)]) * rh;
-                S* dv = A.du + (long long)m * A.fs;
-                double acc = FIRST ? 0.0 : double(dv[q]);
-                acc = acc + tP;
-                acc = acc + tM;
-                dv[q] = S(acc);
+                S* o = &A.du[m * A.fs + q];
+                if constexpr (ACC) *o = S((double(*o) + tP) + tM);
+                else __builtin_nontemporal_store(S(tP + tM), o);
             }
         }
     }
 }
 
-template <int DIR, int SCH, typename S>
-void launch_char_dir(const SweepArgsT<S>& a, bool first, hipStream_t st) {
-    constexpr int NS = CharTile<DIR>::NS, NA = CharTile<DIR>::NA;
-    const Geo& g = a.g;
-    const int n_dir = DIR == 0 ? g.nx : DIR == 1 ? g.ny : g.nz;
-    const int n_acr = DIR == 0 ? g.ny : g.nx;
-    const int third = DIR == 0 ? g.nz : DIR == 1 ? g.nz : g.ny;
-    const dim3 grid = DIR == 0 ? dim3((n_dir + NS - 1) / NS, (n_acr + NA - 1) / NA, third)
-                               : dim3((n_acr + NA - 1) / NA, (n_dir + NS - 1) / NS, third);
-    if (first) hipLaunchKernelGGL((k_char<DIR, SCH, true, S>), grid, dim3(256), 0, st, a);
-    else hipLaunchKernelGGL((k_char<DIR, SCH, false, S>), grid, dim3(256), 0, st, a);
+// y/z tile shapes (output nodes x columns).  FP64: 14 nodes x 16 columns
+// (128-byte row segments): on the 1024x384x256 swept ramp the y sweep 3.58-3.74
+// -> 3.43-3.53 ms and the z sweep 3.91-4.00 -> 3.53-3.58 ms against 28 x 8 (12 x
+// 16 in between; 56 x 4, 4.4 and 6.2 ms), although it splits 1.57 nodes per
+// output node against 1.29.
+template <typename S> struct YZ { static constexpr int NS = 14, NA = 16; };
+template <> struct YZ<float> { static constexpr int NS = 15, NA = 16; };
+
+// ---------------------------------------------------------------------------
+// One launch per direction: x writes du, y and z add to it.  A wave of the x
+// sweep is a block of its own.
+// ---------------------------------------------------------------------------
+template <int SCH, int XR, typename S, bool LEARN>
+__global__ void __launch_bounds__(64) k_sweep_x(SweepArgsT<S> A) {
+    __shared__ S sh[640];
+    const Blk B = xcd_block();
+    sweep_x<SCH, XR, 1, false, S, LEARN>(A, B.x, B.y, B.z, sh);
 }
+template <int DIR, int SCH, typename S>
+__global__ void __launch_bounds__(256) k_sweep_yz(SweepArgsT<S> A) {
+    constexpr int NS = YZ<S>::NS, NA = YZ<S>::NA;
+    __shared__ S sh[10 * (NS + 8) * NA];
+    const Blk B = xcd_block();
+    sweep_yz<DIR, SCH, NS, NA, true, S>(A, B.x, B.y, B.z, sh);
+}
+// hybrid_auto is held to 3 waves per SIMD (168 VGPRs, 8 spilled): at 2 the
+// kernel is latency-bound (203x93x45, one launch: x 139 -> 111 us; y and z,
+// which were at 3, 79 -> 77 and 62 -> 60; at 4 waves 124, 90, 69).  The SYMBO
+// forms need 256 and would spill half of them.
+template <int DIR, int SCH, typename S>
+__global__ void __launch_bounds__(256, SCH == OCFD_HYBRIDAUTO ? 3 : 2) k_char(SweepArgsT<S> A) {
+    using C = CharTile<DIR>;
+    __shared__ S sh[10 * (C::NS + 8) * C::NA];
+    __shared__ S shb[2][10][8];
+    const Blk B = xcd_block();
+    sweep_char<DIR, SCH, DIR != 0, S>(A, B.x, B.y, B.z, sh, shb);
+}
+
+// ---------------------------------------------------------------------------
+// The three sweeps in one launch, each direction writing its part of du to
+// its own five fields, which the RK stage adds: the sweeps then
+// depend on nothing but the stage's state.  For small grids (sweeps_merged):
+// a launch of theirs is as long as its slowest block, and three of them with
+// their gaps are replaced by one (64^3: 24 + 21 + 21 us -> 48 us, 20x16x12: 9 +
+// 10 + 10 -> 10).  On larger ones it gains less than the stage pays for reading
+// three parts (256x128x128: 712 -> 670 us, the stage 234 -> 297;
+// 1024x256x128: 2.96 -> 2.92 ms and 2.02 -> 2.60).  Blocks in the order x, y, z;
+// cutting the domain into boxes whose x, y and z blocks follow one another, for
+// the Infinity Cache, was slower at every size (64^3 51-59 us, 256x128x128
+// 720-860).
+// ---------------------------------------------------------------------------
+struct SweepGrid {
+    int nt[3][3];  // tiles of a direction along x, y, z
+    int run[3];    // its blocks, a multiple of 8
+};
+// Tile of block b of a direction: the blocks an XCD gets (every eighth) are
+// neighbours, as in xcd_block(); false: a padding block.
+__device__ __forceinline__ bool run_tile(unsigned b, int run, const int* nt, Blk& t) {
+    const int q = (int)(b & 7u) * (run >> 3) + (int)(b >> 3);
+    if (q >= nt[0] * nt[1] * nt[2]) return false;
+    t.x = q % nt[0];
+    t.y = (q / nt[0]) % nt[1];
+    t.z = q / (nt[0] * nt[1]);
+    return true;
+}
+constexpr int XWAVES = 4;  // waves of an x block here
+template <int SCH, int XR, typename S>
+__global__ void __launch_bounds__(256) k_sweeps(SweepArgsT<S> A, SweepGrid G) {
+    constexpr int NS = YZ<S>::NS, NA = YZ<S>::NA;
+    constexpr int LDS_YZ = 10 * (NS + 8) * NA, LDS_X = 640 * XWAVES;
+    __shared__ S sh[LDS_YZ > LDS_X ? LDS_YZ : LDS_X];
+    unsigned b = blockIdx.x;
+    Blk t;
+    if (b < (unsigned)G.run[0]) {
+        if (run_tile(b, G.run[0], G.nt[0], t)) sweep_x<SCH, XR, XWAVES, true, S, false>(A, t.x, t.y, t.z, sh);
+        return;
+    }
+    b -= G.run[0];
+    if (b < (unsigned)G.run[1]) {
+        if (run_tile(b, G.run[1], G.nt[1], t)) sweep_yz<1, SCH, NS, NA, false, S>(A, t.x, t.y, t.z, sh);
+        return;
+    }
+    b -= G.run[1];
+    if (run_tile(b, G.run[2], G.nt[2], t)) sweep_yz<2, SCH, NS, NA, false, S>(A, t.x, t.y, t.z, sh);
+}
+
+int tiles(int n, int t) { return (n + t - 1) / t; }
+// Two segments per wave where a row's waves then come to less than half.
+bool two_segments(const Geo& g) { return tiles(g.nx, XSeg<2>::XS) < 2 * tiles(g.nx, XSeg<1>::XS); }
+
+// first: 0 for all three directions, 1 for y and z.
 template <int SCH, typename S>
-void launch_char_scheme(int dir, const SweepArgsT<S>& a, bool first, hipStream_t st) {
-    if (dir == 0) launch_char_dir<0, SCH>(a, first, st);
-    else if (dir == 1) launch_char_dir<1, SCH>(a, first, st);
-    else launch_char_dir<2, SCH>(a, first, st);
+void launch_merged(const SweepArgsT<S>& a, int first, hipStream_t st) {
+    const Geo& g = a.g;
+    constexpr int NS = YZ<S>::NS, NA = YZ<S>::NA;
+    const bool two = two_segments(g);
+    const int xs = two ? XSeg<2>::XS : XSeg<1>::XS, rows = XWAVES * (two ? 2 : 1);
+    const SweepGrid z{};
+    SweepGrid G = z;
+    const int nt[3][3] = {{tiles(g.nx, xs), tiles(g.ny, rows), g.nz},
+                          {tiles(g.nx, NA), tiles(g.ny, NS), g.nz},
+                          {tiles(g.nx, NA), tiles(g.nz, NS), g.ny}};
+    unsigned nb = 0;
+    for (int d = first; d < 3; d++) {
+        for (int q = 0; q < 3; q++) G.nt[d][q] = nt[d][q];
+        G.run[d] = tiles(nt[d][0] * nt[d][1] * nt[d][2], 8) * 8;
+        nb += G.run[d];
+    }
+    if (two) hipLaunchKernelGGL((k_sweeps<SCH, 2, S>), dim3(nb), dim3(256), 0, st, a, G);
+    else hipLaunchKernelGGL((k_sweeps<SCH, 1, S>), dim3(nb), dim3(256), 0, st, a, G);
 }
 
-#ifndef OCFD_LMARCH
-#define OCFD_LMARCH 32  // output nodes per marching chunk (k_march)
-#endif
-// y/z tile shapes (output nodes x columns).  Measured on the 512x128x64 ramp
-// (FP64, 28 x 8 tiles): NS = 32 with 320 threads (no partial tile on lines
-// of 64 and 128 nodes) is 10-20 % slower than NS = 28 with 256 threads; a
-// per-block queue that hands
-// the rare WENO faces of hybrid_auto to all threads, and a form with the face
-// pass fused into the node pass by cross-lane shuffles (one more resident
-// wave per SIMD), were no faster.
-// FP64: 14 nodes x 16 columns (128-byte row segments): on the 1024x384x256
-// swept ramp the y sweep 3.58-3.74 -> 3.43-3.53 ms and the z sweep
-// 3.91-4.00 -> 3.53-3.58 ms against 28 x 8 (12 x 16 in between; 56 x 4, 4.4
-// and 6.2 ms), although it splits 1.57 nodes per output node against 1.29.
-#ifndef OCFD_YZ_NS_D
-#define OCFD_YZ_NS_D 14
-#endif
-#ifndef OCFD_YZ_NA_D
-#define OCFD_YZ_NA_D 16
-#endif
-#ifndef OCFD_YZ_NS_F
-#define OCFD_YZ_NS_F 15
-#endif
-#ifndef OCFD_YZ_NA_F
-#define OCFD_YZ_NA_F 16
-#endif
-#ifndef OCFD_MARCH_F32
-#define OCFD_MARCH_F32 0  // y/z sweeps of the float path: 1 = k_march, 0 = k_tile
-#endif
-constexpr int LMARCH = OCFD_LMARCH;
-template <typename S> struct YZ { static constexpr int NS = OCFD_YZ_NS_D, NA = OCFD_YZ_NA_D; };
-template <> struct YZ<float> { static constexpr int NS = OCFD_YZ_NS_F, NA = OCFD_YZ_NA_F; };
-
-template <int DIR, int SCH, typename S>
-void launch_dir(const SweepArgsT<S>& a, bool first, hipStream_t st) {
+template <int SCH, typename S>
+void launch_scheme(int dir, const SweepArgsT<S>& a, hipStream_t st) {
     const Geo& g = a.g;
-    if constexpr (DIR == 0) {
-        dim3 grid((g.nx + XS - 1) / XS, (g.ny + XA - 1) / XA, g.nz);
+    constexpr int NS = YZ<S>::NS, NA = YZ<S>::NA;
+    if (dir < 0) {
+        launch_merged<SCH>(a, dir == SWEEP_YZ, st);
+    } else if (dir == 0) {
         if constexpr (SCH == OCFD_HYBRIDAUTO) {
-            if (a.mlp.P && first) {
-                hipLaunchKernelGGL((k_sweep<SCH, true, S, true>), grid, dim3(64 * XA), 0, st, a);
+            if (a.mlp.P) {
+                hipLaunchKernelGGL((k_sweep_x<SCH, 1, S, true>), dim3(tiles(g.nx, XSeg<1>::XS), g.ny, g.nz), dim3(64), 0,
+                                   st, a);
                 return;
             }
         }
-        if (first) hipLaunchKernelGGL((k_sweep<SCH, true, S>), grid, dim3(64 * XA), 0, st, a);
-        else hipLaunchKernelGGL((k_sweep<SCH, false, S>), grid, dim3(64 * XA), 0, st, a);
+        if (two_segments(g))
+            hipLaunchKernelGGL((k_sweep_x<SCH, 2, S, false>), dim3(tiles(g.nx, XSeg<2>::XS), tiles(g.ny, 2), g.nz),
+                               dim3(64), 0, st, a);
+        else
+            hipLaunchKernelGGL((k_sweep_x<SCH, 1, S, false>), dim3(tiles(g.nx, XSeg<1>::XS), g.ny, g.nz), dim3(64), 0, st,
+                               a);
+    } else if (dir == 1) {
+        hipLaunchKernelGGL((k_sweep_yz<1, SCH, S>), dim3(tiles(g.nx, NA), tiles(g.ny, NS), g.nz), dim3(256), 0, st, a);
     } else {
-        const int n_dir = DIR == 1 ? g.ny : g.nz, n_acr = DIR == 1 ? g.nz : g.ny;
-        if constexpr (std::is_same<S, float>::value && OCFD_MARCH_F32) {
-            dim3 grid((g.nx + 63) / 64, (n_acr + 3) / 4, (n_dir + LMARCH - 1) / LMARCH);
-            hipLaunchKernelGGL((k_march<DIR, SCH, LMARCH, S>), grid, dim3(64, 4), 0, st, a);
-        } else {
-            constexpr int NS = YZ<S>::NS, NA = YZ<S>::NA;
-            dim3 grid((g.nx + NA - 1) / NA, (n_dir + NS - 1) / NS, n_acr);
-            hipLaunchKernelGGL((k_tile<DIR, SCH, NS, NA, S>), grid, dim3(256), 0, st, a);
-        }
+        hipLaunchKernelGGL((k_sweep_yz<2, SCH, S>), dim3(tiles(g.nx, NA), tiles(g.nz, NS), g.ny), dim3(256), 0, st, a);
     }
 }
-
 template <int SCH, typename S>
-void launch_scheme(int dir, const SweepArgsT<S>& a, bool first, hipStream_t st) {
-    if (dir == 0) launch_dir<0, SCH>(a, first, st);
-    else if (dir == 1) launch_dir<1, SCH>(a, first, st);
-    else launch_dir<2, SCH>(a, first, st);
+void launch_char_scheme(int dir, const SweepArgsT<S>& a, hipStream_t st) {
+    const Geo& g = a.g;
+    if (dir == 0)
+        hipLaunchKernelGGL((k_char<0, SCH, S>), dim3(tiles(g.nx, CharTile<0>::NS), tiles(g.ny, CharTile<0>::NA), g.nz),
+                           dim3(256), 0, st, a);
+    else if (dir == 1)
+        hipLaunchKernelGGL((k_char<1, SCH, S>), dim3(tiles(g.nx, CharTile<1>::NA), tiles(g.ny, CharTile<1>::NS), g.nz),
+                           dim3(256), 0, st, a);
+    else
+        hipLaunchKernelGGL((k_char<2, SCH, S>), dim3(tiles(g.nx, CharTile<2>::NA), tiles(g.nz, CharTile<2>::NS), g.ny),
+                           dim3(256), 0, st, a);
 }
 
 }  // namespace
 
-template <typename S>
-int launch_sweep(int scheme, int dir, const SweepArgsT<S>& a, bool first, hipStream_t st) {
-    switch (scheme) {
-    case OCFD_UP7: launch_scheme<OCFD_UP7>(dir, a, first, st); break;
-    case OCFD_WENO5: launch_scheme<OCFD_WENO5>(dir, a, first, st); break;
-    case OCFD_WENO7: launch_scheme<OCFD_WENO7>(dir, a, first, st); break;
-    case OCFD_WENO7_SYMBO: launch_scheme<OCFD_WENO7_SYMBO>(dir, a, first, st); break;
-    case OCFD_WENO7_SYMBO_LIM: launch_scheme<OCFD_WENO7_SYMBO_LIM>(dir, a, first, st); break;
-    case OCFD_NND2: launch_scheme<OCFD_NND2>(dir, a, first, st); break;
-    case OCFD_OMP6_HR: launch_scheme<OCFD_OMP6_HR>(dir, a, first, st); break;
-    case OCFD_OMP6_LD: launch_scheme<OCFD_OMP6_LD>(dir, a, first, st); break;
-    case OCFD_OMP6_CD8: launch_scheme<OCFD_OMP6_CD8>(dir, a, first, st); break;
-    case OCFD_HYBRIDAUTO: launch_scheme<OCFD_HYBRIDAUTO>(dir, a, first, st); break;
-    default: return -1;
-    }
-    return 0;
-}
-template int launch_sweep<double>(int, int, const SweepArgsT<double>&, bool, hipStream_t);
-template int launch_sweep<float>(int, int, const SweepArgsT<float>&, bool, hipStream_t);
+// Points up to which the three sweeps of a stage run in one launch, on one
+// stream with the rest of the stage: 20x16x12 140 -> 63 us a step, 64^3
+// 296 -> 244, 61x47x39 161 -> 114, 97x61x53 540 -> 510; above, 131x99x80 mixed
+// 660 -> 667, 256x128x128 3168 -> 3300.
+bool sweeps_merged(const Geo& g) { return (long long)g.nx * g.ny * g.nz <= 500000; }
 
 template <typename S>
-int launch_sweep_char(int scheme, int dir, const SweepArgsT<S>& a, bool first, hipStream_t st) {
+int launch_sweep(int scheme, int dir, const SweepArgsT<S>& a, hipStream_t st) {
     switch (scheme) {
-    case OCFD_WENO7_SYMBO: launch_char_scheme<OCFD_WENO7_SYMBO>(dir, a, first, st); break;
-    case OCFD_WENO7_SYMBO_LIM: launch_char_scheme<OCFD_WENO7_SYMBO_LIM>(dir, a, first, st); break;
-    case OCFD_HYBRIDAUTO: launch_char_scheme<OCFD_HYBRIDAUTO>(dir, a, first, st); break;
+    case OCFD_UP7: launch_scheme<OCFD_UP7>(dir, a, st); break;
+    case OCFD_WENO5: launch_scheme<OCFD_WENO5>(dir, a, st); break;
+    case OCFD_WENO7: launch_scheme<OCFD_WENO7>(dir, a, st); break;
+    case OCFD_WENO7_SYMBO: launch_scheme<OCFD_WENO7_SYMBO>(dir, a, st); break;
+    case OCFD_WENO7_SYMBO_LIM: launch_scheme<OCFD_WENO7_SYMBO_LIM>(dir, a, st); break;
+    case OCFD_NND2: launch_scheme<OCFD_NND2>(dir, a, st); break;
+    case OCFD_OMP6_HR: launch_scheme<OCFD_OMP6_HR>(dir, a, st); break;
+    case OCFD_OMP6_LD: launch_scheme<OCFD_OMP6_LD>(dir, a, st); break;
+    case OCFD_OMP6_CD8: launch_scheme<OCFD_OMP6_CD8>(dir, a, st); break;
+    case OCFD_HYBRIDAUTO: launch_scheme<OCFD_HYBRIDAUTO>(dir, a, st); break;
     default: return -1;
     }
     return 0;
 }
-template int launch_sweep_char<double>(int, int, const SweepArgsT<double>&, bool, hipStream_t);
-template int launch_sweep_char<float>(int, int, const SweepArgsT<float>&, bool, hipStream_t);
+template int launch_sweep<double>(int, int, const SweepArgsT<double>&, hipStream_t);
+template int launch_sweep<float>(int, int, const SweepArgsT<float>&, hipStream_t);
+
+template <typename S>
+int launch_sweep_char(int scheme, int dir, const SweepArgsT<S>& a, hipStream_t st) {
+    switch (scheme) {
+    case OCFD_WENO7_SYMBO: launch_char_scheme<OCFD_WENO7_SYMBO>(dir, a, st); break;
+    case OCFD_WENO7_SYMBO_LIM: launch_char_scheme<OCFD_WENO7_SYMBO_LIM>(dir, a, st); break;
+    case OCFD_HYBRIDAUTO: launch_char_scheme<OCFD_HYBRIDAUTO>(dir, a, st); break;
+    default: return -1;
+    }
+    return 0;
+}
+template int launch_sweep_char<double>(int, int, const SweepArgsT<double>&, hipStream_t);
+template int launch_sweep_char<float>(int, int, const SweepArgsT<float>&, hipStream_t);

@@ -62,14 +62,15 @@ __global__ void __launch_bounds__(256) k_stage(StageArgsT<S> A) {
     const int i = blockIdx.x * 64 + threadIdx.x, j = blockIdx.y * 4 + threadIdx.y, k = blockIdx.z;
     if (i >= A.g.nx || j >= A.g.ny) return;
     const long long q = gidx(A.g, i, j, k);
-    // du, plus its viscous part dv (components 1..4) when that is kept apart
-    // du and dv are read once, as streaming (non-temporal) loads
+    // the inviscid part (or parts of x, y and z), then the viscous part
+    // (components 1..4), all read once as streaming (non-temporal) loads
     double du[5];
 #pragma unroll
-    for (int m = 0; m < 5; m++) du[m] = double(__builtin_nontemporal_load(&A.du[m * A.fs + q]));
-    if (A.dv) {
-#pragma unroll
-        for (int m = 1; m < 5; m++) du[m] += double(__builtin_nontemporal_load(&A.dv[(m - 1) * A.fs + q]));
+    for (int m = 0; m < 5; m++) {
+        auto part = [&](int dir) { return double(__builtin_nontemporal_load(&A.du[(5 * dir + m) * A.fs + q])); };
+        du[m] = part(0);
+        if (A.parts == 3) du[m] = (du[m] + part(1)) + part(2);
+        if (m) du[m] += double(__builtin_nontemporal_load(&A.dv[(m - 1) * A.fs + q]));
     }
     // the sweeps and the divergence leave out the node's Ajac, by which the
     // reference multiplies each of their terms: it is applied to the sum here

@@ -14,8 +14,7 @@
 //                YF_Pe_XF, src/OCFD_NS_Jacobian3d.cu:304-440,
 //                src/commen_kernel.cu:158-169), no atomics, and with it the
 //                RK stage of the point; or, for callers that want the
-//                right-hand side in memory, the divergence alone (FP64: into
-//                its own buffer dv, so that it may run beside the sweeps).
+//                right-hand side in memory, the divergence alone.
 //   k_qcrit    : the Q criterion of the analysis events (same derivatives).
 //
 // S (double or float) is the type of u,v,w,T, mu, the derivatives, the
@@ -289,14 +288,14 @@ __device__ __forceinline__ void p2c5(double d, double u, double v, double w, dou
 // neighbours; periodic neighbours are read where they are, so the Ev ghost
 // layers are never filled and stay 0) and, with KRK = 1..3, the RK stage of
 // the point that it completes: the viscous terms never go to memory.  KRK = 0
-// leaves the right-hand side in memory (dv, or added to du) for the callers
-// that want it there.
+// leaves them in memory (dv) for the callers that want them there.
 //
 // The stage as OCFD_time_advance_ker1/2/3 (src/OCFD_time.cu:44-94) with
 // cons->prim + p (cons_to_pri_kernel, src/commen_kernel.cu:77-109).  FP64: the
 // conserved state of stages 1 and 2 is not written; the next stage forms it
 // from the primitives, which hold the same state in the same precision (an
 // ulp).  The mixed path, whose primitives are FP32, keeps f in every stage.
+// PARTS: groups of du to add (1, or 3 where each sweep writes its own).
 // G.faces: f of the six faces from the primitives as OCFD_bc leaves it
 // (src/OCFD_boundary.cu:40-91), for runs whose boundary condition changes
 // nothing else; G.ghost[dir]: the point's copy in the periodic ghost layers.
@@ -310,7 +309,7 @@ __device__ __forceinline__ void p2c5(double d, double u, double v, double w, dou
 // ms, 512x128x64 296 -> 232 us, mixed 215 -> 172 us, 640x192x96 mixed 567 -> 510
 // us.
 constexpr int NTD = TX * TY;
-template <int SV, typename S, int KRK>
+template <int SV, typename S, int KRK, int PARTS>
 __global__ void __launch_bounds__(NTD, sizeof(S) == 8 ? 2 : 4) k_visc_div(ViscArgsT<S> A, StageArgsT<S> G, int kz) {
     static_assert(TY == 8, "one y-halo value per thread: 8 halo rows of TX columns");
     constexpr bool FROM_PRIM = std::is_same<S, double>::value;  // f of stages 1 and 2 lives in the primitives
@@ -363,12 +362,15 @@ __global__ void __launch_bounds__(NTD, sizeof(S) == 8 ? 2 : 4) k_visc_div(ViscAr
     };
     // the stage's own values of the point: du, Ajac, the base state fn and
     // the state before the stage (the primitives, or f on the mixed path)
-    double sr[5], sj = 0.0, sn[5], so[5];
+    // (as loaded: nothing waits for them before the point is formed)
+    S sr[PARTS][5];
+    double sj = 0.0, sn[5], so[5];
     auto load_point = [&](int k) {
-        if (KRK || !A.dv)
-#pragma unroll
-            for (int m = 0; m < 5; m++) sr[m] = double(bs(A.du, m, k).template ld<BUF_STREAM>(oo));
         if (!KRK) return;
+#pragma unroll
+        for (int p = 0; p < PARTS; p++)
+#pragma unroll
+            for (int m = 0; m < 5; m++) sr[p][m] = bs(G.du, 5 * p + m, k).template ld<BUF_STREAM>(oo);
         sj = bd(G.jac, 0, k).template ld<BUF_STREAM>(od);
 #pragma unroll
         for (int m = 0; m < 5; m++) sn[m] = bd(G.fn, m, k).template ld<BUF_STREAM>(od);
@@ -428,10 +430,7 @@ __global__ void __launch_bounds__(NTD, sizeof(S) == 8 ? 2 : 4) k_visc_div(ViscAr
         else derivs(std::false_type{});
         if (!KRK) {
 #pragma unroll
-            for (int m = 0; m < NC; m++) {
-                if (A.dv) bs(A.dv, m, k).st(oo, S(dv[m]));
-                else bs(A.du, m + 1, k).st(oo, S(sr[m + 1] + dv[m]));
-            }
+            for (int m = 0; m < NC; m++) bs(A.dv, m, k).st(oo, S(dv[m]));
         } else {
             const double dt = G.dt;
             double fo[5], fv[5];
@@ -443,7 +442,11 @@ __global__ void __launch_bounds__(NTD, sizeof(S) == 8 ? 2 : 4) k_visc_div(ViscAr
             }
 #pragma unroll
             for (int m = 0; m < 5; m++) {
-                const double r = (m ? sr[m] + dv[m - 1] : sr[m]) * sj;
+                double r = double(sr[0][m]);
+#pragma unroll
+                for (int p = 1; p < PARTS; p++) r += double(sr[p][m]);
+                if (m) r += dv[m - 1];
+                r *= sj;
                 if (KRK == 1) fv[m] = sn[m] + dt * r;
                 else if (KRK == 2) fv[m] = 3.0 / 4.0 * sn[m] + 1.0 / 4.0 * (fo[m] + dt * r);
                 else fv[m] = 1.0 / 3.0 * sn[m] + 2.0 / 3.0 * (fo[m] + dt * r);
@@ -563,10 +566,17 @@ template <int SV, typename S>
 void launch_div(const ViscArgsT<S>& a, const StageArgsT<S>& st_, int krk, hipStream_t st) {
     int kz;
     const dim3 grid = grid25<S>(a.g, kz), blk(TX, TY);
-    if (krk == 0) hipLaunchKernelGGL((k_visc_div<SV, S, 0>), grid, blk, 0, st, a, st_, kz);
-    else if (krk == 1) hipLaunchKernelGGL((k_visc_div<SV, S, 1>), grid, blk, 0, st, a, st_, kz);
-    else if (krk == 2) hipLaunchKernelGGL((k_visc_div<SV, S, 2>), grid, blk, 0, st, a, st_, kz);
-    else hipLaunchKernelGGL((k_visc_div<SV, S, 3>), grid, blk, 0, st, a, st_, kz);
+    auto go = [&](auto k, auto parts) {
+        hipLaunchKernelGGL((k_visc_div<SV, S, decltype(k)::value, decltype(parts)::value>), grid, blk, 0, st, a, st_, kz);
+    };
+    auto stage = [&](auto parts) {
+        if (krk == 1) go(std::integral_constant<int, 1>{}, parts);
+        else if (krk == 2) go(std::integral_constant<int, 2>{}, parts);
+        else go(std::integral_constant<int, 3>{}, parts);
+    };
+    if (krk == 0) go(std::integral_constant<int, 0>{}, std::integral_constant<int, 1>{});
+    else if (st_.parts == 3) stage(std::integral_constant<int, 3>{});
+    else stage(std::integral_constant<int, 1>{});
 }
 }  // namespace
 template <typename S>

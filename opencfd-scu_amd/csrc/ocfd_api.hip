@@ -70,10 +70,10 @@ struct ocfd_ctx {
     // the plain path; float (the s* pointers) on the mixed path
     bool mixed = false;
     double *d = nullptr, *u = nullptr, *v = nullptr, *w = nullptr, *T = nullptr, *P = nullptr;
-    // dv: the viscous part of du[1..4] on the FP64 path (the mixed path adds
-    // it to du after the sweeps: measured faster there, while on the FP64
-    // path running the divergence beside the sweeps and adding du + dv in
-    // the stage is faster)
+    // du: the inviscid part, or with du_parts = 3 (small grids, sweeps_merged)
+    // 3 x 5 fields, one group written by each sweep; dv: the viscous part of
+    // du[1..4].  The stage adds them.
+    int du_parts = 1;
     double *du = nullptr, *amu = nullptr, *ev = nullptr, *dv = nullptr;
     float *sd = nullptr, *su = nullptr, *sv = nullptr, *sw = nullptr, *sT = nullptr, *sP = nullptr;
     float *sdu = nullptr, *samu = nullptr, *sev = nullptr, *sdv = nullptr;
@@ -500,7 +500,7 @@ ViscArgsT<S> visc_args(ocfd_ctx* x) {
     for (int q = 0; q < 3; q++) va.per[q] = x->cfg.iperiodic[q];
     va.u = V.u; va.v = V.v; va.w = V.w; va.T = V.T; va.amu = V.amu;
     for (int m = 0; m < M_COUNT; m++) va.M[m] = x->M[m];
-    va.ev = V.ev; va.du = V.du; va.dv = V.dv; va.fs = x->fs;
+    va.ev = V.ev; va.dv = V.dv; va.fs = x->fs;
     return va;
 }
 
@@ -540,50 +540,57 @@ int rhs(ocfd_ctx* x, int krk, bool fused = false, bool ghosts = false) {
     // the viscous terms read the primitives and metrics and write only Ev
     // and dv: on the second stream they overlap the sweeps (which write only
     // du).  Kernel timing runs everything in order on one stream.
-    const bool overlap = !x->prof && !x->serial;
+    // Small grids (the merged sweeps) stay on one stream too: there the events
+    // of a fork and a join cost more than the overlap gives (20x16x12: 104 -> 72
+    // us a step, 61x47x39 130 -> 115, 64^3 275 -> 269, 97x61x53 528 either way).
+    const bool overlap = !x->prof && !x->serial && x->du_parts == 1;
     if (overlap) {
         HIPCK(hipEventRecord(x->ev_fork, x->st));
         HIPCK(hipStreamWaitEvent(x->st2, x->ev_fork, 0));
         launch_visc_gf(va, x->st2);
-        if (va.dv && !fused) launch_visc_div(va, x->st2);
+        if (!fused) launch_visc_div(va, x->st2);
         HIPCK(hipGetLastError());
         HIPCK(hipEventRecord(x->ev_join, x->st2));
     }
-    static const char* names[3] = {"sweep_x", "sweep_y", "sweep_z"};
-    const int mk[3][3] = {{M_KX, M_KY, M_KZ}, {M_IX, M_IY, M_IZ}, {M_SX, M_SY, M_SZ}};
+    SweepArgsT<S> a;
+    a.g = x->g;
+    a.c = x->c;
+    a.d = V.d; a.u = V.u; a.v = V.v; a.w = V.w; a.T = V.T;
+    for (int m = 0; m < M_COUNT; m++) a.M[m] = x->M[m];
+    a.du = V.du;
+    a.fs = x->fs;
+    const double h[3] = {x->g.hx, x->g.hy, x->g.hz};
     for (int dir = 0; dir < 3; dir++) {
-        SweepArgsT<S> a;
-        a.g = x->g;
-        a.c = x->c;
-        a.d = V.d; a.u = V.u; a.v = V.v; a.w = V.w; a.T = V.T;
-        a.m1 = x->M[mk[dir][0]]; a.m2 = x->M[mk[dir][1]]; a.m3 = x->M[mk[dir][2]];
-        a.jac = x->M[M_JAC];
-        a.flag = x->flag[dir];
-        a.du = V.du;
-        a.fs = x->fs;
-        a.h = dir == 0 ? x->g.hx : dir == 1 ? x->g.hy : x->g.hz;
-        a.bl = C.dif_bound[2 * dir]; a.br = C.dif_bound[2 * dir + 1];
-        a.nrp = C.non_ref[2 * dir]; a.nrm = C.non_ref[2 * dir + 1];
-        const bool fuse = fuse_learned && dir == 0;
-        for (int m = 0; m < M_COUNT; m++) a.mlp.M[m] = x->M[m];
-        a.mlp.P = fuse ? ma.params : nullptr;
-        a.mlp.lo = ma.lo; a.mlp.hi = ma.hi;
-        a.mlp.fx = ma.fx; a.mlp.fy = ma.fy; a.mlp.fz = ma.fz;
-        a.mlp.prob = ma.prob;
-        int lrc = 0;
-        if (C.charteric)
-            TRY(timed(x, names[dir], [&] { lrc = launch_sweep_char(C.scheme_invis, dir, a, dir == 0, x->st); }));
-        else
-            TRY(timed(x, fuse ? "sweep_x_learned" : names[dir],
-                      [&] { lrc = launch_sweep(C.scheme_invis, dir, a, dir == 0, x->st); }));
-        if (lrc) return fail(OCFD_ERR_UNSUPPORTED, "scheme not supported");
+        a.flag[dir] = x->flag[dir];
+        a.h[dir] = h[dir];
+        a.bl[dir] = C.dif_bound[2 * dir]; a.br[dir] = C.dif_bound[2 * dir + 1];
+        a.nrp[dir] = C.non_ref[2 * dir]; a.nrm[dir] = C.non_ref[2 * dir + 1];
     }
+    a.mlp.P = nullptr;
+    a.mlp.lo = ma.lo; a.mlp.hi = ma.hi;
+    a.mlp.prob = ma.prob;
+    static const char* names[3] = {"sweep_x", "sweep_y", "sweep_z"};
+    int lrc = 0;
+    auto sweep = [&](int dir, const char* name) -> int {
+        a.mlp.P = fuse_learned && dir == 0 ? ma.params : nullptr;
+        return timed(x, a.mlp.P ? "sweep_x_learned" : name, [&] {
+            lrc = C.charteric ? launch_sweep_char(C.scheme_invis, dir, a, x->st) : launch_sweep(C.scheme_invis, dir, a, x->st);
+        });
+    };
+    if (x->du_parts == 3) {
+        // the learned sensor's x sweep writes the flags that y and z read
+        if (fuse_learned) TRY(sweep(0, names[0]));
+        if (!lrc) TRY(sweep(fuse_learned ? SWEEP_YZ : SWEEP_ALL, "sweeps"));
+    } else {
+        for (int dir = 0; dir < 3 && !lrc; dir++) TRY(sweep(dir, names[dir]));
+    }
+    if (lrc) return fail(OCFD_ERR_UNSUPPORTED, "scheme not supported");
     if (overlap) {
         HIPCK(hipStreamWaitEvent(x->st, x->ev_join, 0));
     } else {
         TRY(timed(x, "visc_flux", [&] { launch_visc_gf(va, x->st); }));
+        if (!fused) TRY(timed(x, "visc_div", [&] { launch_visc_div(va, x->st); }));
     }
-    if (!fused && (!overlap || !va.dv)) TRY(timed(x, "visc_div", [&] { launch_visc_div(va, x->st); }));
     x->div_pending = fused;
     return 0;
 }
@@ -660,7 +667,7 @@ StageArgsT<S> stage_args(ocfd_ctx* x, int krk, bool write_flap) {
     const View<S> V = view<S>(x);
     StageArgsT<S> sa;
     sa.g = x->g; sa.c = x->c; sa.krk = krk; sa.dt = x->cfg.dt;
-    sa.f = x->f; sa.fn = x->fn; sa.du = V.du; sa.dv = V.dv; sa.jac = x->M[M_JAC];
+    sa.f = x->f; sa.fn = x->fn; sa.du = V.du; sa.parts = x->du_parts; sa.dv = V.dv; sa.jac = x->M[M_JAC];
     sa.flap = write_flap ? x->flap : nullptr;
     sa.d = V.d; sa.u = V.u; sa.v = V.v; sa.w = V.w; sa.T = V.T; sa.amu = V.amu;
     // the pressure is read only after a step (filter, get_pressure, analysis):
@@ -1076,6 +1083,8 @@ int ocfd_create(const ocfd_config* cfg, int device, ocfd_ctx** out) {
     c.tv_max = 0.2;
 
     x->mixed = C.precision == OCFD_PREC_MIXED;
+    // the characteristic sweeps run one direction at a time
+    x->du_parts = !C.charteric && sweeps_merged(g) ? 3 : 1;
     int rc = 0;
     double* met = alloc_fields(x, M_COUNT, rc);
     double* fa = rc ? nullptr : alloc_fields(x, 5, rc);
@@ -1084,7 +1093,7 @@ int ocfd_create(const ocfd_config* cfg, int device, ocfd_ctx** out) {
     if (!rc && C.nfilter > 0) x->flap = alloc_fields(x, 5, rc);
     if (!x->mixed) {
         double* prim = rc ? nullptr : alloc_fields(x, 6, rc);  // d,u,v,w,T,P
-        double* dua = rc ? nullptr : alloc_fields(x, 5, rc);
+        double* dua = rc ? nullptr : alloc_fields(x, 5 * x->du_parts, rc);
         double* am = rc ? nullptr : alloc_fields(x, 1, rc);
         double* ev = rc ? nullptr : alloc_fields(x, 12, rc);
         double* dva = rc ? nullptr : alloc_fields(x, 4, rc);
@@ -1095,13 +1104,14 @@ int ocfd_create(const ocfd_config* cfg, int device, ocfd_ctx** out) {
         }
     } else {
         float* prim = rc ? nullptr : alloc_fields_f32(x, 6, rc);
-        float* dua = rc ? nullptr : alloc_fields_f32(x, 5, rc);
+        float* dua = rc ? nullptr : alloc_fields_f32(x, 5 * x->du_parts, rc);
         float* am = rc ? nullptr : alloc_fields_f32(x, 1, rc);
         float* ev = rc ? nullptr : alloc_fields_f32(x, 12, rc);
+        float* dva = rc ? nullptr : alloc_fields_f32(x, 4, rc);
         if (!rc) {
             x->sd = prim; x->su = prim + x->fs; x->sv = prim + 2 * x->fs; x->sw = prim + 3 * x->fs;
             x->sT = prim + 4 * x->fs; x->sP = prim + 5 * x->fs;
-            x->sdu = dua; x->samu = am; x->sev = ev;
+            x->sdu = dua; x->samu = am; x->sev = ev; x->sdv = dva;
         }
     }
     for (int dd = 0; dd < 3 && !rc; dd++) x->flag[dd] = alloc_bytes(x, (size_t)x->fs, rc);
@@ -1399,16 +1409,21 @@ int ocfd_get_du(ocfd_ctx* x, double* du5) {
     if (!x || !du5) return fail(OCFD_ERR_ARG, "null argument");
     TRY(finish_rhs(x));
     const size_t n = (size_t)x->g.nx * x->g.ny * x->g.nz;
-    for (int m = 0; m < 5; m++)
-        TRY(x->mixed ? download_any(x, (const float*)x->sdu + m * x->fs, du5 + m * n)
-                     : download_any(x, (const double*)x->du + m * x->fs, du5 + m * n));
-    // the viscous part of components 1..4 when it is kept apart, added as
-    // the RK stage adds it, then the Jacobian factor the stage applies
+    // the parts of x, y and z and the viscous part of components 1..4, added as
+    // the RK stage adds them, then the Jacobian factor it applies
     std::vector<double> tmp(n);
-    if (!x->mixed) {
-        for (int m = 1; m < 5; m++) {
-            TRY(download_any(x, (const double*)x->dv + (m - 1) * x->fs, tmp.data()));
-            for (size_t p = 0; p < n; p++) du5[m * n + p] += tmp[p];
+    auto get = [&](int part, int m, double* out) {
+        const long long o = (part < 3 ? 5 * part + m : m - 1) * x->fs;
+        return x->mixed ? download_any(x, (const float*)((part < 3 ? x->sdu : x->sdv) + o), out)
+                        : download_any(x, (const double*)((part < 3 ? x->du : x->dv) + o), out);
+    };
+    for (int m = 0; m < 5; m++) {
+        double* d = du5 + m * n;
+        TRY(get(0, m, d));
+        for (int part = 1; part < (m ? 4 : 3); part++) {
+            if (part < 3 && part >= x->du_parts) continue;
+            TRY(get(part, m, tmp.data()));
+            for (size_t p = 0; p < n; p++) d[p] += tmp[p];
         }
     }
     TRY(download_any(x, (const double*)x->M[M_JAC], tmp.data()));
@@ -1851,7 +1866,7 @@ int ocfd_get_q(ocfd_ctx* x, double* q) {
         for (int m = 0; m < 6; m++) va.bnd[m] = C.dif_bound[m];
         va.u = x->su; va.v = x->sv; va.w = x->sw; va.T = x->sT; va.amu = x->samu;
         for (int m = 0; m < M_COUNT; m++) va.M[m] = x->M[m];
-        va.ev = x->sev; va.du = x->sdu; va.dv = x->sdv; va.fs = x->fs;
+        va.ev = x->sev; va.dv = x->sdv; va.fs = x->fs;
         TRY(timed(x, "qcrit", [&] { launch_qcrit(va, out, x->st); }));
     } else {
         ViscArgsT<double> va;
@@ -1859,7 +1874,7 @@ int ocfd_get_q(ocfd_ctx* x, double* q) {
         for (int m = 0; m < 6; m++) va.bnd[m] = C.dif_bound[m];
         va.u = x->u; va.v = x->v; va.w = x->w; va.T = x->T; va.amu = x->amu;
         for (int m = 0; m < M_COUNT; m++) va.M[m] = x->M[m];
-        va.ev = x->ev; va.du = x->du; va.dv = x->dv; va.fs = x->fs;
+        va.ev = x->ev; va.dv = x->dv; va.fs = x->fs;
         TRY(timed(x, "qcrit", [&] { launch_qcrit(va, out, x->st); }));
     }
     return download_any(x, (const double*)out, q);

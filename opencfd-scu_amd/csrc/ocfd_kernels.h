@@ -9,39 +9,41 @@
 #include "ocfd_dev.h"
 #include "../../include/ocfd.h"
 
-// Inviscid sweep along one direction.
+// Inviscid sweeps.  Arrays of three: x, y, z.
 template <typename S>
 struct SweepArgsT {
     Geo g;
     Consts c;
     const S *d, *u, *v, *w, *T;          // primitives (LAP layout)
-    const double *m1, *m2, *m3;          // the direction's cofactors
-    const double *jac;                   // Ajac
-    const int8_t *flag;                  // hybrid flags of this direction (face j+1/2 at node j) or null
-    S *du;                               // 5 fields, stride fs
+    const double *M[M_COUNT];            // cofactors: M[3 dir .. 3 dir + 2] of a direction
+    int8_t *flag[3];                     // hybrid flags (face j+1/2 at node j) or null
+    S *du;                               // 5 fields, stride fs; or 3 x 5, one group per direction
     long long fs;
-    double h;                            // hx / hy / hz
-    int bl, br;                          // DIF_BOUND on the low / high face
-    int nrp, nrm;                        // NON_REFLETION for the P / M flux
+    double h[3];                         // hx, hy, hz
+    int bl[3], br[3];                    // DIF_BOUND on the low / high face
+    int nrp[3], nrm[3];                  // NON_REFLETION for the P / M flux
     // The learned hybrid sensor, run by the x sweep of the first RK stage
     // (hybrid_auto only): when P is set the x sweep computes the flags of its
-    // rows' nodes (i >= -1) itself, writes them to fx, fy, fz and the
-    // probabilities to prob, and uses them for its own faces.
+    // rows' nodes (i >= -1) itself, writes them to flag and the probabilities
+    // to prob, and uses them for its own faces (the y and z sweeps follow it).
     struct {
-        const double* M[M_COUNT];        // cofactors and Ajac (the features' contravariant velocities)
         const float* P;                  // packed network weights (launch_mlp_pack), or null
         float lo, hi;                    // confidence band that falls back to the plain sensor
-        int8_t *fx, *fy, *fz;
         float* prob;
     } mlp;
 };
+// The sweep along dir, in the order x, y, z (x writes du, y and z add to it), or
+// all three (SWEEP_ALL), or y and z after x (SWEEP_YZ), in one launch, each
+// direction into its own group of du.
+enum { SWEEP_ALL = -1, SWEEP_YZ = -2 };
 template <typename S>
-int launch_sweep(int scheme, int dir, const SweepArgsT<S>& a, bool first, hipStream_t st);
-// The same sweep with the reconstruction in characteristic space
-// (CHARTERIC = 1): WENO7_SYMBO, WENO7_SYMBO_LIM and SCHEME_HYBRIDAUTO only
-// (returns -1 for the other schemes, which the reference cannot run so).
+int launch_sweep(int scheme, int dir, const SweepArgsT<S>& a, hipStream_t st);
+// The same with the reconstruction in characteristic space (CHARTERIC = 1;
+// WENO7_SYMBO, WENO7_SYMBO_LIM, hybrid_auto): one direction at a time.
 template <typename S>
-int launch_sweep_char(int scheme, int dir, const SweepArgsT<S>& a, bool first, hipStream_t st);
+int launch_sweep_char(int scheme, int dir, const SweepArgsT<S>& a, hipStream_t st);
+// Whether a grid takes the form with a group of du per direction.
+bool sweeps_merged(const Geo& g);
 
 // Viscous terms.
 template <typename S>
@@ -54,14 +56,12 @@ struct ViscArgsT {
     const S *u, *v, *w, *T, *amu;
     const double *M[M_COUNT];
     S *ev;                                   // 12 fields: Ev1..4 for x, y, z
-    S *du;                                   // 5 fields
-    S *dv;                                   // 4 fields: the viscous part of du[1..4], or null (added to du)
+    S *dv;                                   // 4 fields: the viscous part of du[1..4]
     long long fs;
 };
 // Gradients of u,v,w,T (kept in registers) and the 12 viscous fluxes.
 template <typename S> void launch_visc_gf(const ViscArgsT<S>& a, hipStream_t st);
-// The divergence of the fluxes: written to dv when it is set (so that it may
-// run beside the inviscid sweeps), else added to du after the sweeps.
+// The divergence of the fluxes into dv.
 template <typename S> void launch_visc_div(const ViscArgsT<S>& a, hipStream_t st);
 // Q criterion of u, v, w at every interior point into q (LAP layout, FP64).
 template <typename S> void launch_qcrit(const ViscArgsT<S>& a, double* q, hipStream_t st);
@@ -82,8 +82,9 @@ struct StageArgsT {
     double dt;
     double *f;
     const double *fn;
-    const S *du;                             // right-hand side without the Jacobian factor
-    const S *dv;                             // 4 fields, the viscous part of du[1..4], or null
+    const S *du;                             // inviscid part, without the Jacobian factor: 5 fields, or
+    int parts;                               // 3 x 5 to be added (parts = 3)
+    const S *dv;                             // 4 fields, the viscous part of du[1..4] (launch_stage)
     const double *jac;                       // Ajac: the stage advances with Ajac * (du + dv)
     double *flap;                            // 5 fields or null (written in stage 3 when non-null)
     S *d, *u, *v, *w, *T;
@@ -96,8 +97,8 @@ struct StageArgsT {
     int ghost[3];
 };
 template <typename S> void launch_stage(const StageArgsT<S>& a, hipStream_t st);
-// The divergence of the viscous fluxes and the RK stage in one pass (a.du
-// holds the inviscid part; the viscous part never goes to memory).  On the
+// The divergence of the viscous fluxes and the RK stage in one pass (the
+// viscous part of du never goes to memory).  On the
 // FP64 path f is written in stage 3 only: stages 2 and 3 form it from the
 // primitives.
 template <typename S>
