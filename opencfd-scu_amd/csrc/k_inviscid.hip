@@ -29,68 +29,77 @@
 
 namespace {
 
-// Square root for the sound speed: correctly rounded in FP64; on the FP32
-// path (whose sweeps are VALU-bound) the hardware square root, 1 ulp, inside
-// the FP32 rounding the mixed path already carries (measured on the
-// 1024x384x256 swept ramp: y and z sweeps 2.5 % faster).
-template <typename R>
-__device__ __forceinline__ R sqrt_s(R x) {
-    if constexpr (std::is_same<R, float>::value) return __builtin_amdgcn_sqrtf(x);
-    else return sqrt(x);
+// sqrt(x) and 1/sqrt(x) together.  FP64: two coupled Newton steps from the
+// hardware's estimate (5e-8) and a last correction of each: 15 instructions,
+// where a square root and a division of their own, with the scaling that only
+// subnormal and huge arguments need, take 30.  Largest errors over 2e6
+// arguments of e^-40..e^40: root 1.1e-16, reciprocal 1.7e-16, as before.  x = 0 gives NaN in both (ROOT0: the root is 0).  FP32: the
+// hardware's 1-ulp instructions.
+template <bool ROOT0, typename R>
+__device__ __forceinline__ void sqrt_pair(R x, R& root, R& inv) {
+    if constexpr (std::is_same<R, float>::value) {
+        if constexpr (ROOT0) {
+            root = __builtin_amdgcn_sqrtf(x);
+        } else {
+            inv = __builtin_amdgcn_rsqf(x);
+            root = x * inv;
+        }
+    } else {
+        double y = __builtin_amdgcn_rsq(x);
+        if (ROOT0) y = x == 0.0 ? 0.0 : y;
+        double g = x * y, h = 0.5 * y;
+        double e = fma(-h, g, 0.5);
+        g = fma(g, e, g);
+        h = fma(h, e, h);
+        e = fma(-h, g, 0.5);
+        g = fma(g, e, g);
+        h = fma(h, e, h);
+        root = fma(fma(-g, g, x), h, g);
+        inv = h + h;
+        inv = fma(fma(-root, inv, 1.0), inv, inv);
+    }
 }
 
-// Steger-Warming split of one node (src/OCFD_split.cu:92-142).  FP32: |A|
-// and 1/|A| from the hardware reciprocal square root (1 ulp) instead of a
-// correctly rounded square root and division.
+// Steger-Warming split of one node (src/OCFD_split.cu:92-142).  With n = A/|A|,
+// t = l2 + l3 and D = c (l3 - l2), the reference's sums over the three waves
+// are
+//   f0 = C1 l1 + t,  f_i = u_i f0 + n_i D,
+//   f4 = l1 (gamma-1)|u|^2 + t (|u|^2/2 + c^2/2 + W c^2) + (u.n) D
+// (its |u -+ c n|^2 written out with |n| = 1): 85 instructions a node against
+// 165, its error against 80-bit arithmetic the same or smaller in every
+// component (rms over Mach 0.1-8: FP64 0.93-1.00, FP32 0.84-1.00 of the sums'),
+// and the y sweep of 256x128x128 WENO7 204 -> 194 us, of 1024x256x128 1068 ->
+// 1041.  l = (E +- |E|)/2 with the factor rho/(2 gamma) in it.
 template <typename R>
 __device__ __forceinline__ void sw_split(R tmp0d, R u, R v, R w, R cc, R A1, R A2, R A3, const Consts& c,
                                          R* fp, R* fm) {
-    const R s2 = A1 * A1 + A2 * A2 + A3 * A3;
     R ss, rs;
-    if constexpr (std::is_same<R, float>::value) {
-        rs = __builtin_amdgcn_rsqf(s2);
-        ss = s2 * rs;
-    } else {
-        ss = sqrt(s2);
-        rs = R(1.0) / ss;
-    }
-    R E1 = A1 * u + A2 * v + A3 * w;
-    R E2 = E1 - cc * ss;
-    R E3 = E1 + cc * ss;
-    ss = rs;
-    A1 *= ss; A2 *= ss; A3 *= ss;
+    sqrt_pair<false>(A1 * A1 + A2 * A2 + A3 * A3, ss, rs);
+    const R E1 = A1 * u + A2 * v + A3 * w;
+    const R E2 = E1 - cc * ss, E3 = E1 + cc * ss;
     const R eps = R(c.epsl_sw);
-    R E1P, E2P, E3P;
+    R a1, a2, a3;
     if (eps == R(0)) {
         // sqrt(x*x) == |x| in binary floating point with round-to-nearest
         // (no underflow of x*x): the same values without three square roots
-        E1P = (E1 + fabs(E1)) * R(0.50);
-        E2P = (E2 + fabs(E2)) * R(0.50);
-        E3P = (E3 + fabs(E3)) * R(0.50);
+        a1 = fabs(E1); a2 = fabs(E2); a3 = fabs(E3);
     } else {
-        E1P = (E1 + sqrt(E1 * E1 + eps * eps)) * R(0.50);
-        E2P = (E2 + sqrt(E2 * E2 + eps * eps)) * R(0.50);
-        E3P = (E3 + sqrt(E3 * E3 + eps * eps)) * R(0.50);
+        a1 = sqrt(E1 * E1 + eps * eps); a2 = sqrt(E2 * E2 + eps * eps); a3 = sqrt(E3 * E3 + eps * eps);
     }
-    R E1M = E1 - E1P, E2M = E2 - E2P, E3M = E3 - E3P;
-    R uc1 = u - cc * A1, uc2 = u + cc * A1;
-    R vc1 = v - cc * A2, vc2 = v + cc * A2;
-    R wc1 = w - cc * A3, wc2 = w + cc * A3;
-    R vvc1 = (uc1 * uc1 + vc1 * vc1 + wc1 * wc1) * R(0.50);
-    R vvc2 = (uc2 * uc2 + vc2 * vc2 + wc2 * wc2) * R(0.50);
-    R vv = (R(c.gamma) - R(1.0)) * (u * u + v * v + w * w);
-    R W2 = R(c.split_c3) * cc * cc;
-    const R C1 = R(c.split_c1);
-    fp[0] = tmp0d * (C1 * E1P + E2P + E3P);
-    fp[1] = tmp0d * (C1 * E1P * u + E2P * uc1 + E3P * uc2);
-    fp[2] = tmp0d * (C1 * E1P * v + E2P * vc1 + E3P * vc2);
-    fp[3] = tmp0d * (C1 * E1P * w + E2P * wc1 + E3P * wc2);
-    fp[4] = tmp0d * (E1P * vv + E2P * vvc1 + E3P * vvc2 + W2 * (E2P + E3P));
-    fm[0] = tmp0d * (C1 * E1M + E2M + E3M);
-    fm[1] = tmp0d * (C1 * E1M * u + E2M * uc1 + E3M * uc2);
-    fm[2] = tmp0d * (C1 * E1M * v + E2M * vc1 + E3M * vc2);
-    fm[3] = tmp0d * (C1 * E1M * w + E2M * wc1 + E3M * wc2);
-    fm[4] = tmp0d * (E1M * vv + E2M * vvc1 + E3M * vvc2 + W2 * (E2M + E3M));
+    const R k2 = u * u + v * v + w * w, c2 = cc * cc, ccr = cc * rs;
+    const R vv = (R(c.gamma) - R(1.0)) * k2;
+    const R K = fma(R(c.split_c3), c2, R(0.50) * (k2 + c2));
+    const R C1 = R(c.split_c1), q = R(0.50) * tmp0d;
+    auto side = [&](R l1, R l2, R l3, R* f) {
+        const R t = l2 + l3, D = (l3 - l2) * ccr;
+        f[0] = fma(C1, l1, t);
+        f[1] = fma(u, f[0], A1 * D);
+        f[2] = fma(v, f[0], A2 * D);
+        f[3] = fma(w, f[0], A3 * D);
+        f[4] = fma(t, K, fma(E1, D, l1 * vv));
+    };
+    side((E1 + a1) * q, (E2 + a2) * q, (E3 + a3) * q, fp);
+    side((E1 - a1) * q, (E2 - a2) * q, (E3 - a3) * q, fm);
 }
 
 // f+ and f- of node (i, j, k) along direction DIR.
@@ -98,7 +107,9 @@ template <int DIR, typename S>
 __device__ __forceinline__ void split_node(const SweepArgsT<S>& A, int i, int j, int k, S* fp, S* fm) {
     const long long q = gidx(A.g, i, j, k);
     const S d = A.d[q], u = A.u[q], v = A.v[q], w = A.w[q], T = A.T[q];
-    const S cc = sqrt_s(T) * S(A.c.rama);  // sound_speed_kernel, src/commen_kernel.cu:144-153
+    S root, inv;
+    sqrt_pair<true>(T, root, inv);
+    const S cc = root * S(A.c.rama);  // sound_speed_kernel, src/commen_kernel.cu:144-153
     sw_split<S>(d * S(A.c.tmp0), u, v, w, cc, S(A.M[3 * DIR][q]), S(A.M[3 * DIR + 1][q]), S(A.M[3 * DIR + 2][q]), A.c,
                 fp, fm);
 }
@@ -848,7 +859,9 @@ __global__ void __launch_bounds__(256, SCH == OCFD_HYBRIDAUTO ? 3 : 2) k_char(Sw
 // 1024x256x128: 2.96 -> 2.92 ms and 2.02 -> 2.60).  Blocks in the order x, y, z;
 // cutting the domain into boxes whose x, y and z blocks follow one another, for
 // the Infinity Cache, was slower at every size (64^3 51-59 us, 256x128x128
-// 720-860).
+// 720-860).  The SYMBO schemes are held to 4 waves per SIMD (128 VGPRs, 2
+// spilled) where they would take 3: 97x61x53, 91 -> 84 us; k_sweep_yz, which
+// would spill 18, is not (256x128x128: 249 us, held 299).
 // ---------------------------------------------------------------------------
 struct SweepGrid {
     int nt[3][3];  // tiles of a direction along x, y, z
@@ -866,7 +879,7 @@ __device__ __forceinline__ bool run_tile(unsigned b, int run, const int* nt, Blk
 }
 constexpr int XWAVES = 4;  // waves of an x block here
 template <int SCH, int XR, typename S>
-__global__ void __launch_bounds__(256) k_sweeps(SweepArgsT<S> A, SweepGrid G) {
+__global__ void __launch_bounds__(256, SCH == OCFD_WENO7_SYMBO || SCH == OCFD_WENO7_SYMBO_LIM ? 4 : 1) k_sweeps(SweepArgsT<S> A, SweepGrid G) {
     constexpr int NS = YZ<S>::NS, NA = YZ<S>::NA;
     constexpr int LDS_YZ = 10 * (NS + 8) * NA, LDS_X = 640 * XWAVES;
     __shared__ S sh[LDS_YZ > LDS_X ? LDS_YZ : LDS_X];

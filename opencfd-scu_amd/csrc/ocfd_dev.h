@@ -178,16 +178,14 @@ template <typename R, typename W = R> __device__ __forceinline__ R weno7_dn(cons
     return weno7_up<R, W>(m);
 }
 
-// UP7 (src/OCFD_Schemes.cu:865-931).  The division by 420 is a multiplication
-// by its reciprocal (an ulp-level difference; a division costs ten FP64
-// instructions, the whole reconstruction eight).
+// UP7 (src/OCFD_Schemes.cu:865-931), its coefficients already divided by 420.
 template <typename R> __device__ __forceinline__ R up7_up(const R* s) {
-    return (R(-3) * s[0] + R(25) * s[1] - R(101) * s[2] + R(319) * s[3] + R(214) * s[4] - R(38) * s[5] +
-            R(4) * s[6]) * R(1.0 / 420.0);
+    return R(-3.0 / 420.0) * s[0] + R(25.0 / 420.0) * s[1] + R(-101.0 / 420.0) * s[2] + R(319.0 / 420.0) * s[3] +
+           R(214.0 / 420.0) * s[4] + R(-38.0 / 420.0) * s[5] + R(4.0 / 420.0) * s[6];
 }
 template <typename R> __device__ __forceinline__ R up7_dn(const R* s) {  // s[1..7]
-    return (R(-3) * s[7] + R(25) * s[6] - R(101) * s[5] + R(319) * s[4] + R(214) * s[3] - R(38) * s[2] +
-            R(4) * s[1]) * R(1.0 / 420.0);
+    return R(-3.0 / 420.0) * s[7] + R(25.0 / 420.0) * s[6] + R(-101.0 / 420.0) * s[5] + R(319.0 / 420.0) * s[4] +
+           R(214.0 / 420.0) * s[3] + R(-38.0 / 420.0) * s[2] + R(4.0 / 420.0) * s[1];
 }
 
 // WENO5 Jiang-Shu (src/OCFD_Schemes.cu:1118-1210) and the one-sided subsets
