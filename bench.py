@@ -37,6 +37,7 @@ ALGO_BYTES = {
     "sweep_x": (5 + 3 + 5) * 8,           # rho,u,v,w,T + 3 cofactors; write du(5) (Ajac applied by the stage)
     "sweep_y": (5 + 3 + 5 + 5) * 8,       # same + read-modify-write du(5)
     "sweep_z": (5 + 3 + 5 + 5) * 8,
+    "sweep_xy": (5 + 6 + 5) * 8,          # x and y in one launch: 6 cofactors, du written once
     "visc_flux": (4 + 10 + 12) * 8,       # u,v,w,T, 9 cofactors + Ajac; write 12 Ev (mu formed from T)
     # divergence and RK stage: 12 Ev, du, Ajac, fn; write 5 primitives; the
     # primitives in stages 2-3; f and p written in stage 3 (mean of the stages)

@@ -114,24 +114,30 @@ __device__ __forceinline__ void split_node(const SweepArgsT<S>& A, int i, int j,
                 fp, fm);
 }
 
-// The direction's part of du at node i along it (linear index q): P then M, in
-// the reference's order, the sum in double.  face(v, 0 / 1): value v (P of
-// variable v < 5, M of v - 5) at the node's left / right face.  PARTS: into the
-// direction's own group of du, else into the one du.  ACC: added to pre, what
-// du holds there; else written, streamed (nothing reads it before the next
-// sweep or the RK stage).
-template <int DIR, bool PARTS, bool ACC, typename S, typename F>
-__device__ __forceinline__ void put_du(const SweepArgsT<S>& A, int i, long long q, const double* pre, F&& face) {
+// The direction's part of du's variable m at node i along it, added to pre if
+// ACC: P then M, in the reference's order, the sum in double.  face(v, 0 / 1):
+// value v (P of variable v < 5, M of v - 5) at the node's left / right face.
+template <int DIR, bool ACC, typename S, typename F>
+__device__ __forceinline__ S du_of(const SweepArgsT<S>& A, int i, int m, double pre, F&& face) {
     const int n_dir = DIR == 0 ? A.g.nx : DIR == 1 ? A.g.ny : A.g.nz;
     const bool zp = A.nrp[DIR] && i == 0, zm = A.nrm[DIR] && i == n_dir - 1;
     const double rh = 1.0 / A.h[DIR];
+    const double dP = zp ? 0.0 : double(face(m, 1) - face(m, 0));
+    const double dM = zm ? 0.0 : double(face(5 + m, 1) - face(5 + m, 0));
+    return S(fma(-dM, rh, ACC ? fma(-dP, rh, pre) : -dP * rh));
+}
+// du_of for the five variables of a node (linear index q).  PARTS: into the
+// direction's own group of du, else into the one du.  ACC: added to pre, the
+// earlier directions' part; else written, streamed (nothing reads it before the
+// next sweep or the RK stage).
+template <int DIR, bool PARTS, bool ACC, typename S, typename F>
+__device__ __forceinline__ void put_du(const SweepArgsT<S>& A, int i, long long q, const double* pre, F&& face) {
 #pragma unroll
     for (int m = 0; m < 5; m++) {
-        const double dP = zp ? 0.0 : double(face(m, 1) - face(m, 0));
-        const double dM = zm ? 0.0 : double(face(5 + m, 1) - face(5 + m, 0));
         S* o = &A.du[((PARTS ? 5 * DIR : 0) + m) * A.fs + q];
-        if constexpr (ACC) *o = S(fma(-dM, rh, fma(-dP, rh, pre[m])));
-        else __builtin_nontemporal_store(S(fma(-dM, rh, -dP * rh)), o);
+        const S r = du_of<DIR, ACC>(A, i, m, ACC ? pre[m] : 0.0, face);
+        if constexpr (ACC) *o = r;
+        else __builtin_nontemporal_store(r, o);
     }
 }
 // P and M half-node values of all five variables at face j+1/2 (c = j+1, r =
@@ -318,8 +324,8 @@ __device__ __forceinline__ R recon_m_hybrid(int mc, const R* g) {
 // special faces per wave in one pass; a wave with more takes the per-face
 // path.  Same formulas, so the same values.  Used in the x sweep, which is
 // VALU-bound (91 % VALU busy on the 1024x384x256 swept ramp; 2.40 -> 2.23 ms
-// per launch); the y and z tiles, at 48-60 % VALU busy, measured the same or
-// 2 % slower with it and keep the per-face path.
+// per launch); the tiles, at 48-60 % VALU busy, measured the same or 2 %
+// slower with it and keep the per-face path.
 constexpr int COMPACT_MAX = 6;  // special faces per wave spread in one pass (10 values each)
 // The lane of the n-th special face of the wave (n-th set bit of mask).
 __device__ __forceinline__ int nth_lane(unsigned long long mask, int n) {
@@ -487,105 +493,116 @@ __device__ __forceinline__ void sweep_x(const SweepArgsT<S>& A, int bx, int by, 
         put_du<0, PARTS, false>(A, i, gidx(g, i, j, k2), nullptr, [&](int v, int right) { return w[64 * v + lane + right]; });
 }
 
-// y and z sweeps: a block owns NA x-consecutive columns (one NA*8-byte row
-// segment per node) and NS output nodes along the sweep, for one value of the
-// third index.  The same three phases; a thread may handle up to two faces and
-// two nodes.
-template <int DIR, int SCH, int NS, int NA, bool ACC, typename S>
-__device__ __forceinline__ void sweep_yz(const SweepArgsT<S>& A, int bx, int by, int bz, S* sh) {
-    static_assert(DIR == 1 || DIR == 2, "x is swept by sweep_x");
-    constexpr int NN = NS + 8, NF = NS + 1;
-    constexpr int FPT = (NF * NA + 255) / 256, NPT = (NS * NA + 255) / 256;
-    static_assert(FPT <= 2 && NN * NA >= NF * NA, "at most two faces per thread");
+// Half-node values of one direction over a tile of TX x TR nodes in x and R (1:
+// y, 2: z), at index k2 of the third direction: the flux split of the tile and
+// its halo along DIR (0 or R) into LDS, then the faces' P and M values over
+// them, value v of face f of line a at sh[tile_at(v, f, a, TX|TR + 1)].  Lines
+// of x keep their nodes together, lines of R their x neighbours: both as memory
+// has them.
+template <bool ALONG, int NA> __device__ __forceinline__ int tile_at(int v, int n, int a, int len) {
+    return ALONG ? (v * NA + a) * len + n : (v * len + n) * NA + a;
+}
+template <int DIR, int R, int SCH, int TX, int TR, typename S>
+__device__ __forceinline__ void tile_faces(const SweepArgsT<S>& A, int x0, int r0, int k2, S* sh) {
+    constexpr bool ALONG = DIR == 0;
+    static_assert((R == 1 || R == 2) && (DIR == 0 || DIR == R), "x or R");
+    constexpr int NS = ALONG ? TX : TR, NA = ALONG ? TR : TX, NN = NS + 8, NF = NS + 1;
+    static_assert(NF * NA <= 256, "a face per thread");
     const Geo& g = A.g;
     const int tid = threadIdx.x;
-    const int a0 = bx * NA, s0 = by * NS, k2 = bz;
-    const int n_dir = DIR == 1 ? g.ny : g.nz;
-    auto lin = [&](int s, int a) -> long long { return DIR == 1 ? gidx(g, a, s, k2) : gidx(g, a, k2, s); };
-    auto at = [](int v, int n, int a) { return (v * NN + n) * NA + a; };
+    const int a0 = ALONG ? r0 : x0, s0 = ALONG ? x0 : r0;
+    const int n_dir = DIR == 0 ? g.nx : DIR == 1 ? g.ny : g.nz, n_a = !ALONG ? g.nx : R == 1 ? g.ny : g.nz;
+    // (x, y, z) of position s of line a
+    auto ix = [&](int s, int a) { return ALONG ? s : a; };
+    auto iy = [&](int s, int a) { return R == 1 ? (ALONG ? a : s) : k2; };
+    auto iz = [&](int s, int a) { return R == 2 ? (ALONG ? a : s) : k2; };
+    // item idx of a tile of lines of len: its position and line
+    auto pos = [](int idx, int len) { return ALONG ? idx % len : idx / NA; };
+    auto line = [](int idx, int len) { return ALONG ? idx / len : idx % NA; };
 
-    // the du of this thread's output nodes and the hybrid flags of its faces are
-    // fetched first, so that their latency hides behind phases 1 and 2
-    double pre_du[NPT][5];
-    if constexpr (ACC) {
-#pragma unroll
-        for (int t = 0; t < NPT; t++) {
-            const int idx = tid + 256 * t;
-            const int i = s0 + idx / NA, ac = a0 + idx % NA;
-            if (idx < NS * NA && i < n_dir && ac < g.nx) {
-                const long long q = lin(i, ac);
-#pragma unroll
-                for (int m = 0; m < 5; m++) pre_du[t][m] = double(A.du[m * A.fs + q]);
-            }
-        }
-    }
-    int pre_hy[FPT];
-#pragma unroll
-    for (int t = 0; t < FPT; t++) {
-        pre_hy[t] = 0;
-        const int idx = tid + 256 * t;
-        const int j = s0 - 1 + idx / NA, ac = a0 + idx % NA;
-        if (SCH == OCFD_HYBRIDAUTO && idx < NF * NA && j <= n_dir - 1 && ac < g.nx) pre_hy[t] = A.flag[DIR][lin(j, ac)];
-    }
+    // this thread's face, j+1/2 of line a0 + al; its hybrid flag is fetched
+    // first, so that its latency hides behind phase 1
+    const int al = line(tid, NF), fl = pos(tid, NF), j = s0 - 1 + fl;
+    const bool valid = tid < NF * NA && j <= n_dir - 1 && a0 + al < n_a;
+    int hy = 0;
+    if (SCH == OCFD_HYBRIDAUTO && valid) hy = A.flag[DIR][gidx(g, ix(j, a0 + al), iy(j, a0 + al), iz(j, a0 + al))];
 
     // ---- phase 1: split of NN x NA nodes into LDS
     for (int idx = tid; idx < NN * NA; idx += 256) {
-        const int a = idx % NA, n = idx / NA;
+        const int a = line(idx, NN), n = pos(idx, NN);
         const int s = s0 - 4 + n, ac = a0 + a;
         S fp[5], fm[5];
-        if (s <= n_dir + 3 && ac < g.nx) {
-            split_node<DIR>(A, ac, DIR == 1 ? s : k2, DIR == 1 ? k2 : s, fp, fm);
+        if (s <= n_dir + 3 && ac < n_a) {
+            split_node<DIR>(A, ix(s, ac), iy(s, ac), iz(s, ac), fp, fm);
         } else {
 #pragma unroll
             for (int m = 0; m < 5; m++) { fp[m] = S(0); fm[m] = S(0); }
         }
 #pragma unroll
         for (int m = 0; m < 5; m++) {
-            sh[at(m, n, a)] = fp[m];
-            sh[at(5 + m, n, a)] = fm[m];
+            sh[tile_at<ALONG, NA>(m, n, a, NN)] = fp[m];
+            sh[tile_at<ALONG, NA>(5 + m, n, a, NN)] = fm[m];
         }
     }
     __syncthreads();
 
-    // ---- phase 2: half nodes
-    S hp[FPT][5], hm[FPT][5];
+    // ---- phase 2: the thread's face
+    S hp[5], hm[5];
 #pragma unroll
-    for (int t = 0; t < FPT; t++) {
-        const int idx = tid + 256 * t;
-        if (idx >= NF * NA) break;
-        const int a_loc = idx % NA, f_loc = idx / NA;
-        const int j = s0 - 1 + f_loc;  // face j+1/2
-        const int ac = a0 + a_loc;
-        if (j <= n_dir - 1 && ac < g.nx) {
-            face_all<S, double, SCH>([&](int v, int k) { return sh[at(v, f_loc + k, a_loc)]; }, j + 1, j - n_dir,
-                                     A.bl[DIR], A.br[DIR], pre_hy[t], S(A.c.tv_lim), S(A.c.tv_max), hp[t], hm[t]);
-        } else {
+    for (int m = 0; m < 5; m++) { hp[m] = S(0); hm[m] = S(0); }
+    if (valid)
+        face_all<S, double, SCH>([&](int v, int k) { return sh[tile_at<ALONG, NA>(v, fl + k, al, NN)]; }, j + 1, j - n_dir,
+                                 A.bl[DIR], A.br[DIR], hy, S(A.c.tv_lim), S(A.c.tv_max), hp, hm);
+    __syncthreads();
+    if (tid < NF * NA) {
 #pragma unroll
-            for (int m = 0; m < 5; m++) { hp[t][m] = S(0); hm[t][m] = S(0); }
+        for (int m = 0; m < 5; m++) {  // tile_at of the face
+            sh[m * NF * NA + tid] = hp[m];
+            sh[(5 + m) * NF * NA + tid] = hm[m];
         }
     }
     __syncthreads();
-#pragma unroll
-    for (int t = 0; t < FPT; t++) {
-        const int idx = tid + 256 * t;
-        if (idx >= NF * NA) break;
-#pragma unroll
-        for (int m = 0; m < 5; m++) {
-            sh[m * NF * NA + idx] = hp[t][m];
-            sh[(5 + m) * NF * NA + idx] = hm[t][m];
-        }
-    }
-    __syncthreads();
-
-    // ---- phase 3: du at nodes
-#pragma unroll
-    for (int t = 0; t < NPT; t++) {
-        const int idx = tid + 256 * t;
-        const int i = s0 + idx / NA, ac = a0 + idx % NA;
-        if (idx < NS * NA && i < n_dir && ac < g.nx)
-            put_du<DIR, !ACC, ACC>(A, i, lin(i, ac), pre_du[t], [&](int v, int right) { return sh[v * NF * NA + idx + right * NA]; });
-    }
 }
+
+// Sweep along R of a tile, and before it (XTOO) along x, whose part of du stays
+// in registers: idx = x + TX r is a thread's output node in both.  ACC: added
+// to du.
+template <int R, int SCH, int TX, int TR, bool XTOO, bool ACC, bool PARTS, typename S>
+__device__ __forceinline__ void sweep_tile(const SweepArgsT<S>& A, int bx, int by, int bz, S* sh) {
+    constexpr int NPT = (TX * TR + 255) / 256;
+    const Geo& g = A.g;
+    const int x0 = bx * TX, r0 = by * TR, n_r = R == 1 ? g.ny : g.nz;
+    double part[NPT][5];
+    auto nodes = [&](auto&& f) {
+#pragma unroll
+        for (int t = 0; t < NPT; t++) {
+            const int idx = threadIdx.x + 256 * t;
+            const int i = x0 + idx % TX, r = r0 + idx / TX;
+            if (idx < TX * TR && i < g.nx && r < n_r) f(t, idx, i, r, R == 1 ? gidx(g, i, r, bz) : gidx(g, i, bz, r));
+        }
+    };
+    if constexpr (XTOO) {
+        tile_faces<0, R, SCH, TX, TR>(A, x0, r0, bz, sh);
+        nodes([&](int t, int idx, int i, int, long long) {
+            auto face = [&](int v, int right) { return sh[tile_at<true, TR>(v, idx % TX + right, idx / TX, TX + 1)]; };
+#pragma unroll
+            for (int m = 0; m < 5; m++) part[t][m] = double(du_of<0, false>(A, i, m, 0.0, face));
+        });
+        __syncthreads();
+    } else if constexpr (ACC) {
+        // fetched before the faces, so that its latency hides behind them
+        nodes([&](int t, int, int, int, long long q) {
+#pragma unroll
+            for (int m = 0; m < 5; m++) part[t][m] = double(A.du[m * A.fs + q]);
+        });
+    }
+    tile_faces<R, R, SCH, TX, TR>(A, x0, r0, bz, sh);
+    nodes([&](int t, int idx, int, int r, long long q) {
+        put_du<R, PARTS, XTOO || ACC>(A, r, q, part[t],
+                                      [&](int v, int right) { return sh[v * (TR + 1) * TX + idx + right * TX]; });
+    });
+}
+
 
 // ---------------------------------------------------------------------------
 // Characteristic-space reconstruction (CHARTERIC = 1):
@@ -819,8 +836,22 @@ template <typename S> struct YZ { static constexpr int NS = 14, NA = 16; };
 template <> struct YZ<float> { static constexpr int NS = 15, NA = 16; };
 
 // ---------------------------------------------------------------------------
-// One launch per direction: x writes du, y and z add to it.  A wave of the x
-// sweep is a block of its own.
+// Larger grids: x and y in one launch (k_sweep_tile with XTOO), z after it; or
+// x, y and z by themselves, x writing du, the others adding to it.  A wave of
+// the x sweep is a block of its own.
+//
+// x and y together move 128 B a point in FP64 instead of 248 (the primitives
+// once, du written and not read back), yet take as long as the two alone where
+// these run at the copy rate (1024x256x128 ramp 1.77 -> 1.80 ms): barriers, LDS
+// (57 % of the cycles) and VALU (57 %) bound the tile.  What they leave to the
+// gradient kernel on the other stream is the gain: a step of 1024x256x128
+// 19.88 -> 19.55 ms, 640x192x96 5.18 -> 5.00, 256x128x128 WENO7 3.08 -> 3.00 (x + y
+// 465 -> 431 us), mixed 512x128x64 1.69 -> 1.61, mixed 131x99x80 0.648 -> 0.626.
+// Two neighbouring faces a thread, which read 40 LDS values a face for 70,
+// need 104-122 VGPRs for 76 and were slower (276 -> 310 us at 512x128x64), and so
+// were more threads a block; x lines spread free of bank conflicts (17 % of the
+// LDS cycles), and hybrid_auto's special faces given out over the wave as in
+// sweep_x, changed nothing.
 // ---------------------------------------------------------------------------
 template <int SCH, int XR, typename S, bool LEARN>
 __global__ void __launch_bounds__(64) k_sweep_x(SweepArgsT<S> A) {
@@ -828,12 +859,13 @@ __global__ void __launch_bounds__(64) k_sweep_x(SweepArgsT<S> A) {
     const Blk B = xcd_block();
     sweep_x<SCH, XR, 1, false, S, LEARN>(A, B.x, B.y, B.z, sh);
 }
-template <int DIR, int SCH, typename S>
-__global__ void __launch_bounds__(256) k_sweep_yz(SweepArgsT<S> A) {
+template <int DIR, int SCH, bool XTOO, typename S>
+__global__ void __launch_bounds__(256) k_sweep_tile(SweepArgsT<S> A) {
     constexpr int NS = YZ<S>::NS, NA = YZ<S>::NA;
-    __shared__ S sh[10 * (NS + 8) * NA];
+    constexpr int LR = (NS + 8) * NA, LX = XTOO ? (NA + 8) * NS : 0;
+    __shared__ S sh[10 * (LR > LX ? LR : LX)];
     const Blk B = xcd_block();
-    sweep_yz<DIR, SCH, NS, NA, true, S>(A, B.x, B.y, B.z, sh);
+    sweep_tile<DIR, SCH, NA, NS, XTOO, !XTOO, false, S>(A, B.x, B.y, B.z, sh);
 }
 // hybrid_auto is held to 3 waves per SIMD (168 VGPRs, 8 spilled): at 2 the
 // kernel is latency-bound (203x93x45, one launch: x 139 -> 111 us; y and z,
@@ -860,7 +892,7 @@ __global__ void __launch_bounds__(256, SCH == OCFD_HYBRIDAUTO ? 3 : 2) k_char(Sw
 // cutting the domain into boxes whose x, y and z blocks follow one another, for
 // the Infinity Cache, was slower at every size (64^3 51-59 us, 256x128x128
 // 720-860).  The SYMBO schemes are held to 4 waves per SIMD (128 VGPRs, 2
-// spilled) where they would take 3: 97x61x53, 91 -> 84 us; k_sweep_yz, which
+// spilled) where they would take 3: 97x61x53, 91 -> 84 us; k_sweep_tile, which
 // would spill 18, is not (256x128x128: 249 us, held 299).
 // ---------------------------------------------------------------------------
 struct SweepGrid {
@@ -891,11 +923,11 @@ __global__ void __launch_bounds__(256, SCH == OCFD_WENO7_SYMBO || SCH == OCFD_WE
     }
     b -= G.run[0];
     if (b < (unsigned)G.run[1]) {
-        if (run_tile(b, G.run[1], G.nt[1], t)) sweep_yz<1, SCH, NS, NA, false, S>(A, t.x, t.y, t.z, sh);
+        if (run_tile(b, G.run[1], G.nt[1], t)) sweep_tile<1, SCH, NA, NS, false, false, true, S>(A, t.x, t.y, t.z, sh);
         return;
     }
     b -= G.run[1];
-    if (run_tile(b, G.run[2], G.nt[2], t)) sweep_yz<2, SCH, NS, NA, false, S>(A, t.x, t.y, t.z, sh);
+    if (run_tile(b, G.run[2], G.nt[2], t)) sweep_tile<2, SCH, NA, NS, false, false, true, S>(A, t.x, t.y, t.z, sh);
 }
 
 int tiles(int n, int t) { return (n + t - 1) / t; }
@@ -928,26 +960,27 @@ template <int SCH, typename S>
 void launch_scheme(int dir, const SweepArgsT<S>& a, hipStream_t st) {
     const Geo& g = a.g;
     constexpr int NS = YZ<S>::NS, NA = YZ<S>::NA;
-    if (dir < 0) {
+    if (dir == SWEEP_XY) {
+        hipLaunchKernelGGL((k_sweep_tile<1, SCH, true, S>), dim3(tiles(g.nx, NA), tiles(g.ny, NS), g.nz), dim3(256), 0, st,
+                           a);
+    } else if (dir < 0) {
         launch_merged<SCH>(a, dir == SWEEP_YZ, st);
-    } else if (dir == 0) {
-        if constexpr (SCH == OCFD_HYBRIDAUTO) {
-            if (a.mlp.P) {
-                hipLaunchKernelGGL((k_sweep_x<SCH, 1, S, true>), dim3(tiles(g.nx, XSeg<1>::XS), g.ny, g.nz), dim3(64), 0,
-                                   st, a);
-                return;
-            }
-        }
-        if (two_segments(g))
+    } else if (dir == 2) {
+        hipLaunchKernelGGL((k_sweep_tile<2, SCH, false, S>), dim3(tiles(g.nx, NA), tiles(g.nz, NS), g.ny), dim3(256), 0, st,
+                           a);
+    } else if constexpr (SCH == OCFD_HYBRIDAUTO) {  // the one scheme for which x and y may be apart (sweeps_xy)
+        if (dir == 1)
+            hipLaunchKernelGGL((k_sweep_tile<1, SCH, false, S>), dim3(tiles(g.nx, NA), tiles(g.ny, NS), g.nz), dim3(256), 0,
+                               st, a);
+        else if (a.mlp.P)
+            hipLaunchKernelGGL((k_sweep_x<SCH, 1, S, true>), dim3(tiles(g.nx, XSeg<1>::XS), g.ny, g.nz), dim3(64), 0, st,
+                               a);
+        else if (two_segments(g))
             hipLaunchKernelGGL((k_sweep_x<SCH, 2, S, false>), dim3(tiles(g.nx, XSeg<2>::XS), tiles(g.ny, 2), g.nz),
                                dim3(64), 0, st, a);
         else
             hipLaunchKernelGGL((k_sweep_x<SCH, 1, S, false>), dim3(tiles(g.nx, XSeg<1>::XS), g.ny, g.nz), dim3(64), 0, st,
                                a);
-    } else if (dir == 1) {
-        hipLaunchKernelGGL((k_sweep_yz<1, SCH, S>), dim3(tiles(g.nx, NA), tiles(g.ny, NS), g.nz), dim3(256), 0, st, a);
-    } else {
-        hipLaunchKernelGGL((k_sweep_yz<2, SCH, S>), dim3(tiles(g.nx, NA), tiles(g.nz, NS), g.ny), dim3(256), 0, st, a);
     }
 }
 template <int SCH, typename S>
@@ -971,6 +1004,19 @@ void launch_char_scheme(int dir, const SweepArgsT<S>& a, hipStream_t st) {
 // 296 -> 244, 61x47x39 161 -> 114, 97x61x53 540 -> 510; above, 131x99x80 mixed
 // 660 -> 667, 256x128x128 3168 -> 3300.
 bool sweeps_merged(const Geo& g) { return (long long)g.nx * g.ny * g.nz <= 500000; }
+
+// Whether x and y of a larger grid are one launch.  hybrid_auto in FP64, whose x
+// sweep alone is the cheapest, keeps them apart between 1.5 and 10 million
+// points (a step: 256x128x64 1.324 ms apart, 1.346 together; 512x128x64 2.432,
+// 2.484; 512x128x128 4.91, 5.01), where du stays in the Infinity Cache between
+// the two; below, a launch and its tail less count for more (200x90x60 0.801,
+// 0.742), above, du's bytes.
+template <typename S> bool sweeps_xy(int scheme, const Geo& g) {
+    const long long n = (long long)g.nx * g.ny * g.nz;
+    return scheme != OCFD_HYBRIDAUTO || sizeof(S) == 4 || n < 1500000 || n > 10000000;
+}
+template bool sweeps_xy<double>(int, const Geo&);
+template bool sweeps_xy<float>(int, const Geo&);
 
 template <typename S>
 int launch_sweep(int scheme, int dir, const SweepArgsT<S>& a, hipStream_t st) {

@@ -581,8 +581,11 @@ int rhs(ocfd_ctx* x, int krk, bool fused = false, bool ghosts = false) {
         // the learned sensor's x sweep writes the flags that y and z read
         if (fuse_learned) TRY(sweep(0, names[0]));
         if (!lrc) TRY(sweep(fuse_learned ? SWEEP_YZ : SWEEP_ALL, "sweeps"));
-    } else {
+    } else if (C.charteric || fuse_learned || !sweeps_xy<S>(C.scheme_invis, x->g)) {
         for (int dir = 0; dir < 3 && !lrc; dir++) TRY(sweep(dir, names[dir]));
+    } else {
+        TRY(sweep(SWEEP_XY, "sweep_xy"));
+        if (!lrc) TRY(sweep(2, names[2]));
     }
     if (lrc) return fail(OCFD_ERR_UNSUPPORTED, "scheme not supported");
     if (overlap) {

@@ -32,16 +32,19 @@ struct SweepArgsT {
         float* prob;
     } mlp;
 };
-// The sweep along dir, in the order x, y, z (x writes du, y and z add to it), or
+// The sweep along dir, in the order x, y, z (x writes du, y and z add to it); x
+// and y in one launch (SWEEP_XY, which writes du; if sweeps_xy, and only then);
 // all three (SWEEP_ALL), or y and z after x (SWEEP_YZ), in one launch, each
 // direction into its own group of du.
-enum { SWEEP_ALL = -1, SWEEP_YZ = -2 };
+enum { SWEEP_ALL = -1, SWEEP_YZ = -2, SWEEP_XY = -3 };
 template <typename S>
 int launch_sweep(int scheme, int dir, const SweepArgsT<S>& a, hipStream_t st);
 // The same with the reconstruction in characteristic space (CHARTERIC = 1;
 // WENO7_SYMBO, WENO7_SYMBO_LIM, hybrid_auto): one direction at a time.
 template <typename S>
 int launch_sweep_char(int scheme, int dir, const SweepArgsT<S>& a, hipStream_t st);
+// Whether a grid whose sweeps are not merged takes x and y in one launch.
+template <typename S> bool sweeps_xy(int scheme, const Geo& g);
 // Whether a grid takes the form with a group of du per direction.
 bool sweeps_merged(const Geo& g);
 
