@@ -245,10 +245,48 @@ template <typename S>
 __device__ __forceinline__ void put_prim(const BCArgsT<S>& A, long long q, const Prim5<S>& p) {
     A.d[q] = p.d; A.u[q] = p.u; A.v[q] = p.v; A.w[q] = p.w; A.T[q] = p.T;
 }
+// (C) for face point t: its primitives after the condition, written, with the
+// viscosity and the conservative variables they give.
+template <typename S, typename F>
+__device__ __forceinline__ void refresh_face(const BCArgsT<S>& A, long long t, F&& final_prims) {
+    const Geo& g = A.g;
+    const long long nyz = (long long)g.ny * g.nz, nxz = (long long)g.nx * g.nz, nxy = (long long)g.nx * g.ny;
+    int i, j, k;
+    bool mu = false;
+    if (t < 2 * nyz) {
+        const int side = (int)(t / nyz);
+        const long long r = t % nyz;
+        i = side ? g.nx - 1 : 0; j = (int)(r % g.ny); k = (int)(r / g.ny);
+        mu = (A.mu_faces >> side) & 1;
+    } else if ((t -= 2 * nyz) < 2 * nxz) {
+        const int side = (int)(t / nxz);
+        const long long r = t % nxz;
+        i = (int)(r % g.nx); j = side ? g.ny - 1 : 0; k = (int)(r / g.nx);
+        mu = (A.mu_faces >> (2 + side)) & 1;
+    } else if ((t -= 2 * nxz) < 2 * nxy) {
+        const int side = (int)(t / nxy);
+        const long long r = t % nxy;
+        i = (int)(r % g.nx); j = (int)(r / g.nx); k = side ? g.nz - 1 : 0;
+        mu = (A.mu_faces >> (4 + side)) & 1;
+    } else {
+        return;
+    }
+    const long long q = gidx(g, i, j, k);
+    const Prim5<S> p = final_prims(i, j, k);
+    put_prim(A, q, p);
+    const double T = p.T;
+    if (mu && A.amu) A.amu[q] = S(A.c.amu_c0 * sqrt(T * T * T) / (A.c.tsb + T));
+    const double d = p.d, u = p.u, v = p.v, w = p.w;
+    A.f[q] = d;
+    A.f[A.fs + q] = u * d;
+    A.f[2 * A.fs + q] = v * d;
+    A.f[3 * A.fs + q] = w * d;
+    A.f[4 * A.fs + q] = d * ((u * u + v * v + w * w) * 0.5 + A.c.cv * T);
+}
 template <typename S>
 __global__ void k_bc108_faces(BCArgsT<S> A) {
     const Geo& g = A.g;
-    const long long nyz = (long long)g.ny * g.nz, nxz = (long long)g.nx * g.nz, nxy = (long long)g.nx * g.ny;
+    const long long nyz = (long long)g.ny * g.nz, nxz = (long long)g.nx * g.nz;
     long long t = (long long)blockIdx.x * blockDim.x + threadIdx.x;
     // inlet ghosts i = -4..-1: the four of a row on consecutive threads, 32
     // contiguous bytes per field (measured: the launch 209 -> 197 us on the
@@ -274,37 +312,7 @@ __global__ void k_bc108_faces(BCArgsT<S> A) {
         return;
     }
     t -= 4 * nxz;
-    int i, j, k;
-    bool mu = false;
-    if (t < 2 * nyz) {
-        const int side = (int)(t / nyz);
-        const long long r = t % nyz;
-        i = side ? g.nx - 1 : 0; j = (int)(r % g.ny); k = (int)(r / g.ny);
-        mu = (A.mu_faces >> side) & 1;
-    } else if ((t -= 2 * nyz) < 2 * nxz) {
-        const int side = (int)(t / nxz);
-        const long long r = t % nxz;
-        i = (int)(r % g.nx); j = side ? g.ny - 1 : 0; k = (int)(r / g.nx);
-        mu = (A.mu_faces >> (2 + side)) & 1;
-    } else if ((t -= 2 * nxz) < 2 * nxy) {
-        const int side = (int)(t / nxy);
-        const long long r = t % nxy;
-        i = (int)(r % g.nx); j = (int)(r / g.nx); k = side ? g.nz - 1 : 0;
-        mu = (A.mu_faces >> (4 + side)) & 1;
-    } else {
-        return;
-    }
-    const long long q = gidx(g, i, j, k);
-    const Prim5<S> p = bc108_final(A, i, j, k);
-    put_prim(A, q, p);
-    const double T = p.T;
-    if (mu && A.amu) A.amu[q] = S(A.c.amu_c0 * sqrt(T * T * T) / (A.c.tsb + T));
-    const double d = p.d, u = p.u, v = p.v, w = p.w;
-    A.f[q] = d;
-    A.f[A.fs + q] = u * d;
-    A.f[2 * A.fs + q] = v * d;
-    A.f[3 * A.fs + q] = w * d;
-    A.f[4 * A.fs + q] = d * ((u * u + v * v + w * w) * 0.5 + A.c.cv * T);
+    refresh_face(A, t, [&](int i, int j, int k) { return bc108_final(A, i, j, k); });
 }
 
 // ---------------------------------------------------------------------------
@@ -315,67 +323,101 @@ __global__ void k_bc108_faces(BCArgsT<S> A) {
 // disturbance table exists, else no slip; T = Tw with the density from
 // 2nd-order extrapolated pressure, or T and rho extrapolated when Tw <= 0),
 // then the symmetry planes (y ghosts mirrored about j = 0 and j = ny-1, v
-// odd).  One launch per step of the reference, in its order.
+// odd), get_Amu on the faces it changes and the face refresh: one launch, as
+// for IBC 108, where there were nine of 3 us each (97x61x53: 32 -> 9 us a stage, a step 489 -> 426).  A
+// thread derives its point's primitives from the tables and from points that
+// the condition leaves unchanged, where planes meet by the reference's order:
+// inlet, then upper, then wall, then the mirrors.
 // ---------------------------------------------------------------------------
 template <typename S>
-__global__ void k_bc124_inlet(BCArgsT<S> A) {
-    const int j = blockIdx.x * blockDim.x + threadIdx.x, k = blockIdx.y;
+__device__ __forceinline__ Prim5<S> bc124_inlet(const BCArgsT<S>& A, int j, int k) {
+    const long long t = (long long)A.g.nz * A.g.ny, o = (long long)k * A.g.ny + j;
+    Prim5<S> p;
+    p.d = S(A.in124[o]);
+    p.u = S(A.in124[t + o]);
+    p.v = S(A.in124[2 * t + o]);
+    p.w = S(A.in124[3 * t + o]);
+    p.T = S(A.in124[4 * t + o]);
+    return p;
+}
+// primitives of (i, j, k), 0 <= i, after inlet and upper
+template <typename S>
+__device__ __forceinline__ Prim5<S> bc124_after_upper(const BCArgsT<S>& A, int i, int j, int k) {
     const Geo& g = A.g;
-    if (j >= g.ny) return;
-    const long long t = (long long)g.nz * g.ny, o = (long long)k * g.ny + j;
-    for (int i = -4; i <= 0; i++) {
+    Prim5<S> p;
+    if (k == g.nz - 1) {
+        const long long t = (long long)g.ny * g.nx, o = (long long)j * g.nx + i;
+        const double dist = A.udist124[o];
+        if (A.up124) {  // do_u2d_upper_kernel
+            p.d = S(A.up124[o]);
+            p.u = S(A.up124[t + o] + dist);
+            p.v = S(A.up124[2 * t + o]);
+            p.w = S(A.up124[3 * t + o]);
+            p.T = S(A.up124[4 * t + o]);
+        } else {  // do_u_dist_upper_kernel
+            p.d = S(1.0);
+            p.u = S(A.cos_aoa + dist);
+            p.v = S(0.0);
+            p.w = S(A.sin_aoa);
+            p.T = S(1.0);
+        }
+    } else if (i == 0) {
+        p = bc124_inlet(A, j, k);
+    } else {
         const long long q = gidx(g, i, j, k);
-        A.d[q] = S(A.in124[o]);
-        A.u[q] = S(A.in124[t + o]);
-        A.v[q] = S(A.in124[2 * t + o]);
-        A.w[q] = S(A.in124[3 * t + o]);
-        A.T[q] = S(A.in124[4 * t + o]);
+        p.d = A.d[q]; p.u = A.u[q]; p.v = A.v[q]; p.w = A.w[q]; p.T = A.T[q];
     }
+    return p;
 }
+// after the wall too
 template <typename S>
-__global__ void k_bc124_upper(BCArgsT<S> A) {
-    const int i = blockIdx.x * blockDim.x + threadIdx.x, j = blockIdx.y;
-    const Geo& g = A.g;
-    if (i >= g.nx) return;
-    const long long q = gidx(g, i, j, g.nz - 1), t = (long long)g.ny * g.nx, o = (long long)j * g.nx + i;
-    const double dist = A.udist124[o];
-    if (A.up124) {  // do_u2d_upper_kernel
-        A.d[q] = S(A.up124[o]);
-        A.u[q] = S(A.up124[t + o] + dist);
-        A.v[q] = S(A.up124[2 * t + o]);
-        A.w[q] = S(A.up124[3 * t + o]);
-        A.T[q] = S(A.up124[4 * t + o]);
-    } else {  // do_u_dist_upper_kernel
-        A.d[q] = S(1.0);
-        A.u[q] = S(A.cos_aoa + dist);
-        A.v[q] = S(0.0);
-        A.w[q] = S(A.sin_aoa);
-        A.T[q] = S(1.0);
-    }
-}
-template <typename S>
-__global__ void k_bc124_wall(BCArgsT<S> A) {
-    const int i = blockIdx.x * blockDim.x + threadIdx.x, j = blockIdx.y;
-    const Geo& g = A.g;
-    if (i >= g.nx) return;
-    const long long q0 = gidx(g, i, j, 0), q1 = gidx(g, i, j, 1), q2 = gidx(g, i, j, 2);
-    const long long t = (long long)g.ny * g.nx, o = (long long)j * g.nx + i;
+__device__ __forceinline__ Prim5<S> bc124_final(const BCArgsT<S>& A, int i, int j, int k) {
+    if (k != 0) return bc124_after_upper(A, i, j, k);
+    const Prim5<S> p1 = bc124_after_upper(A, i, j, 1), p2 = bc124_after_upper(A, i, j, 2);
+    Prim5<S> p;
     if (A.coeff124) {  // do_wall_kernel_*_V
-        A.u[q0] = S(A.coeff124[o] * A.ht);
-        A.v[q0] = S(A.coeff124[t + o] * A.ht);
-        A.w[q0] = S(A.coeff124[2 * t + o] * A.ht);
+        const long long t = (long long)A.g.ny * A.g.nx, o = (long long)j * A.g.nx + i;
+        p.u = S(A.coeff124[o] * A.ht);
+        p.v = S(A.coeff124[t + o] * A.ht);
+        p.w = S(A.coeff124[2 * t + o] * A.ht);
     } else {  // do_wall_kernel_*_NV
-        A.u[q0] = S(0.0);
-        A.v[q0] = S(0.0);
-        A.w[q0] = S(0.0);
+        p.u = p.v = p.w = S(0.0);
     }
     if (A.tw > 0.0) {
-        A.T[q0] = S(A.tw);
-        A.d[q0] = S((4.0 * double(A.d[q1]) * double(A.T[q1]) - double(A.d[q2]) * double(A.T[q2])) / (3.0 * A.tw));
+        p.T = S(A.tw);
+        p.d = S((4.0 * double(p1.d) * double(p1.T) - double(p2.d) * double(p2.T)) / (3.0 * A.tw));
     } else {
-        A.T[q0] = S((4.0 * double(A.T[q1]) - double(A.T[q2])) / 3.0);
-        A.d[q0] = S((4.0 * double(A.d[q1]) - double(A.d[q2])) / 3.0);
+        p.T = S((4.0 * double(p1.T) - double(p2.T)) / 3.0);
+        p.d = S((4.0 * double(p1.d) - double(p2.d)) / 3.0);
     }
+    return p;
+}
+template <typename S>
+__global__ void k_bc124_faces(BCArgsT<S> A, int sym) {
+    const Geo& g = A.g;
+    const long long nyz = (long long)g.ny * g.nz, nxz = (long long)g.nx * g.nz;
+    long long t = (long long)blockIdx.x * blockDim.x + threadIdx.x;
+    if (t < 4 * nyz) {  // inlet ghosts i = -4..-1
+        const int i = -4 + (int)(t & 3);
+        const long long r = t >> 2;
+        const int j = (int)(r % g.ny), k = (int)(r / g.ny);
+        put_prim(A, gidx(g, i, j, k), bc124_inlet(A, j, k));
+        return;
+    }
+    t -= 4 * nyz;
+    if (sym) {  // ghost j = -1-l from row 1+l, j = ny+l from ny-2-l
+        if (t < 8 * nxz) {
+            const int l = (int)(t / nxz);
+            const long long r = t % nxz;
+            const int i = (int)(r % g.nx), k = (int)(r / g.nx);
+            Prim5<S> p = bc124_final(A, i, l < 4 ? 1 + l : g.ny + 2 - l, k);
+            p.v = -p.v;
+            put_prim(A, gidx(g, i, l < 4 ? -1 - l : g.ny + l - 4, k), p);
+            return;
+        }
+        t -= 8 * nxz;
+    }
+    refresh_face(A, t, [&](int i, int j, int k) { return bc124_final(A, i, j, k); });
 }
 template <typename T>
 __global__ void k_mirror_y(Geo g, T* f, double sign) {
@@ -788,15 +830,11 @@ void launch_mirror_y(const Geo& g, T* f, double sign, hipStream_t st) {
 }
 
 template <typename S>
-void launch_bc124(const BCArgsT<S>& a, int sym, hipStream_t st) {
+void launch_bc124_faces(const BCArgsT<S>& a, int sym, hipStream_t st) {
     const Geo& g = a.g;
-    hipLaunchKernelGGL(k_bc124_inlet<S>, dim3((g.ny + 63) / 64, g.nz), dim3(64), 0, st, a);
-    hipLaunchKernelGGL(k_bc124_upper<S>, dim3((g.nx + 63) / 64, g.ny), dim3(64), 0, st, a);
-    hipLaunchKernelGGL(k_bc124_wall<S>, dim3((g.nx + 63) / 64, g.ny), dim3(64), 0, st, a);
-    if (sym) {
-        S* f[5] = {a.d, a.u, a.v, a.w, a.T};
-        for (int m = 0; m < 5; m++) launch_mirror_y(g, f[m], m == 2 ? -1.0 : 1.0, st);
-    }
+    const long long nyz = (long long)g.ny * g.nz, nxz = (long long)g.nx * g.nz, nxy = (long long)g.nx * g.ny;
+    const long long tot = 4 * nyz + (sym ? 8 * nxz : 0) + 2 * (nyz + nxz + nxy);
+    hipLaunchKernelGGL(k_bc124_faces<S>, dim3((unsigned)((tot + 255) / 256)), dim3(256), 0, st, a, sym);
 }
 
 template <typename S>
@@ -887,7 +925,7 @@ void launch_diag_final(const double* partE, const double* partT, long long nb, c
     template void launch_stage<S>(const StageArgsT<S>&, hipStream_t);                                        \
     template void launch_bc108<S>(const BCArgsT<S>&, hipStream_t);                                           \
     template void launch_bc108_faces<S>(const BCArgsT<S>&, hipStream_t);                                     \
-    template void launch_bc124<S>(const BCArgsT<S>&, int, hipStream_t);                                      \
+    template void launch_bc124_faces<S>(const BCArgsT<S>&, int, hipStream_t);                                \
     template void launch_mirror_y<S>(const Geo&, S*, double, hipStream_t);                                   \
     template void launch_face_refresh<S>(const BCArgsT<S>&, hipStream_t);                                    \
     template void launch_sensor<S>(const Geo&, const Consts&, const S*, const S*, int8_t*, int8_t*, int8_t*, \

@@ -465,7 +465,8 @@ int apply_bc(ocfd_ctx* x) {
             ht = 1.;
         }
         a.ht = ht;
-        TRY(timed(x, "bc124", [&] { launch_bc124(a, x->cfg.bc_npara[0] == 1, x->st); }));
+        TRY(timed(x, "bc124", [&] { launch_bc124_faces(a, x->cfg.bc_npara[0] == 1, x->st); }));
+        return 0;
     } else {
         a.amu = nullptr;  // no face changes primitives: mu is already current
     }

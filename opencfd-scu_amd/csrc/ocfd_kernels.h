@@ -177,8 +177,9 @@ template <typename S> void launch_bc108(const BCArgsT<S>& a, hipStream_t st);
 // launch_bc108 then launch_face_refresh).
 template <typename S> void launch_bc108_faces(const BCArgsT<S>& a, hipStream_t st);
 // IBC 124 (bc_user_Liftbody3d, src/OCFD_boundary_Liftbody3D.cu:185-294):
-// inlet, upper face, wall, then the symmetry planes when sym != 0.
-template <typename S> void launch_bc124(const BCArgsT<S>& a, int sym, hipStream_t st);
+// inlet, upper face, wall, the symmetry planes when sym != 0, and the face
+// refresh.
+template <typename S> void launch_bc124_faces(const BCArgsT<S>& a, int sym, hipStream_t st);
 // Mirror of one LAP field into the y ghost layers about j = 0 and j = ny-1,
 // times sign, over the interior x and z (boundary_Jac3d_kernal_y_l/r,
 // src/OCFD_Comput_Jacobian3d.cu:429-448; do_symmetry_kernel_m/p).
