@@ -324,9 +324,10 @@ __global__ void k_bc108_faces(BCArgsT<S> A) {
 // 2nd-order extrapolated pressure, or T and rho extrapolated when Tw <= 0),
 // then the symmetry planes (y ghosts mirrored about j = 0 and j = ny-1, v
 // odd), get_Amu on the faces it changes and the face refresh: one launch, as
-// for IBC 108, where there were nine of 3 us each (97x61x53: 32 -> 9 us a stage, a step 489 -> 426).  A
-// thread derives its point's primitives from the tables and from points that
-// the condition leaves unchanged, where planes meet by the reference's order:
+// for IBC 108, where there were nine of 3 us each (97x61x53: 32 -> 9 us a stage,
+// a step 489 -> 426).  A thread derives its point's primitives from the tables
+// and from points that the condition leaves unchanged, where planes meet in
+// the reference's order:
 // inlet, then upper, then wall, then the mirrors.
 // ---------------------------------------------------------------------------
 template <typename S>
