@@ -102,16 +102,24 @@ __device__ __forceinline__ void sw_split(R tmp0d, R u, R v, R w, R cc, R A1, R A
     side((E1 - a1) * q, (E2 - a2) * q, (E3 - a3) * q, fm);
 }
 
-// f+ and f- of node (i, j, k) along direction DIR.
+// What the split of a node reads, and f+ and f- of it along direction DIR.
+template <typename S> struct NodeIn { S d, u, v, w, T, a[3]; };
+template <int DIR, typename S>
+__device__ __forceinline__ NodeIn<S> load_node(const SweepArgsT<S>& A, int i, int j, int k) {
+    const long long q = gidx(A.g, i, j, k);
+    return {A.d[q], A.u[q], A.v[q], A.w[q], A.T[q],
+            {S(A.M[3 * DIR][q]), S(A.M[3 * DIR + 1][q]), S(A.M[3 * DIR + 2][q])}};
+}
+template <typename S>
+__device__ __forceinline__ void split_node(const SweepArgsT<S>& A, const NodeIn<S>& n, S* fp, S* fm) {
+    S root, inv;
+    sqrt_pair<true>(n.T, root, inv);
+    const S cc = root * S(A.c.rama);  // sound_speed_kernel, src/commen_kernel.cu:144-153
+    sw_split<S>(n.d * S(A.c.tmp0), n.u, n.v, n.w, cc, n.a[0], n.a[1], n.a[2], A.c, fp, fm);
+}
 template <int DIR, typename S>
 __device__ __forceinline__ void split_node(const SweepArgsT<S>& A, int i, int j, int k, S* fp, S* fm) {
-    const long long q = gidx(A.g, i, j, k);
-    const S d = A.d[q], u = A.u[q], v = A.v[q], w = A.w[q], T = A.T[q];
-    S root, inv;
-    sqrt_pair<true>(T, root, inv);
-    const S cc = root * S(A.c.rama);  // sound_speed_kernel, src/commen_kernel.cu:144-153
-    sw_split<S>(d * S(A.c.tmp0), u, v, w, cc, S(A.M[3 * DIR][q]), S(A.M[3 * DIR + 1][q]), S(A.M[3 * DIR + 2][q]), A.c,
-                fp, fm);
+    split_node<S>(A, load_node<DIR>(A, i, j, k), fp, fm);
 }
 
 // The direction's part of du's variable m at node i along it, added to pre if
@@ -527,13 +535,18 @@ __device__ __forceinline__ void tile_faces(const SweepArgsT<S>& A, int x0, int r
     int hy = 0;
     if (SCH == OCFD_HYBRIDAUTO && valid) hy = A.flag[DIR][gidx(g, ix(j, a0 + al), iy(j, a0 + al), iz(j, a0 + al))];
 
-    // ---- phase 1: split of NN x NA nodes into LDS
-    for (int idx = tid; idx < NN * NA; idx += 256) {
-        const int a = line(idx, NN), n = pos(idx, NN);
-        const int s = s0 - 4 + n, ac = a0 + a;
+    // ---- phase 1: split of NN x NA nodes into LDS.  FP64 issues the loads of a
+    // thread's both nodes before the first split (1024x256x128 ramp: x and y
+    // 1800 -> 1745 us, z 1086 -> 1077; 512x128x64: y 149 -> 146, z 142 -> 139); in FP32,
+    // which would lose waves to their registers, node after node is faster (x
+    // and y 180 us against 187, z 93 against 97).  The loads of y issued before
+    // the faces of x cost FP64 its fifth wave or spills (1770-1950 us).
+    constexpr int NT = NN * NA;
+    static_assert(NT <= 512, "at most two nodes per thread");
+    auto put = [&](int n, int a, bool ok, auto&& split) {
         S fp[5], fm[5];
-        if (s <= n_dir + 3 && ac < n_a) {
-            split_node<DIR>(A, ix(s, ac), iy(s, ac), iz(s, ac), fp, fm);
+        if (ok) {
+            split(fp, fm);
         } else {
 #pragma unroll
             for (int m = 0; m < 5; m++) { fp[m] = S(0); fm[m] = S(0); }
@@ -542,6 +555,28 @@ __device__ __forceinline__ void tile_faces(const SweepArgsT<S>& A, int x0, int r
         for (int m = 0; m < 5; m++) {
             sh[tile_at<ALONG, NA>(m, n, a, NN)] = fp[m];
             sh[tile_at<ALONG, NA>(5 + m, n, a, NN)] = fm[m];
+        }
+    };
+    if constexpr (sizeof(S) == 8) {
+        NodeIn<S> in[2];
+        bool ok[2];
+#pragma unroll
+        for (int p = 0; p < 2; p++) {
+            const int idx = tid + 256 * p, s = s0 - 4 + pos(idx, NN), ac = a0 + line(idx, NN);
+            ok[p] = idx < NT && s <= n_dir + 3 && ac < n_a;
+            if (ok[p]) in[p] = load_node<DIR>(A, ix(s, ac), iy(s, ac), iz(s, ac));
+        }
+#pragma unroll
+        for (int p = 0; p < 2; p++) {
+            const int idx = tid + 256 * p;
+            if (idx < NT) put(pos(idx, NN), line(idx, NN), ok[p], [&](S* fp, S* fm) { split_node<S>(A, in[p], fp, fm); });
+        }
+    } else {
+        for (int idx = tid; idx < NT; idx += 256) {
+            const int a = line(idx, NN), n = pos(idx, NN);
+            const int s = s0 - 4 + n, ac = a0 + a;
+            put(n, a, s <= n_dir + 3 && ac < n_a,
+                [&](S* fp, S* fm) { split_node<DIR>(A, ix(s, ac), iy(s, ac), iz(s, ac), fp, fm); });
         }
     }
     __syncthreads();
