@@ -877,7 +877,7 @@ template <> struct YZ<float> { static constexpr int NS = 15, NA = 16; };
 //
 // x and y together move 128 B a point in FP64 instead of 248 (the primitives
 // once, du written and not read back), yet take as long as the two alone where
-// these run at the copy rate (1024x256x128 ramp 1.77 -> 1.80 ms): barriers, LDS
+// these run at the copy rate (1024x256x128 ramp 1.77 -> 1.75 ms): barriers, LDS
 // (57 % of the cycles) and VALU (57 %) bound the tile.  What they leave to the
 // gradient kernel on the other stream is the gain: a step of 1024x256x128
 // 19.88 -> 19.55 ms, 640x192x96 5.18 -> 5.00, 256x128x128 WENO7 3.08 -> 3.00 (x + y
@@ -920,7 +920,7 @@ __global__ void __launch_bounds__(256, SCH == OCFD_HYBRIDAUTO ? 3 : 2) k_char(Sw
 // its own five fields, which the RK stage adds: the sweeps then
 // depend on nothing but the stage's state.  For small grids (sweeps_merged):
 // a launch of theirs is as long as its slowest block, and three of them with
-// their gaps are replaced by one (64^3: 24 + 21 + 21 us -> 48 us, 20x16x12: 9 +
+// their gaps are replaced by one (64^3: 24 + 21 + 21 us -> 48 us, 43 now, 20x16x12: 9 +
 // 10 + 10 -> 10).  On larger ones it gains less than the stage pays for reading
 // three parts (256x128x128: 712 -> 670 us, the stage 234 -> 297;
 // 1024x256x128: 2.96 -> 2.92 ms and 2.02 -> 2.60).  Blocks in the order x, y, z;
