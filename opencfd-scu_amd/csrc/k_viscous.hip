@@ -291,10 +291,11 @@ __device__ __forceinline__ void p2c5(double d, double u, double v, double w, dou
 // leaves them in memory (dv) for the callers that want them there.
 //
 // The stage as OCFD_time_advance_ker1/2/3 (src/OCFD_time.cu:44-94) with
-// cons->prim + p (cons_to_pri_kernel, src/commen_kernel.cu:77-109).  FP64: the
-// conserved state of stages 1 and 2 is not written; the next stage forms it
-// from the primitives, which hold the same state in the same precision (an
-// ulp).  The mixed path, whose primitives are FP32, keeps f in every stage.
+// cons->prim + p (cons_to_pri_kernel, src/commen_kernel.cu:77-109).  f is written
+// in every stage and read by the next: formed again from the primitives, which
+// would save 40 B/pt of writes in stages 1 and 2, it goes through four
+// divisions, a difference and back, and the error of the state after 10 to 40
+// steps against 80-bit arithmetic grows by 9 % (energy up to 28 %).
 // PARTS: groups of du to add (1, or 3 where each sweep writes its own).
 // G.faces: f of the six faces from the primitives as OCFD_bc leaves it
 // (src/OCFD_boundary.cu:40-91), for runs whose boundary condition changes
@@ -305,14 +306,13 @@ __device__ __forceinline__ void p2c5(double d, double u, double v, double w, dou
 // the 40 addresses of a point took the kernel to 255 VGPRs and spills (FP32:
 // slower than the separate kernels, 252 us against 215 on 512x128x64); with
 // them it needs 203, FP32 124.  Divergence and stage as one launch against
-// three (two of two flux components, then the stage): 1024x256x128 2.42 -> 2.02
-// ms, 512x128x64 296 -> 232 us, mixed 215 -> 172 us, 640x192x96 mixed 567 -> 510
+// three (two of two flux components, then the stage): 1024x256x128 2.42 -> 2.17
+// ms, 512x128x64 296 -> 251 us, mixed 215 -> 172 us, 640x192x96 mixed 567 -> 510
 // us.
 constexpr int NTD = TX * TY;
 template <int SV, typename S, int KRK, int PARTS>
 __global__ void __launch_bounds__(NTD, sizeof(S) == 8 ? 2 : 4) k_visc_div(ViscArgsT<S> A, StageArgsT<S> G, int kz) {
     static_assert(TY == 8, "one y-halo value per thread: 8 halo rows of TX columns");
-    constexpr bool FROM_PRIM = std::is_same<S, double>::value;  // f of stages 1 and 2 lives in the primitives
     // FP64, at 2 waves per SIMD, has registers to fetch the point's values a
     // plane ahead (512x128x64: 252 -> 232 us against loads after the derivatives
     // at 3 waves); FP32 fetches them before the derivatives and keeps 4 waves
@@ -361,8 +361,8 @@ __global__ void __launch_bounds__(NTD, sizeof(S) == 8 ? 2 : 4) k_visc_div(ViscAr
             for (int f = 0; f < NC; f++) xhv[f] = bs(A.ev, f, k).ld(oxh);
     };
     // the stage's own values of the point: du, Ajac, the base state fn and
-    // the state before the stage (the primitives, or f on the mixed path)
-    // (as loaded: nothing waits for them before the point is formed)
+    // the state f before the stage (as loaded: nothing waits for them before
+    // the point is formed)
     S sr[PARTS][5];
     double sj = 0.0, sn[5], so[5];
     auto load_point = [&](int k) {
@@ -376,8 +376,7 @@ __global__ void __launch_bounds__(NTD, sizeof(S) == 8 ? 2 : 4) k_visc_div(ViscAr
         for (int m = 0; m < 5; m++) sn[m] = bd(G.fn, m, k).template ld<BUF_STREAM>(od);
         if (KRK == 1) return;
 #pragma unroll
-        for (int m = 0; m < 5; m++)
-            so[m] = FROM_PRIM ? double(bs(G.d, m, k).ld(oo)) : bd(G.f, m, k).template ld<BUF_STREAM>(od);
+        for (int m = 0; m < 5; m++) so[m] = bd(G.f, m, k).template ld<BUF_STREAM>(od);
     };
 #pragma unroll
     for (int m = 0; m < 8; m++)
@@ -433,13 +432,7 @@ __global__ void __launch_bounds__(NTD, sizeof(S) == 8 ? 2 : 4) k_visc_div(ViscAr
             for (int m = 0; m < NC; m++) bs(A.dv, m, k).st(oo, S(dv[m]));
         } else {
             const double dt = G.dt;
-            double fo[5], fv[5];
-            if (KRK > 1) {
-                if (FROM_PRIM) p2c5(so[0], so[1], so[2], so[3], so[4], G.c.cv, fo);
-                else
-#pragma unroll
-                    for (int m = 0; m < 5; m++) fo[m] = so[m];
-            }
+            double fv[5];
 #pragma unroll
             for (int m = 0; m < 5; m++) {
                 double r = double(sr[0][m]);
@@ -448,8 +441,8 @@ __global__ void __launch_bounds__(NTD, sizeof(S) == 8 ? 2 : 4) k_visc_div(ViscAr
                 if (m) r += dv[m - 1];
                 r *= sj;
                 if (KRK == 1) fv[m] = sn[m] + dt * r;
-                else if (KRK == 2) fv[m] = 3.0 / 4.0 * sn[m] + 1.0 / 4.0 * (fo[m] + dt * r);
-                else fv[m] = 1.0 / 3.0 * sn[m] + 2.0 / 3.0 * (fo[m] + dt * r);
+                else if (KRK == 2) fv[m] = 3.0 / 4.0 * sn[m] + 1.0 / 4.0 * (so[m] + dt * r);
+                else fv[m] = 1.0 / 3.0 * sn[m] + 2.0 / 3.0 * (so[m] + dt * r);
             }
             const double d1 = fv[0], u1 = fv[1] / d1, v1 = fv[2] / d1, w1 = fv[3] / d1;
             const double T2 = (fv[4] - 0.5 * d1 * (u1 * u1 + v1 * v1 + w1 * w1)) / (d1 * G.c.cv);
@@ -457,15 +450,13 @@ __global__ void __launch_bounds__(NTD, sizeof(S) == 8 ? 2 : 4) k_visc_div(ViscAr
 #pragma unroll
             for (int m = 0; m < 5; m++) bs(G.d, m, k).st(oo, pr[m]);
             if (KRK == 3) bs(G.P, 0, k).template st<BUF_STREAM>(oo, S(T2 * d1 / (G.c.gamma * G.c.ama * G.c.ama)));
-            if (KRK == 3 || !FROM_PRIM) {
-                if (KRK == 3 && G.flap)
+            if (KRK == 3 && G.flap)
 #pragma unroll
-                    for (int m = 0; m < 5; m++) bd(G.flap, m, k).template st<BUF_STREAM>(od, fv[m]);
-                if (G.faces && (t.i == 0 || t.i == g.nx - 1 || t.j == 0 || t.j == g.ny - 1 || k == 0 || k == g.nz - 1))
-                    p2c5(double(pr[0]), double(pr[1]), double(pr[2]), double(pr[3]), double(pr[4]), G.c.cv, fv);
+                for (int m = 0; m < 5; m++) bd(G.flap, m, k).template st<BUF_STREAM>(od, fv[m]);
+            if (G.faces && (t.i == 0 || t.i == g.nx - 1 || t.j == 0 || t.j == g.ny - 1 || k == 0 || k == g.nz - 1))
+                p2c5(double(pr[0]), double(pr[1]), double(pr[2]), double(pr[3]), double(pr[4]), G.c.cv, fv);
 #pragma unroll
-                for (int m = 0; m < 5; m++) bd(G.f, m, k).template st<BUF_STREAM>(od, fv[m]);
-            }
+            for (int m = 0; m < 5; m++) bd(G.f, m, k).template st<BUF_STREAM>(od, fv[m]);
             auto copy_to = [&](int kk, unsigned o) {
 #pragma unroll
                 for (int m = 0; m < 5; m++) bs(G.d, m, kk).st(o, pr[m]);

@@ -101,9 +101,7 @@ struct StageArgsT {
 };
 template <typename S> void launch_stage(const StageArgsT<S>& a, hipStream_t st);
 // The divergence of the viscous fluxes and the RK stage in one pass (the
-// viscous part of du never goes to memory).  On the
-// FP64 path f is written in stage 3 only: stages 2 and 3 form it from the
-// primitives.
+// viscous part of du never goes to memory).
 template <typename S>
 void launch_visc_stage(const ViscArgsT<S>& a, const StageArgsT<S>& s, hipStream_t st);
 
