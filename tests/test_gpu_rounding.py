@@ -26,3 +26,20 @@ def test_stages_keep_the_conserved_state(ma):
     inner = np.s_[:, 1:-1, 1:-1, 1:-1]
     assert (np.abs(f1 - f0)[inner] <= np.spacing(np.abs(f0))[inner]).all()
     g.close()
+
+
+@pytest.mark.parametrize("ma", [0.1, 0.3])
+def test_initial_energy(ma):
+    """d (|u|^2 / 2 + cv T) at low Mach, where cv T is nearly all of it: one
+    fused sum and one product, 2^-53 each, and three roundings of the square
+    in the kinetic share.  A product cv T rounded by itself would add a third 2^-53."""
+    case = cases.wavy_box(40, 32, 24, ma=ma)
+    g = case.load(capi.Solver(case.cfg))
+    E = g.get_state()[4]
+    g.close()
+    d, u, v, w, T = (a.astype(np.longdouble) for a in case.prims)
+    gamma = case.cfg.gamma
+    cv = np.longdouble(1.0 / (gamma * (gamma - 1.0) * ma * ma))
+    kin = d * (u * u + v * v + w * w) / 2
+    exact = kin + d * cv * T
+    assert (np.abs(E - exact) <= (2 * exact + 3 * kin) * 2.0 ** -53).all()
