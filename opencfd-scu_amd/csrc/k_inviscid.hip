@@ -60,16 +60,17 @@ __device__ __forceinline__ void sqrt_pair(R x, R& root, R& inv) {
     }
 }
 
-// Steger-Warming split of one node (src/OCFD_split.cu:92-142).  With n = A/|A|,
-// t = l2 + l3 and D = c (l3 - l2), the reference's sums over the three waves
-// are
-//   f0 = C1 l1 + t,  f_i = u_i f0 + n_i D,
-//   f4 = l1 (gamma-1)|u|^2 + t (|u|^2/2 + c^2/2 + W c^2) + (u.n) D
-// (its |u -+ c n|^2 written out with |n| = 1): 85 instructions a node against
-// 165, its error against 80-bit arithmetic the same or smaller in every
-// component (rms over Mach 0.1-8: FP64 0.93-1.00, FP32 0.84-1.00 of the sums'),
-// and the y sweep of 256x128x128 WENO7 204 -> 194 us, of 1024x256x128 1068 ->
-// 1041.  l = (E +- |E|)/2 with the factor rho/(2 gamma) in it.
+// Steger-Warming split of one node (src/OCFD_split.cu:92-142), the reference's
+// sums over the three waves with u -+ c n formed in one fused operation from
+// c/|A| and the waves' energies |u -+ c n|^2/2 + W c^2 formed once for both
+// sides: about 100 instructions a node against 165.  Summed instead as f_i =
+// u_i f0 + n_i c (l3 - l2), 85 instructions, the energy of a low-Mach flow
+// cancels: du's error against 80-bit arithmetic was up to 8 % (ramp 14 %) above
+// the reference's sums' in a component, while a step took 1 % less (1024x256x128
+// 19.75 ms, now 19.95; y sweep of 512x128x64 147.8 us, 148.3).  Written with n
+// normalised first or with W c^2 apart it rounds no better in the state and
+// the z sweep loses its fifth wave (1083 -> 1127 us).  l = (E +- |E|)/2 with the
+// factor rho/(2 gamma) in it.
 template <typename R>
 __device__ __forceinline__ void sw_split(R tmp0d, R u, R v, R w, R cc, R A1, R A2, R A3, const Consts& c,
                                          R* fp, R* fm) {
@@ -86,17 +87,20 @@ __device__ __forceinline__ void sw_split(R tmp0d, R u, R v, R w, R cc, R A1, R A
     } else {
         a1 = sqrt(E1 * E1 + eps * eps); a2 = sqrt(E2 * E2 + eps * eps); a3 = sqrt(E3 * E3 + eps * eps);
     }
-    const R k2 = u * u + v * v + w * w, c2 = cc * cc, ccr = cc * rs;
-    const R vv = (R(c.gamma) - R(1.0)) * k2;
-    const R K = fma(R(c.split_c3), c2, R(0.50) * (k2 + c2));
+    const R k2 = u * u + v * v + w * w, ccr = cc * rs;
+    // u -+ c n
+    const R um = fma(-ccr, A1, u), up = fma(ccr, A1, u), vm = fma(-ccr, A2, v), vp = fma(ccr, A2, v),
+            wm = fma(-ccr, A3, w), wp = fma(ccr, A3, w);
+    const R vv = (R(c.gamma) - R(1.0)) * k2, W2 = R(c.split_c3) * cc * cc;
+    const R Km = fma(R(0.50), um * um + vm * vm + wm * wm, W2), Kp = fma(R(0.50), up * up + vp * vp + wp * wp, W2);
     const R C1 = R(c.split_c1), q = R(0.50) * tmp0d;
     auto side = [&](R l1, R l2, R l3, R* f) {
-        const R t = l2 + l3, D = (l3 - l2) * ccr;
-        f[0] = fma(C1, l1, t);
-        f[1] = fma(u, f[0], A1 * D);
-        f[2] = fma(v, f[0], A2 * D);
-        f[3] = fma(w, f[0], A3 * D);
-        f[4] = fma(t, K, fma(E1, D, l1 * vv));
+        const R a = C1 * l1;
+        f[0] = fma(C1, l1, l2) + l3;
+        f[1] = fma(l3, up, fma(l2, um, a * u));
+        f[2] = fma(l3, vp, fma(l2, vm, a * v));
+        f[3] = fma(l3, wp, fma(l2, wm, a * w));
+        f[4] = fma(l3, Kp, fma(l2, Km, l1 * vv));
     };
     side((E1 + a1) * q, (E2 + a2) * q, (E3 + a3) * q, fp);
     side((E1 - a1) * q, (E2 - a2) * q, (E3 - a3) * q, fm);
