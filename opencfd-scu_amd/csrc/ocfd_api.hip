@@ -49,9 +49,10 @@ struct ocfd_ctx {
     ocfd_config cfg;
     int device = 0;
     hipStream_t st = nullptr;
-    // second stream: the viscous gradients, fluxes and divergence run beside
-    // the inviscid sweeps (they share inputs only; the divergence writes its
-    // own buffer dv); joined before the RK stage
+    // second stream: the viscous gradients and fluxes (and, where a right-hand
+    // side is asked for by itself, their divergence into dv) run beside the
+    // inviscid sweeps, with which they share inputs only; joined before the
+    // RK stage
     hipStream_t st2 = nullptr;
     hipEvent_t ev_fork = nullptr, ev_join = nullptr;
     bool serial = false;  // OCFD_SERIAL=1: one stream (per-kernel timing with an external profiler)
@@ -72,7 +73,8 @@ struct ocfd_ctx {
     double *d = nullptr, *u = nullptr, *v = nullptr, *w = nullptr, *T = nullptr, *P = nullptr;
     // du: the inviscid part, or with du_parts = 3 (small grids, sweeps_merged)
     // 3 x 5 fields, one group written by each sweep; dv: the viscous part of
-    // du[1..4].  The stage adds them.
+    // du[1..4], allocated by the first call that wants a right-hand side in
+    // memory (need_dv: a step's stage forms it in registers).
     int du_parts = 1;
     double *du = nullptr, *amu = nullptr, *ev = nullptr, *dv = nullptr;
     float *sd = nullptr, *su = nullptr, *sv = nullptr, *sw = nullptr, *sT = nullptr, *sP = nullptr;
@@ -240,6 +242,29 @@ int8_t* alloc_bytes(ocfd_ctx* x, size_t n, int& rc) {
         return nullptr;
     }
     return (int8_t*)p + 96;
+}
+
+// The device of a context for the allocations of a call that may come from a
+// thread whose current device is another one.
+struct OnDevice {
+    int prev = -1;
+    explicit OnDevice(int d) {
+        if (hipGetDevice(&prev) != hipSuccess || prev == d || hipSetDevice(d) != hipSuccess) prev = -1;
+    }
+    ~OnDevice() {
+        if (prev >= 0) (void)hipSetDevice(prev);
+    }
+};
+
+// The buffer dv: 4 fields beside the 56 (mixed: 32 and 24 FP32) of a context,
+// which a run that only steps never reads.
+int need_dv(ocfd_ctx* x) {
+    if (x->dv || x->sdv) return 0;
+    OnDevice on(x->device);
+    int rc = 0;
+    if (x->mixed) x->sdv = alloc_fields_f32(x, 4, rc);
+    else x->dv = alloc_fields(x, 4, rc);
+    return rc;
 }
 
 bool supported_scheme(int s) { return (s >= OCFD_UP7 && s <= OCFD_HYBRIDAUTO); }
@@ -507,11 +532,12 @@ ViscArgsT<S> visc_args(ocfd_ctx* x) {
 
 // The right-hand side of a stage: the inviscid part into du, the viscous
 // fluxes into Ev and, unless the caller's stage takes their divergence itself
-// (fused: launch_visc_stage), the viscous part into dv or du.  ghosts: the
+// (fused: launch_visc_stage), the viscous part into dv.  ghosts: the
 // periodic ghost layers of the primitives already hold the stage's state.
 template <typename S>
 int rhs(ocfd_ctx* x, int krk, bool fused = false, bool ghosts = false) {
     const ocfd_config& C = x->cfg;
+    if (!fused) TRY(need_dv(x));
     const View<S> V = view<S>(x);
     // hybrid_auto flags, once per step at the first stage: the plain sensor
     // before the periodic fill, as du_comput orders it (it reads the ghost
@@ -609,6 +635,7 @@ int finish_rhs_t(ocfd_ctx* x) {
     return 0;
 }
 int finish_rhs(ocfd_ctx* x) {
+    TRY(need_dv(x));
     if (!x->div_pending) return 0;
     return x->mixed ? finish_rhs_t<float>(x) : finish_rhs_t<double>(x);
 }
@@ -1100,22 +1127,20 @@ int ocfd_create(const ocfd_config* cfg, int device, ocfd_ctx** out) {
         double* dua = rc ? nullptr : alloc_fields(x, 5 * x->du_parts, rc);
         double* am = rc ? nullptr : alloc_fields(x, 1, rc);
         double* ev = rc ? nullptr : alloc_fields(x, 12, rc);
-        double* dva = rc ? nullptr : alloc_fields(x, 4, rc);
         if (!rc) {
             x->d = prim; x->u = prim + x->fs; x->v = prim + 2 * x->fs; x->w = prim + 3 * x->fs;
             x->T = prim + 4 * x->fs; x->P = prim + 5 * x->fs;
-            x->du = dua; x->amu = am; x->ev = ev; x->dv = dva;
+            x->du = dua; x->amu = am; x->ev = ev;
         }
     } else {
         float* prim = rc ? nullptr : alloc_fields_f32(x, 6, rc);
         float* dua = rc ? nullptr : alloc_fields_f32(x, 5 * x->du_parts, rc);
         float* am = rc ? nullptr : alloc_fields_f32(x, 1, rc);
         float* ev = rc ? nullptr : alloc_fields_f32(x, 12, rc);
-        float* dva = rc ? nullptr : alloc_fields_f32(x, 4, rc);
         if (!rc) {
             x->sd = prim; x->su = prim + x->fs; x->sv = prim + 2 * x->fs; x->sw = prim + 3 * x->fs;
             x->sT = prim + 4 * x->fs; x->sP = prim + 5 * x->fs;
-            x->sdu = dua; x->samu = am; x->sev = ev; x->sdv = dva;
+            x->sdu = dua; x->samu = am; x->sev = ev;
         }
     }
     for (int dd = 0; dd < 3 && !rc; dd++) x->flag[dd] = alloc_bytes(x, (size_t)x->fs, rc);

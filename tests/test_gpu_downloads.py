@@ -37,3 +37,25 @@ def test_flow_comes_back_as_loaded(size, prec):
     assert get(s.h, None, as_p(u), None, None, as_p(T), None, None) == 0
     assert np.array_equal(u, prims[1]) and np.array_equal(T, prims[4])
     s.close()
+
+
+@pytest.mark.parametrize("prec", [capi.PREC_FP64, capi.PREC_MIXED])
+def test_a_stepping_run_holds_no_viscous_right_hand_side(prec):
+    """The four fields of the viscous part of the right-hand side are
+    allocated by the first call that wants them in memory, not by a run that
+    only steps."""
+    case = cases.wavy_box(160, 128, 64, scheme="UP7", precision=prec)
+    s = case.load(capi.Solver(case.cfg))
+    hip = C.CDLL("libamdhip64.so")
+
+    def free():
+        a, b = C.c_size_t(), C.c_size_t()
+        assert hip.hipMemGetInfo(C.byref(a), C.byref(b)) == 0
+        return a.value
+
+    s.step(2)  # with what the runtime allocates for the streams
+    before = free()
+    assert np.isfinite(s.get_du()).all()
+    fields = 4 * case.npoints * (8 if prec == capi.PREC_FP64 else 4)
+    assert fields <= before - free() <= 2 * fields
+    s.close()
