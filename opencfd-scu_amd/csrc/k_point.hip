@@ -57,26 +57,30 @@ __global__ void __launch_bounds__(256) k_fill(Geo g, T* base, int nf, long long 
 // with cons->prim + p (cons_to_pri_kernel, src/commen_kernel.cu:77-109) and
 // Sutherland's law (get_Amu_kernal, src/commen_kernel.cu:122-131).
 // ---------------------------------------------------------------------------
+// The right-hand side of a point: the inviscid part (or parts of x, y and z),
+// then the viscous part (components 1..4), all read once as streaming
+// (non-temporal) loads.  The sweeps and the divergence leave out the node's
+// Ajac, by which the reference multiplies each of their terms: it is applied to
+// the sum here.
 template <typename S>
-__global__ void __launch_bounds__(256) k_stage(StageArgsT<S> A) {
-    const int i = blockIdx.x * 64 + threadIdx.x, j = blockIdx.y * 4 + threadIdx.y, k = blockIdx.z;
-    if (i >= A.g.nx || j >= A.g.ny) return;
-    const long long q = gidx(A.g, i, j, k);
-    // the inviscid part (or parts of x, y and z), then the viscous part
-    // (components 1..4), all read once as streaming (non-temporal) loads
-    double du[5];
+__device__ __forceinline__ void sum_du(const StageArgsT<S>& A, long long q, double* du) {
+    const double ajac = __builtin_nontemporal_load(&A.jac[q]);
 #pragma unroll
     for (int m = 0; m < 5; m++) {
         auto part = [&](int dir) { return double(__builtin_nontemporal_load(&A.du[(5 * dir + m) * A.fs + q])); };
         du[m] = part(0);
         if (A.parts == 3) du[m] = (du[m] + part(1)) + part(2);
         if (m) du[m] += double(__builtin_nontemporal_load(&A.dv[(m - 1) * A.fs + q]));
+        du[m] *= ajac;
     }
-    // the sweeps and the divergence leave out the node's Ajac, by which the
-    // reference multiplies each of their terms: it is applied to the sum here
-    const double ajac = __builtin_nontemporal_load(&A.jac[q]);
-#pragma unroll
-    for (int m = 0; m < 5; m++) du[m] *= ajac;
+}
+template <typename S>
+__global__ void __launch_bounds__(256) k_stage(StageArgsT<S> A) {
+    const int i = blockIdx.x * 64 + threadIdx.x, j = blockIdx.y * 4 + threadIdx.y, k = blockIdx.z;
+    if (i >= A.g.nx || j >= A.g.ny) return;
+    const long long q = gidx(A.g, i, j, k);
+    double du[5];
+    sum_du(A, q, du);
     stage_point(A, q, du);
 }
 
@@ -786,6 +790,22 @@ __global__ void __launch_bounds__(256) k_pack(PackArgsT<S> A) {
     for (int f = 0; f < A.nf; f++) __builtin_nontemporal_store(A.src[f][q], &d[f * n]);
 }
 
+// The right-hand side for the host in one launch and one download: 20x16x12 279
+// -> 21 us, 97x61x53 4.36 -> 0.68 ms, mixed 256x128x128 30.6 -> 12.5 ms against
+// the parts fetched one by one and added on the host.
+template <typename S>
+__global__ void __launch_bounds__(256) k_pack_du(StageArgsT<S> A, double* __restrict__ dst) {
+    const Geo& g = A.g;
+    const int i = blockIdx.x * 64 + threadIdx.x, j = blockIdx.y * 4 + threadIdx.y, k = blockIdx.z;
+    if (i >= g.nx || j >= g.ny) return;
+    const long long n = (long long)g.nx * g.ny * g.nz;
+    double du[5];
+    sum_du(A, gidx(g, i, j, k), du);
+    double* d = dst + i + (long long)g.nx * (j + (long long)g.ny * k);
+#pragma unroll
+    for (int m = 0; m < 5; m++) __builtin_nontemporal_store(du[m], &d[m * n]);
+}
+
 template <typename To, typename From>
 __global__ void k_convert(To* dst, const From* src, long long n) {
     const long long t = (long long)blockIdx.x * blockDim.x + threadIdx.x;
@@ -895,6 +915,11 @@ void launch_pack(const PackArgsT<S>& a, hipStream_t st) {
     hipLaunchKernelGGL(k_pack<S>, pgrid(a.g), dim3(64, 4), 0, st, a);
 }
 
+template <typename S>
+void launch_pack_du(const StageArgsT<S>& a, double* dst, hipStream_t st) {
+    hipLaunchKernelGGL(k_pack_du<S>, pgrid(a.g), dim3(64, 4), 0, st, a, dst);
+}
+
 template <typename To, typename From>
 void launch_convert(To* dst, const From* src, long long n, hipStream_t st) {
     hipLaunchKernelGGL((k_convert<To, From>), dim3((unsigned)((n + 255) / 256)), dim3(256), 0, st, dst, src, n);
@@ -934,6 +959,7 @@ void launch_diag_final(const double* partE, const double* partT, long long nb, c
     template void launch_filter<S>(const FilterArgsT<S>&, hipStream_t);                                      \
     template void launch_p2c_all<S>(const BCArgsT<S>&, hipStream_t);                                         \
     template void launch_pack<S>(const PackArgsT<S>&, hipStream_t);                                          \
+    template void launch_pack_du<S>(const StageArgsT<S>&, double*, hipStream_t);                             \
     template void launch_c2p_all<S>(const StageArgsT<S>&, hipStream_t);                                      \
     template void launch_amu_all<S>(const BCArgsT<S>&, hipStream_t);                                        \
     template void launch_diag<S>(const Geo&, const double*, const S*, double*, double*, int*, hipStream_t);  \

@@ -320,28 +320,18 @@ const void* d2h(ocfd_ctx* x, const void* src, size_t bytes, int& rc) {
         if (rc_) return rc_;                          \
     } while (0)
 
-// The interiors of nf fields (null destinations are left out) to host arrays,
-// widened from S.  The GPU packs them without their ghost layers, so that the
-// host copies long runs instead of rows; up to DIRECT bytes it packs straight
+// nf arrays of interior values to host arrays, widened from S: pack(dst) launches
+// what writes them to dst without ghost layers, one after another, so that the
+// host copies long runs instead of rows.  Up to DIRECT bytes it writes straight
 // into the pinned buffer (no copy of its own: a 20x16x12 state 5 copies and
 // waits -> 1), above that the packed values come over in pieces of PIECE bytes,
 // three in flight, while the host copies the one before.
-template <typename S>
-int download_fields(ocfd_ctx* x, const S* const* src, double* const* dst, int nf) {
+template <typename S, typename F>
+int download_packed(ocfd_ctx* x, double* const* out, int nf, F&& pack) {
     constexpr size_t DIRECT = 1u << 20, PIECE = 16u << 20;
     constexpr int SLOTS = 3;
     const size_t n = (size_t)x->g.nx * x->g.ny * x->g.nz;
-    PackArgsT<S> a;
-    double* out[PACK_FIELDS];
-    a.g = x->g;
-    a.nf = 0;
-    for (int q = 0; q < nf; q++)
-        if (dst[q]) {
-            out[a.nf] = dst[q];
-            a.src[a.nf++] = src[q];
-        }
-    if (!a.nf) return 0;
-    const size_t total = n * a.nf, bytes = total * sizeof(S);
+    const size_t total = n * nf, bytes = total * sizeof(S);
     auto unpack = [&](const S* p, size_t first, size_t count) {
         while (count) {
             const size_t o = first % n, m = std::min(count, n - o);
@@ -356,23 +346,22 @@ int download_fields(ocfd_ctx* x, const S* const* src, double* const* dst, int nf
     };
     if (bytes <= DIRECT) {
         TRY(ensure_pin(x, bytes));
-        a.dst = (S*)x->pin;
-        TRY(timed(x, "pack", [&] { launch_pack(a, x->st); }));
+        TRY(timed(x, "pack", [&] { pack((S*)x->pin); }));
         HIPCK(hipStreamSynchronize(x->st));
         unpack((const S*)x->pin, 0, total);
         return 0;
     }
     // packed into the scratch fields after the first (which ocfd_get_q fills)
-    a.dst = (S*)(x->grad + x->fs);
+    S* const dev = (S*)(x->grad + x->fs);
     const size_t piece = PIECE / sizeof(S), np = (total + piece - 1) / piece;
     TRY(ensure_pin(x, std::min(bytes, SLOTS * PIECE)));
     for (auto& e : x->pin_ev)
         if (!e) HIPCK(hipEventCreateWithFlags(&e, hipEventDisableTiming));
-    TRY(timed(x, "pack", [&] { launch_pack(a, x->st); }));
+    TRY(timed(x, "pack", [&] { pack(dev); }));
     auto slot = [&](size_t c) { return (S*)x->pin + (c % SLOTS) * piece; };
     auto count = [&](size_t c) { return std::min(piece, total - c * piece); };
     auto fetch = [&](size_t c) -> int {
-        HIPCK(hipMemcpyAsync(slot(c), a.dst + c * piece, count(c) * sizeof(S), hipMemcpyDeviceToHost, x->st));
+        HIPCK(hipMemcpyAsync(slot(c), dev + c * piece, count(c) * sizeof(S), hipMemcpyDeviceToHost, x->st));
         HIPCK(hipEventRecord(x->pin_ev[c % SLOTS], x->st));
         return 0;
     };
@@ -383,6 +372,25 @@ int download_fields(ocfd_ctx* x, const S* const* src, double* const* dst, int nf
         if (c + SLOTS < np) TRY(fetch(c + SLOTS));
     }
     return 0;
+}
+
+// The interiors of nf fields (null destinations are left out) to host arrays.
+template <typename S>
+int download_fields(ocfd_ctx* x, const S* const* src, double* const* dst, int nf) {
+    PackArgsT<S> a;
+    double* out[PACK_FIELDS];
+    a.g = x->g;
+    a.nf = 0;
+    for (int q = 0; q < nf; q++)
+        if (dst[q]) {
+            out[a.nf] = dst[q];
+            a.src[a.nf++] = src[q];
+        }
+    if (!a.nf) return 0;
+    return download_packed<S>(x, out, a.nf, [&](S* d) {
+        a.dst = d;
+        launch_pack(a, x->st);
+    });
 }
 template <typename S>
 int download_any(ocfd_ctx* x, const S* src, double* dst) {
@@ -1438,27 +1446,12 @@ int ocfd_get_du(ocfd_ctx* x, double* du5) {
     if (!x || !du5) return fail(OCFD_ERR_ARG, "null argument");
     TRY(finish_rhs(x));
     const size_t n = (size_t)x->g.nx * x->g.ny * x->g.nz;
-    // the parts of x, y and z and the viscous part of components 1..4, added as
-    // the RK stage adds them, then the Jacobian factor it applies
-    std::vector<double> tmp(n);
-    auto get = [&](int part, int m, double* out) {
-        const long long o = (part < 3 ? 5 * part + m : m - 1) * x->fs;
-        return x->mixed ? download_any(x, (const float*)((part < 3 ? x->sdu : x->sdv) + o), out)
-                        : download_any(x, (const double*)((part < 3 ? x->du : x->dv) + o), out);
-    };
-    for (int m = 0; m < 5; m++) {
-        double* d = du5 + m * n;
-        TRY(get(0, m, d));
-        for (int part = 1; part < (m ? 4 : 3); part++) {
-            if (part < 3 && part >= x->du_parts) continue;
-            TRY(get(part, m, tmp.data()));
-            for (size_t p = 0; p < n; p++) d[p] += tmp[p];
-        }
-    }
-    TRY(download_any(x, (const double*)x->M[M_JAC], tmp.data()));
-    for (int m = 0; m < 5; m++)
-        for (size_t p = 0; p < n; p++) du5[m * n + p] *= tmp[p];
-    return 0;
+    double* out[5];
+    for (int m = 0; m < 5; m++) out[m] = du5 + m * n;
+    return download_packed<double>(x, out, 5, [&](double* d) {
+        if (x->mixed) launch_pack_du(stage_args<float>(x, 1, false), d, x->st);
+        else launch_pack_du(stage_args<double>(x, 1, false), d, x->st);
+    });
 }
 
 int ocfd_get_pressure(ocfd_ctx* x, double* p) {

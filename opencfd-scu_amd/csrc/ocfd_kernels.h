@@ -274,6 +274,9 @@ struct PackArgsT {
     S* dst;
 };
 template <typename S> void launch_pack(const PackArgsT<S>& a, hipStream_t st);
+// The five components of the right-hand side as the stage takes it (the parts of
+// du and dv added, times Ajac), packed likewise.
+template <typename S> void launch_pack_du(const StageArgsT<S>& a, double* dst, hipStream_t st);
 
 // dst[i] = (To)src[i] for n elements (precision conversion of whole fields).
 template <typename To, typename From>

@@ -59,3 +59,29 @@ def test_a_stepping_run_holds_no_viscous_right_hand_side(prec):
     fields = 4 * case.npoints * (8 if prec == capi.PREC_FP64 else 4)
     assert fields <= before - free() <= 2 * fields
     s.close()
+
+
+@pytest.mark.parametrize("size,scheme,prec", [
+    ((8, 9, 8), "UP7", capi.PREC_FP64), ((20, 16, 12), "WENO7", capi.PREC_MIXED),
+    ((65, 41, 33), "WENO5", capi.PREC_FP64), ((97, 71, 75), "UP7", capi.PREC_MIXED)])
+def test_right_hand_side_in_one_download(size, scheme, prec):
+    """The parts of the right-hand side are added on the GPU and fetched at
+    once, after ocfd_rhs and after a step, in one launch beside the divergence
+    that a step leaves out."""
+    case = cases.wavy_box(*size, scheme=scheme, precision=prec)
+    s = case.load(capi.Solver(case.cfg))
+    s.rhs(1)
+    a = s.get_du()
+    s.profile(True)
+    s.step(1)
+    s.profile_reset()
+    b = s.get_du()
+    assert np.array_equal(b, s.get_du())
+    s.step(1)
+    launches = s.profile_entries()
+    s.profile(False)
+    assert launches["pack"][0] == 2 and launches["visc_div"][0] == 1
+    # the step moved the state by 1e-3 of it or less, and du with it
+    for v in range(5):
+        assert np.linalg.norm(a[v] - b[v]) <= 0.1 * np.linalg.norm(a[v])
+    s.close()
