@@ -85,3 +85,23 @@ def test_right_hand_side_in_one_download(size, scheme, prec):
     for v in range(5):
         assert np.linalg.norm(a[v] - b[v]) <= 0.1 * np.linalg.norm(a[v])
     s.close()
+
+
+# padded fields of 32 and 126 KiB, fetched as they are, and of 133 KiB, packed
+@pytest.mark.parametrize("size,packed", [((8, 8, 8), 0), ((23, 20, 10), 0), ((24, 20, 11), 1)])
+def test_single_small_field_without_a_launch(size, packed):
+    """A single small FP64 field comes over without a launch of its own, with
+    the same values as with others."""
+    case = cases.wavy_box(*size, scheme="UP7")
+    s = case.load(capi.Solver(case.cfg))
+    s.step(2)
+    p = s.get_pressure()
+    d, _, _, _, T = s.get_flow()[0]
+    c = case.cfg
+    assert np.abs(p - d * T / (c.gamma * c.ama ** 2)).max() <= 4 * 2.0 ** -52 * p.max()
+    s.profile(True)
+    s.profile_reset()
+    s.get_pressure()
+    s.step(1)
+    assert s.profile_entries().get("pack", (0, 0.0))[0] == packed
+    s.close()
