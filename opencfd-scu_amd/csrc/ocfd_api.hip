@@ -355,8 +355,11 @@ int download_packed(ocfd_ctx* x, double* const* out, int nf, F&& pack) {
     S* const dev = (S*)(x->grad + x->fs);
     const size_t piece = PIECE / sizeof(S), np = (total + piece - 1) / piece;
     TRY(ensure_pin(x, std::min(bytes, SLOTS * PIECE)));
-    for (auto& e : x->pin_ev)
-        if (!e) HIPCK(hipEventCreateWithFlags(&e, hipEventDisableTiming));
+    {
+        OnDevice on(x->device);  // an event can be recorded on streams of its own device only
+        for (auto& e : x->pin_ev)
+            if (!e) HIPCK(hipEventCreateWithFlags(&e, hipEventDisableTiming));
+    }
     TRY(timed(x, "pack", [&] { pack(dev); }));
     auto slot = [&](size_t c) { return (S*)x->pin + (c % SLOTS) * piece; };
     auto count = [&](size_t c) { return std::min(piece, total - c * piece); };
