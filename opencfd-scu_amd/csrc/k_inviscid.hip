@@ -995,32 +995,42 @@ void launch_merged(const SweepArgsT<S>& a, int first, hipStream_t st) {
     else hipLaunchKernelGGL((k_sweeps<SCH, 1, S>), dim3(nb), dim3(256), 0, st, a, G);
 }
 
+// -1: no kernel for this scheme and direction.
 template <int SCH, typename S>
-void launch_scheme(int dir, const SweepArgsT<S>& a, hipStream_t st) {
+int launch_scheme(int dir, const SweepArgsT<S>& a, hipStream_t st) {
     const Geo& g = a.g;
     constexpr int NS = YZ<S>::NS, NA = YZ<S>::NA;
     if (dir == SWEEP_XY) {
         hipLaunchKernelGGL((k_sweep_tile<1, SCH, true, S>), dim3(tiles(g.nx, NA), tiles(g.ny, NS), g.nz), dim3(256), 0, st,
                            a);
-    } else if (dir < 0) {
+        return 0;
+    }
+    if (dir == SWEEP_ALL || dir == SWEEP_YZ) {
         launch_merged<SCH>(a, dir == SWEEP_YZ, st);
-    } else if (dir == 2) {
+        return 0;
+    }
+    if (dir == 2) {
         hipLaunchKernelGGL((k_sweep_tile<2, SCH, false, S>), dim3(tiles(g.nx, NA), tiles(g.nz, NS), g.ny), dim3(256), 0, st,
                            a);
-    } else if constexpr (SCH == OCFD_HYBRIDAUTO) {  // the one scheme for which x and y may be apart (sweeps_xy)
-        if (dir == 1)
+        return 0;
+    }
+    if constexpr (SCH == OCFD_HYBRIDAUTO) {  // the one scheme for which x and y may be apart (sweeps_xy)
+        if (dir == 1) {
             hipLaunchKernelGGL((k_sweep_tile<1, SCH, false, S>), dim3(tiles(g.nx, NA), tiles(g.ny, NS), g.nz), dim3(256), 0,
                                st, a);
-        else if (a.mlp.P)
-            hipLaunchKernelGGL((k_sweep_x<SCH, 1, S, true>), dim3(tiles(g.nx, XSeg<1>::XS), g.ny, g.nz), dim3(64), 0, st,
-                               a);
-        else if (two_segments(g))
-            hipLaunchKernelGGL((k_sweep_x<SCH, 2, S, false>), dim3(tiles(g.nx, XSeg<2>::XS), tiles(g.ny, 2), g.nz),
-                               dim3(64), 0, st, a);
-        else
-            hipLaunchKernelGGL((k_sweep_x<SCH, 1, S, false>), dim3(tiles(g.nx, XSeg<1>::XS), g.ny, g.nz), dim3(64), 0, st,
-                               a);
+            return 0;
+        }
+        if (dir == 0) {
+            const bool two = !a.mlp.P && two_segments(g);
+            const dim3 grid = two ? dim3(tiles(g.nx, XSeg<2>::XS), tiles(g.ny, 2), g.nz)
+                                  : dim3(tiles(g.nx, XSeg<1>::XS), g.ny, g.nz);
+            if (a.mlp.P) hipLaunchKernelGGL((k_sweep_x<SCH, 1, S, true>), grid, dim3(64), 0, st, a);
+            else if (two) hipLaunchKernelGGL((k_sweep_x<SCH, 2, S, false>), grid, dim3(64), 0, st, a);
+            else hipLaunchKernelGGL((k_sweep_x<SCH, 1, S, false>), grid, dim3(64), 0, st, a);
+            return 0;
+        }
     }
+    return -1;
 }
 template <int SCH, typename S>
 void launch_char_scheme(int dir, const SweepArgsT<S>& a, hipStream_t st) {
@@ -1060,19 +1070,18 @@ template bool sweeps_xy<float>(int, const Geo&);
 template <typename S>
 int launch_sweep(int scheme, int dir, const SweepArgsT<S>& a, hipStream_t st) {
     switch (scheme) {
-    case OCFD_UP7: launch_scheme<OCFD_UP7>(dir, a, st); break;
-    case OCFD_WENO5: launch_scheme<OCFD_WENO5>(dir, a, st); break;
-    case OCFD_WENO7: launch_scheme<OCFD_WENO7>(dir, a, st); break;
-    case OCFD_WENO7_SYMBO: launch_scheme<OCFD_WENO7_SYMBO>(dir, a, st); break;
-    case OCFD_WENO7_SYMBO_LIM: launch_scheme<OCFD_WENO7_SYMBO_LIM>(dir, a, st); break;
-    case OCFD_NND2: launch_scheme<OCFD_NND2>(dir, a, st); break;
-    case OCFD_OMP6_HR: launch_scheme<OCFD_OMP6_HR>(dir, a, st); break;
-    case OCFD_OMP6_LD: launch_scheme<OCFD_OMP6_LD>(dir, a, st); break;
-    case OCFD_OMP6_CD8: launch_scheme<OCFD_OMP6_CD8>(dir, a, st); break;
-    case OCFD_HYBRIDAUTO: launch_scheme<OCFD_HYBRIDAUTO>(dir, a, st); break;
-    default: return -1;
+    case OCFD_UP7: return launch_scheme<OCFD_UP7>(dir, a, st);
+    case OCFD_WENO5: return launch_scheme<OCFD_WENO5>(dir, a, st);
+    case OCFD_WENO7: return launch_scheme<OCFD_WENO7>(dir, a, st);
+    case OCFD_WENO7_SYMBO: return launch_scheme<OCFD_WENO7_SYMBO>(dir, a, st);
+    case OCFD_WENO7_SYMBO_LIM: return launch_scheme<OCFD_WENO7_SYMBO_LIM>(dir, a, st);
+    case OCFD_NND2: return launch_scheme<OCFD_NND2>(dir, a, st);
+    case OCFD_OMP6_HR: return launch_scheme<OCFD_OMP6_HR>(dir, a, st);
+    case OCFD_OMP6_LD: return launch_scheme<OCFD_OMP6_LD>(dir, a, st);
+    case OCFD_OMP6_CD8: return launch_scheme<OCFD_OMP6_CD8>(dir, a, st);
+    case OCFD_HYBRIDAUTO: return launch_scheme<OCFD_HYBRIDAUTO>(dir, a, st);
     }
-    return 0;
+    return -1;
 }
 template int launch_sweep<double>(int, int, const SweepArgsT<double>&, hipStream_t);
 template int launch_sweep<float>(int, int, const SweepArgsT<float>&, hipStream_t);

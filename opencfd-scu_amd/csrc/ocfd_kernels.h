@@ -33,9 +33,11 @@ struct SweepArgsT {
     } mlp;
 };
 // The sweep along dir, in the order x, y, z (x writes du, y and z add to it); x
-// and y in one launch (SWEEP_XY, which writes du; if sweeps_xy, and only then);
-// all three (SWEEP_ALL), or y and z after x (SWEEP_YZ), in one launch, each
-// direction into its own group of du.
+// and y in one launch (SWEEP_XY, which writes du); all three (SWEEP_ALL), or y
+// and z after x (SWEEP_YZ), in one launch, each direction into its own group of
+// du.  x and y by themselves exist for hybrid_auto only (the scheme for which
+// sweeps_xy may be false, and the learned sensor's).  -1, and nothing launched,
+// where there is no kernel.
 enum { SWEEP_ALL = -1, SWEEP_YZ = -2, SWEEP_XY = -3 };
 template <typename S>
 int launch_sweep(int scheme, int dir, const SweepArgsT<S>& a, hipStream_t st);

@@ -160,3 +160,17 @@ def test_create_refuses_more_wall_modes_than_the_tables_hold(hiplib):
     c.bc_npara[4] = 65
     assert hiplib.ocfd_create(C.byref(c), 0, C.byref(h)) == 2
     assert b"MTMAX" in hiplib.ocfd_last_error()
+
+
+@pytest.mark.parametrize("real", ["d", "f"])
+def test_sweeps_without_a_kernel_are_refused(hiplib, real):
+    """x and y alone have kernels for hybrid_auto only: any other scheme's are
+    refused (nothing is launched, so no GPU is needed), as is a direction
+    that is none."""
+    fn = getattr(hiplib, f"_Z12launch_sweepI{real}EiiiRK10SweepArgsTIT_EP12ihipStream_t")
+    fn.restype, fn.argtypes = C.c_int, [C.c_int, C.c_int, C.c_void_p, C.c_void_p]
+    args = C.create_string_buffer(4096)
+    for scheme in range(301, 310):
+        for direction in (0, 1, 3):
+            assert fn(scheme, direction, args, None) == -1, (scheme, direction)
+    assert fn(310, 3, args, None) == -1 and fn(999, 2, args, None) == -1
