@@ -952,7 +952,6 @@ void launch_diag_final(const double* partE, const double* partT, long long nb, c
     template void launch_bc108<S>(const BCArgsT<S>&, hipStream_t);                                           \
     template void launch_bc108_faces<S>(const BCArgsT<S>&, hipStream_t);                                     \
     template void launch_bc124_faces<S>(const BCArgsT<S>&, int, hipStream_t);                                \
-    template void launch_mirror_y<S>(const Geo&, S*, double, hipStream_t);                                   \
     template void launch_face_refresh<S>(const BCArgsT<S>&, hipStream_t);                                    \
     template void launch_sensor<S>(const Geo&, const Consts&, const S*, const S*, int8_t*, int8_t*, int8_t*, \
                                    hipStream_t);                                                              \
@@ -968,4 +967,5 @@ void launch_diag_final(const double* partE, const double* partT, long long nb, c
 OCFD_INSTANTIATE(double)
 OCFD_INSTANTIATE(float)
 #undef OCFD_INSTANTIATE
+template void launch_mirror_y<double>(const Geo&, double*, double, hipStream_t);
 template void launch_convert<float, double>(float*, const double*, long long, hipStream_t);
