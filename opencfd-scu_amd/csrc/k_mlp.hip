@@ -132,8 +132,8 @@ constexpr int PART = MLP_NPARAM + 1;  // a wave's partial: the parameters' gradi
 constexpr int MAX_PART = 1024;      // waves (partials) of one batch at most
 constexpr int UPD_SLICES = 16;      // partial sums taken beside each other in k_mlp_update
 
-int mlp_waves(int nb) {
-    const int t = (nb + TS - 1) / TS;
+int mlp_waves(int nb) {  // nb >= 1, up to the largest int
+    const int t = (nb - 1) / TS + 1;
     return t < MAX_PART ? t : MAX_PART;
 }
 
@@ -169,9 +169,10 @@ __global__ void __launch_bounds__(64) k_mlp_grad(const float* __restrict__ P, co
     const float b3 = P[OB3];
     v16f gW1 = {}, gW2 = {};
     float gb1 = 0.f, gb2 = 0.f, gw3 = 0.f, gb3 = 0.f, gl = 0.f;
-    for (int s0 = blockIdx.x * TS; s0 < nb; s0 += gridDim.x * TS) {
-        const int s = s0 + col;
-        const bool in = s < nb;
+    // unsigned: a step past the largest int stays past nb
+    for (unsigned s0 = blockIdx.x * TS; s0 < (unsigned)nb; s0 += gridDim.x * TS) {
+        const unsigned s = s0 + col;
+        const bool in = s < (unsigned)nb;
         const long long row = in ? (idx ? idx[s] : s) : 0;
         float x[12];
 #pragma unroll

@@ -174,3 +174,12 @@ def test_sweeps_without_a_kernel_are_refused(hiplib, real):
         for direction in (0, 1, 3):
             assert fn(scheme, direction, args, None) == -1, (scheme, direction)
     assert fn(310, 3, args, None) == -1 and fn(999, 2, args, None) == -1
+
+
+def test_training_partials_of_every_batch_size(hiplib):
+    """Floats of the partial gradient sums: 1890 a wave, a wave per 32 samples
+    up to 1024 waves, for any number of samples an int holds."""
+    fn = hiplib._Z15mlp_part_floatsi
+    fn.restype, fn.argtypes = C.c_size_t, [C.c_int]
+    for nb, waves in ((1, 1), (32, 1), (33, 2), (32767, 1024), (32769, 1024), (2**31 - 32, 1024), (2**31 - 1, 1024)):
+        assert fn(nb) == 1890 * waves, nb
