@@ -218,10 +218,12 @@ __global__ void __launch_bounds__(64) k_mlp_grad(const float* __restrict__ P, co
 #pragma unroll
         for (int r = 0; r < 16; r++) {
             const int o = col * TP + unit(r);
+            // nothing from the lanes past the last sample: their activations (of x =
+            // 0) may overflow where the samples' do not, and 0 times that is NaN
             sD1[o] = in ? da[r] * d1[r] : 0.f;  // dz1
-            sA1[o] = a1[r];
-            sD2[o] = d2[r];
-            sG3[o] = dz3 * a2[r];
+            sA1[o] = in ? a1[r] : 0.f;
+            sD2[o] = in ? d2[r] : 0.f;
+            sG3[o] = in ? dz3 * a2[r] : 0.f;
         }
         __syncthreads();
 #pragma unroll

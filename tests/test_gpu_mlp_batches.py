@@ -32,3 +32,27 @@ def test_batch_sizes_match_oracle(n, first):
         assert err <= 1e-4, (k, err)
     prob_ref, _ = M.forward(p64, X64)
     assert np.abs(t.predict(first, n) - prob_ref).max() <= 1e-5
+
+
+@pytest.mark.parametrize("n", [1, 17, 33])
+def test_lanes_past_the_last_sample_add_nothing(n):
+    """A bias that the samples' own inputs cancel: their activations are
+    ordinary, those of a zero input overflow the derivative of the GELU.  Bar as
+    above."""
+    rng = np.random.default_rng(n)
+    X = rng.standard_normal((n, 24)).astype(np.float32) * 0.3
+    X[:, 0] = 1.0
+    y = (rng.random(n) < 0.5).astype(np.float32)
+    p = M.init_params(seed=3, dtype=np.float32)
+    p["W1"][0] = 0.0
+    p["W1"][0, 0], p["b1"][0] = -1e25, 1e25
+    t = capi.Trainer(n)
+    t.set_params(capi.mlp_pack(p))
+    t.put(X, y)
+    loss, g = t.grad(0, n, wpos=2.5)
+    loss_ref, g_ref = M.loss_and_grads({k: v.astype(np.float64) for k, v in p.items()}, X.astype(np.float64),
+                                       y.astype(np.float64), wpos=2.5)
+    assert abs(loss - loss_ref) <= 1e-5 * abs(loss_ref)
+    gg = capi.mlp_unpack(g)
+    for k in g_ref:
+        assert np.abs(gg[k] - g_ref[k]).max() <= 1e-4 * np.abs(g_ref[k]).max(), k
