@@ -39,9 +39,9 @@ ALGO_BYTES = {
     "sweep_z": (5 + 3 + 5 + 5) * 8,
     "sweep_xy": (5 + 6 + 5) * 8,          # x and y in one launch: 6 cofactors, du written once
     "visc_flux": (4 + 10 + 12) * 8,       # u,v,w,T, 9 cofactors + Ajac; write 12 Ev (mu formed from T)
-    # divergence and RK stage: 12 Ev, du, Ajac, fn; write 5 primitives; the
-    # primitives in stages 2-3; f and p written in stage 3 (mean of the stages)
-    "visc_stage": (12 + 5 + 1 + 5 + 5) * 8 + (2 * 5 + 6) * 8 / 3,
+    # divergence and RK stage: 12 Ev, du, Ajac, fn; write f and 5 primitives; f
+    # read in stages 2-3; p written in stage 3 (mean of the stages)
+    "visc_stage": (12 + 5 + 1 + 5 + 5 + 5) * 8 + (2 * 5 + 1) * 8 / 3,
     "sensor": 2 * 8 + 3,                  # rho, T; write 3 int8 flags
 }
 

@@ -33,8 +33,11 @@ namespace {
 // hardware's estimate (5e-8) and a last correction of each: 15 instructions,
 // where a square root and a division of their own, with the scaling that only
 // subnormal and huge arguments need, take 30.  Largest errors over 2e6
-// arguments of e^-40..e^40: root 1.1e-16, reciprocal 1.7e-16, as before.  x = 0 gives NaN in both (ROOT0: the root is 0).  FP32: the
-// hardware's 1-ulp instructions.
+// arguments of e^-40..e^40: root 1.1e-16, reciprocal 1.7e-16, as of the square
+// root and division (du and the state come out the same distance from 80-bit
+// arithmetic with either).  x = 0 gives NaN in both (ROOT0: the root is 0).  FP32:
+// the hardware's instructions, 1 ulp each; without ROOT0 the root is x times the
+// reciprocal root (two roundings), at x = 0 NaN and infinity.
 template <bool ROOT0, typename R>
 __device__ __forceinline__ void sqrt_pair(R x, R& root, R& inv) {
     if constexpr (std::is_same<R, float>::value) {
@@ -881,14 +884,16 @@ template <> struct YZ<float> { static constexpr int NS = 15, NA = 16; };
 //
 // x and y together move 128 B a point in FP64 instead of 248 (the primitives
 // once, du written and not read back), yet take as long as the two alone where
-// these run at the copy rate (1024x256x128 ramp 1.77 -> 1.75 ms): barriers, LDS
-// (57 % of the cycles) and VALU (57 %) bound the tile.  What they leave to the
-// gradient kernel on the other stream is the gain: a step of 1024x256x128
-// 19.88 -> 19.55 ms, 640x192x96 5.18 -> 5.00, 256x128x128 WENO7 3.08 -> 3.00 (x + y
-// 465 -> 431 us), mixed 512x128x64 1.69 -> 1.61, mixed 131x99x80 0.648 -> 0.626.
+// these run at the copy rate (1024x256x128 ramp 1.79 ms, 1.77 apart): barriers,
+// LDS (busy 72 % of the cycles on the 1024x384x256 ramp) and VALU (65 %) bound the
+// tile (profiles/ramp1024x384x256_sweep30_sweep_counters.md).  What they leave to
+// the gradient kernel on the other stream is the gain, measured when the launch
+// came: a step of 1024x256x128 19.88 -> 19.55 ms, 640x192x96 5.18 -> 5.00,
+// 256x128x128 WENO7 3.08 -> 3.00 (x + y 465 -> 431 us), mixed 512x128x64 1.69 ->
+// 1.61, mixed 131x99x80 0.648 -> 0.626.
 // Two neighbouring faces a thread, which read 40 LDS values a face for 70,
 // need 104-122 VGPRs for 76 and were slower (276 -> 310 us at 512x128x64), and so
-// were more threads a block; x lines spread free of bank conflicts (17 % of the
+// were more threads a block; x lines spread free of bank conflicts (18 % of the
 // LDS cycles), and hybrid_auto's special faces given out over the wave as in
 // sweep_x, changed nothing.
 // ---------------------------------------------------------------------------
@@ -924,7 +929,7 @@ __global__ void __launch_bounds__(256, SCH == OCFD_HYBRIDAUTO ? 3 : 2) k_char(Sw
 // its own five fields, which the RK stage adds: the sweeps then
 // depend on nothing but the stage's state.  For small grids (sweeps_merged):
 // a launch of theirs is as long as its slowest block, and three of them with
-// their gaps are replaced by one (64^3: 24 + 21 + 21 us -> 48 us, 43 now, 20x16x12: 9 +
+// their gaps are replaced by one (64^3: 24 + 21 + 21 us -> 48 us, 45 now, 20x16x12: 9 +
 // 10 + 10 -> 10).  On larger ones it gains less than the stage pays for reading
 // three parts (256x128x128: 712 -> 670 us, the stage 234 -> 297;
 // 1024x256x128: 2.96 -> 2.92 ms and 2.02 -> 2.60).  Blocks in the order x, y, z;
@@ -1054,12 +1059,17 @@ void launch_char_scheme(int dir, const SweepArgsT<S>& a, hipStream_t st) {
 // 660 -> 667, 256x128x128 3168 -> 3300.
 bool sweeps_merged(const Geo& g) { return (long long)g.nx * g.ny * g.nz <= 500000; }
 
-// Whether x and y of a larger grid are one launch.  hybrid_auto in FP64, whose x
-// sweep alone is the cheapest, keeps them apart between 1.5 and 10 million
-// points (a step: 256x128x64 1.324 ms apart, 1.346 together; 512x128x64 2.432,
-// 2.484; 512x128x128 4.91, 5.01), where du stays in the Infinity Cache between
-// the two; below, a launch and its tail less count for more (200x90x60 0.801,
-// 0.742), above, du's bytes.
+// Whether x and y of a larger grid are one launch.  They are for every scheme
+// but one: a step of 131x99x80 to 512x256x128, FP64 and mixed, is shorter by 3-7 %
+// with UP7, 4-7 with NND2, 2-4 with WENO5, 1-4 with WENO7.  hybrid_auto in FP64
+// keeps them apart between 1.5 and 10 million points: with shocks in the flow
+// the x sweep by itself spreads its few WENO faces over the wave, which the
+// tiles do not (ramps, ms a step apart and together: 2.1 M points 1.402 and 1.421,
+// 4.2 M 2.68 and 2.74, 8.4 M 5.01 and 5.03); a launch and its tail less count
+// for more below (1.0 M 0.894 and 0.868, still 1.091 and 1.039 at 1.51 M), du's
+// bytes above (12.6 M 7.45 and 7.26, 16.8 M 9.99 and 9.67).  The flow is not
+// known here: without shocks together is shorter there too (box, 4.2 M 2.37 and
+// 2.29).
 template <typename S> bool sweeps_xy(int scheme, const Geo& g) {
     const long long n = (long long)g.nx * g.ny * g.nz;
     return scheme != OCFD_HYBRIDAUTO || sizeof(S) == 4 || n < 1500000 || n > 10000000;

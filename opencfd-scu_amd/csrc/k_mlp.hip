@@ -42,7 +42,7 @@ static_assert(OB3 + 1 == MLP_NPARAM, "parameter layout");
 // plane = 1: the nodes (i >= 0, j = -1, k >= 0), whose flag only the y sweep
 // reads (face -1/2); plane = 2: the nodes (i >= 0, j >= 0, k = -1) for the z
 // sweep.  The x sweep of the first RK stage computes the other nodes itself
-// (k_sweep with the learned sensor), and planes 1 and 2 complete it.
+// (k_sweep_x with LEARN), and planes 1 and 2 complete it.
 // The lane fragments of the weights in the layout lane_weights_packed reads
 // (one wave).
 __global__ void __launch_bounds__(64) k_mlp_pack(const float* __restrict__ P, float* __restrict__ pk) {

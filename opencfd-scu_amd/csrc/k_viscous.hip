@@ -182,12 +182,13 @@ __device__ __forceinline__ bool near_closure(const ViscArgsT<S>& A, const Tile25
 // strips and queue values and the point's metrics are in flight while a plane
 // is computed.  Bound by HBM (512x128x64 5.7 TB/s of traffic) and by latency
 // behind it: what moved it is when loads are issued.  Raw buffer accesses took
-// the FP64 kernel from 233 VGPRs to 206 (still 2 waves per SIMD) and the FP32
+// the FP64 kernel from 233 VGPRs to 204 (still 2 waves per SIMD) and the FP32
 // kernel from 3 waves to 4, and made the ring of strips fetched five planes
 // ahead pointless: 1024x256x128 1.58 -> 1.54 ms, 512x128x64 193 -> 182 us, mixed
-// 120 -> 117 us.  Dropped: metrics loaded after the derivatives to fit 3 waves
-// (182 -> 241 us, mixed 117 -> 167), a plane ahead (194, 141), 32x16 tiles (210,
-// 126).
+// 120 -> 117 us (1024x384x256 1 %, though it fetches 178.5 B/pt for 152.5: a
+// strip's second reader finds it evicted more often).  Dropped: metrics loaded
+// after the derivatives to fit 3 waves (182 -> 241 us, mixed 117 -> 167), a plane
+// ahead (194, 141), 32x16 tiles (210, 126).
 template <int SV, typename S>
 __global__ void __launch_bounds__(TX * TY, sizeof(S) == 8 ? 2 : 4) k_visc_gf(ViscArgsT<S> A, int kz) {
     constexpr int NT = TX * TY;
@@ -305,7 +306,8 @@ __device__ __forceinline__ void p2c5(double d, double u, double v, double w, dou
 // computed.  All accesses are raw buffer accesses (Buf): with plain pointers
 // the 40 addresses of a point took the kernel to 255 VGPRs and spills (FP32:
 // slower than the separate kernels, 252 us against 215 on 512x128x64); with
-// them it needs 203, FP32 124.  Divergence and stage as one launch against
+// them it needs 203, FP32 125 (223, and 128 with 12 spilled, where it adds three
+// parts of du).  Divergence and stage as one launch against
 // three (two of two flux components, then the stage): 1024x256x128 2.42 -> 2.17
 // ms, 512x128x64 296 -> 251 us, mixed 215 -> 172 us, 640x192x96 mixed 567 -> 510
 // us.
@@ -314,8 +316,8 @@ template <int SV, typename S, int KRK, int PARTS>
 __global__ void __launch_bounds__(NTD, sizeof(S) == 8 ? 2 : 4) k_visc_div(ViscArgsT<S> A, StageArgsT<S> G, int kz) {
     static_assert(TY == 8, "one y-halo value per thread: 8 halo rows of TX columns");
     // FP64, at 2 waves per SIMD, has registers to fetch the point's values a
-    // plane ahead (512x128x64: 252 -> 232 us against loads after the derivatives
-    // at 3 waves); FP32 fetches them before the derivatives and keeps 4 waves
+    // plane ahead (512x128x64, then without f in stages 1 and 2: 252 -> 232 us
+    // against loads after the derivatives at 3 waves); FP32 fetches them before the derivatives and keeps 4 waves
     // (172 us; a plane ahead 179 at 3 waves, 192 at 4)
     constexpr bool AHEAD = sizeof(S) == 8;
     constexpr int XW = TX + 8, NC = 4;
@@ -520,12 +522,13 @@ __global__ void __launch_bounds__(256) k_qcrit(ViscArgsT<S> A, double* __restric
 
 // z planes per block.  A launch that does not fill the chip is bound by the
 // longest march: its planes are spread over as many blocks as the GPU holds
-// at once (2 per CU of the FP64 kernels, 4 of the FP32 ones), each block paying the 8 planes of its z queue again
-// from L2.  Measured, a gradient launch, against the fixed chunks: 64^3 82 ->
-// 17.5 us, 61x47x39 84 -> 13.2, 203x93x45 142 -> 53.5 (a divergence of two
-// components 38 -> 9.0, 38.5 -> 7.8, 55 -> 21.2); 512x128x64, which 32 planes
-// fill exactly, keeps them (16: 196 -> 204 us).  Larger launches take the
-// fixed chunk, where the extra z reads are what counts.
+// at once (2 per CU of the FP64 kernels, 4 of the FP32 ones), each block paying the
+// 8 planes of its z queue again from L2.  Measured when it came, a gradient
+// launch, against the fixed chunks: 64^3 82 -> 17.5 us, 61x47x39 84 -> 13.2,
+// 203x93x45 142 -> 53.5 (now 15.8, 11.1 and 48; the divergence, then two components a
+// launch, 38 -> 9.0, 38.5 -> 7.8, 55 -> 21.2 each); 512x128x64, which 32 planes fill
+// exactly, keeps them (16: 196 -> 204 us).  Larger launches take the fixed chunk,
+// where the extra z reads are what counts.
 template <typename S>
 int chunk_planes(const Geo& g, int cols) {
     constexpr int RES = 256 * (sizeof(S) == 8 ? 2 : 4), MOST = 32;
